@@ -1055,8 +1055,9 @@ __device__ __forceinline__ std::uint64_t window_row_ptrs(const ScatterArgs& a, s
 // The window's source rows x[c] from window_row_ptrs (zeros for null), all
 // 8 loads issued before any is used; TF32-rounded unless packed as TF32.
 // Skipping unused rows matters most for the first layer's cold rows, which
-// cross the host link.
-template <int V, bool PACKED>
+// cross the host link.  The lane's features are laneOff + v * STEP (packed
+// rows: STEP 1); with STEP > 1 those past F re-read its first.
+template <int V, bool PACKED, std::uint32_t STEP>
 __device__ __forceinline__ void load_window_rows(const ScatterArgs& a, std::uint64_t rowPtrs, std::uint32_t laneOff,
                                                  float (&x)[8][V]) {
     const std::uint32_t lo = static_cast<std::uint32_t>(rowPtrs);
@@ -1079,9 +1080,17 @@ __device__ __forceinline__ void load_window_rows(const ScatterArgs& a, std::uint
 #pragma unroll
         for (int v = 0; v < V; ++v) x[c][v] = 0.0f;
         if (rp != 0) {
-            const Vec<V> t = load_vec<V>(reinterpret_cast<const float*>(rp) + laneOff);
+            if constexpr (STEP == 1) {
+                const Vec<V> t = load_vec<V>(reinterpret_cast<const float*>(rp) + laneOff);
 #pragma unroll
-            for (int v = 0; v < V; ++v) x[c][v] = t.v[v];
+                for (int v = 0; v < V; ++v) x[c][v] = t.v[v];
+            } else {
+#pragma unroll
+                for (int v = 0; v < V; ++v) {
+                    const std::uint32_t f = laneOff + v * STEP;
+                    x[c][v] = load_global<float>(reinterpret_cast<const float*>(rp) + (f < a.F ? f : laneOff));
+                }
+            }
         }
     }
 #pragma unroll
@@ -1123,6 +1132,14 @@ __device__ __forceinline__ float scatter_vals(const ScatterArgs& a, std::uint64_
     return __lane_id() < static_cast<unsigned>(__popcll(bits)) ? a.data[off + __lane_id()] : 0.0f;
 }
 
+// The features a lane holds: V consecutive ones (the first layer's form, whose
+// row loads cross the host link in whole V-wide requests), or, for rows in
+// device memory, every 64th of the chunk (feature 64v + lane), so that each
+// atomic instruction adds 64 consecutive floats.  The atomics set this
+// kernel's time: they are performed past the L2 in 64-byte requests, and with
+// 4 consecutive floats a lane every instruction touched four times the
+// requests.  1.5M edges of a 100k-node R-MAT graph at F = 256: 5.53 -> 1.36 ms
+// (22M requests of 64 bytes, 17 G/s; a probe of such adds reaches 20 G/s).
 template <int V, bool MIXED, bool VALUES, bool PACKED = false>
 __device__ __forceinline__ void scatter_body(const ScatterArgs& a, std::uint32_t gw) {
     const unsigned lane = __lane_id();
@@ -1131,9 +1148,10 @@ __device__ __forceinline__ void scatter_body(const ScatterArgs& a, std::uint32_t
     if (chunk >= a.numChunks) return;
     const UnitRange u = unit_range(a.winOffset, a.numWindows, a.numBlocks, a.unitBlocks, a.numUnits, unit);
     if (u.b0 >= u.b1 || u.w >= a.numWindows) return;
-    const std::uint32_t f0 = chunk * (kWave * V) + lane * V;
+    constexpr std::uint32_t kStep = MIXED ? 1 : kWave;  // between a lane's features
+    const std::uint32_t f0 = chunk * (kWave * V) + lane * (MIXED ? V : 1);
     const bool active = f0 < a.F;
-    const std::uint32_t laneOff = active ? f0 : f0 - lane * V;  // inactive: lane 0's features
+    const std::uint32_t laneOff = active ? f0 : f0 - lane * (MIXED ? V : 1);  // inactive: lane 0's features
 
     std::uint32_t w = u.w;
     std::uint32_t we = a.winOffset[w + 1];
@@ -1142,7 +1160,7 @@ __device__ __forceinline__ void scatter_body(const ScatterArgs& a, std::uint32_t
         we = a.winOffset[w + 1];
     }
     float x[8][V];
-    load_window_rows<V, PACKED>(a, window_row_ptrs<MIXED>(a, w, used_columns(a.bits, u.b0, min(we, u.b1))), laneOff,
+    load_window_rows<V, PACKED, kStep>(a, window_row_ptrs<MIXED>(a, w, used_columns(a.bits, u.b0, min(we, u.b1))), laneOff,
                                 x);
     std::uint32_t cur = scatter_meta<VALUES>(a, u.b0);
     float curVals = 0.0f;
@@ -1153,7 +1171,7 @@ __device__ __forceinline__ void scatter_body(const ScatterArgs& a, std::uint32_t
                 ++w;
                 we = a.winOffset[w + 1];
             } while (b >= we && w + 1 < a.numWindows);
-            load_window_rows<V, PACKED>(a, window_row_ptrs<MIXED>(a, w, used_columns(a.bits, b, min(we, u.b1))), laneOff,
+            load_window_rows<V, PACKED, kStep>(a, window_row_ptrs<MIXED>(a, w, used_columns(a.bits, b, min(we, u.b1))), laneOff,
                                         x);
         }
         const std::uint64_t bm = meta_bits(cur, 8);
@@ -1192,7 +1210,7 @@ __device__ __forceinline__ void scatter_body(const ScatterArgs& a, std::uint32_t
                 float* out = a.Y + static_cast<std::uint64_t>(row) * a.F + f0;
 #pragma unroll
                 for (int v = 0; v < V; ++v)
-                    if (f0 + v < a.F) atomic_add_f32(out + v, s[v]);
+                    if (f0 + v * kStep < a.F) atomic_add_f32(out + v * kStep, s[v]);
             }
         }
         cur = nxt;
@@ -1200,9 +1218,9 @@ __device__ __forceinline__ void scatter_body(const ScatterArgs& a, std::uint32_t
     }
 }
 
-template <int V, bool MIXED, bool VALUES>
+template <int V, bool VALUES>
 __global__ void __launch_bounds__(kThreads) scatter_kernel(ScatterArgs a) {
-    scatter_body<V, MIXED, VALUES>(a, blockIdx.x * kWaves + uniform(threadIdx.x / kWave));
+    scatter_body<V, false, VALUES>(a, blockIdx.x * kWaves + uniform(threadIdx.x / kWave));
 }
 
 // The first layer's forward in one launch.  The reference runs the hot BCSR
@@ -1373,21 +1391,30 @@ int launch_narrow(GatherArgs a, std::uint32_t requestedK, hipStream_t st) {
     return TCC_OK;
 }
 
-template <bool MIXED>
-int launch_scatter(ScatterArgs a, int V, std::uint32_t requestedK, hipStream_t st) {
+template <bool VALUES>
+void scatter_dispatch(const ScatterArgs& a, int V, dim3 grid, hipStream_t st) {
+    if (V == 1) hipLaunchKernelGGL((scatter_kernel<1, VALUES>), grid, dim3(kThreads), 0, st, a);
+    else if (V == 2) hipLaunchKernelGGL((scatter_kernel<2, VALUES>), grid, dim3(kThreads), 0, st, a);
+    else if (V == 3) hipLaunchKernelGGL((scatter_kernel<3, VALUES>), grid, dim3(kThreads), 0, st, a);
+    else hipLaunchKernelGGL((scatter_kernel<4, VALUES>), grid, dim3(kThreads), 0, st, a);
+}
+
+// Features a lane: as many 64-feature steps as a chunk of at most 256
+// features needs, the chunks of a wider F of equal width (its loads and
+// atomics are one float each, so any F and alignment will do).
+inline int scatter_vec(std::uint32_t F) {
+    const std::uint32_t chunks = (F + 4 * kWave - 1) / (4 * kWave);
+    return static_cast<int>((F + chunks * kWave - 1) / (chunks * kWave));
+}
+
+int launch_scatter(ScatterArgs a, std::uint32_t requestedK, hipStream_t st) {
+    const int V = scatter_vec(a.F);
     const std::uint64_t waves = plan_scatter(a, V, requestedK);
     if (waves == 0) return TCC_OK;
     TCC_REQUIRE(waves <= 0xFFFFFFFFull / kWaves, TCC_ERR_UNSUPPORTED, "SpMM launch too large");
     const dim3 grid(grid_for(waves, kWaves));
-    if (a.data != nullptr) {
-        if (V == 4) hipLaunchKernelGGL((scatter_kernel<4, MIXED, true>), grid, dim3(kThreads), 0, st, a);
-        else if (V == 2) hipLaunchKernelGGL((scatter_kernel<2, MIXED, true>), grid, dim3(kThreads), 0, st, a);
-        else hipLaunchKernelGGL((scatter_kernel<1, MIXED, true>), grid, dim3(kThreads), 0, st, a);
-    } else {
-        if (V == 4) hipLaunchKernelGGL((scatter_kernel<4, MIXED, false>), grid, dim3(kThreads), 0, st, a);
-        else if (V == 2) hipLaunchKernelGGL((scatter_kernel<2, MIXED, false>), grid, dim3(kThreads), 0, st, a);
-        else hipLaunchKernelGGL((scatter_kernel<1, MIXED, false>), grid, dim3(kThreads), 0, st, a);
-    }
+    if (a.data != nullptr) scatter_dispatch<true>(a, V, grid, st);
+    else scatter_dispatch<false>(a, V, grid, st);
     TCC_LAUNCH_CHECK();
     return TCC_OK;
 }
@@ -1719,8 +1746,7 @@ int tcc_bcsc_spmm(const tcc_bcsc* A, const float* X, float* Y, std::uint32_t fea
     clear_last_error();
     TCC_REQUIRE(bcsc_ok(A) && X && Y && feature_dim_ok(featureDim), TCC_ERR_INVALID_ARGUMENT,
                 "invalid BCSC SpMM arguments");
-    return launch_scatter<false>(bcsc_args(A, X, Y, featureDim), pick_vec(featureDim, {X, Y}), A->unitBlocks,
-                                 as_stream(stream));
+    return launch_scatter(bcsc_args(A, X, Y, featureDim), A->unitBlocks, as_stream(stream));
 }
 
 int tcc_bcsc_transpose_spmm(const tcc_bcsc* A, const float* dY, float* dX, std::uint32_t featureDim,
