@@ -24,7 +24,7 @@ ARCH = os.environ.get("TCC_OFFLOAD_ARCH", "gfx950")
 
 LIB_SOURCES = ["swtcf_convert.hip", "swtcf_spmm.hip", "swtcf_plan.hip", "bcsr_spmm.hip", "bcsr_build.hip",
                "hub_tiles.hip", "dense_tn.hip",
-               "errors.cpp"]
+               "scratch.cpp", "errors.cpp"]
 LIB_NAME = "libtcc_swtcf.so"
 
 # -packed-fp32-ops: keep the compiler from emitting v_pk_{add,mul,fma}_f32.

@@ -179,34 +179,6 @@ __device__ __forceinline__ std::uint32_t lane_u32(std::uint32_t v, int l) {
     return static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), l));
 }
 
-__device__ __forceinline__ std::uint32_t uniform(std::uint32_t v) {
-    return static_cast<std::uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
-}
-
-// First index i in [0, n) with off[i] >= key (n if there is none), for a
-// non-decreasing off[], computed by one wave: each round probes 64 evenly
-// spaced entries with one vector load and narrows the range to the gap the
-// ballot points at (3 rounds for 2^18 entries).
-__device__ std::uint32_t wave_lower_bound(const std::uint32_t* off, std::uint32_t n, std::uint32_t key) {
-    const unsigned lane = __lane_id();
-    std::uint32_t lo = 0, hi = n;  // answer in [lo, hi]
-    while (hi - lo > 64) {
-        const std::uint32_t step = (hi - lo + 63) / 64;
-        const std::uint32_t p = lo + (lane + 1) * step - 1;
-        const bool ge = p >= hi || off[p] >= key;
-        const std::uint64_t m = __ballot(ge);
-        if (m == 0) return hi;
-        const std::uint32_t L = static_cast<std::uint32_t>(__builtin_ctzll(m));
-        const std::uint32_t pL = lo + (L + 1) * step - 1;
-        lo = lo + L * step;
-        hi = min(pL, hi);
-    }
-    const std::uint32_t p = lo + lane;
-    const bool ge = p >= hi || off[p] >= key;
-    const std::uint64_t m = __ballot(ge);
-    return m == 0 ? hi : lo + static_cast<std::uint32_t>(__builtin_ctzll(m));
-}
-
 // The blocks [b0, b1) of unit u and the first window it finishes: the
 // window holding block b0, or (when windows start exactly at b0) the first
 // of them, empty ones included.

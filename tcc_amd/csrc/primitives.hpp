@@ -51,13 +51,18 @@ __device__ __forceinline__ void prim_load(const T* __restrict__ p, std::uint64_t
 
 // ------------------------------------------------------------------ scan
 
-__device__ __forceinline__ std::uint32_t wave_inclusive_scan(std::uint32_t v) {
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const std::uint32_t n = __shfl_up(v, d, kWave);
-        if (static_cast<int>(__lane_id()) >= d) v += n;
-    }
-    return v;
+// Inclusive sum over the wave's lanes (all active): within rows of 16 lanes
+// by row shifts, then lane 15 of a row into the next and lane 31 into the
+// upper half, all in the vector ALU (a shuffle goes through the LDS unit).
+__device__ __forceinline__ std::uint32_t wave_inclusive_scan(std::uint32_t x) {
+    int v = static_cast<int>(x);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);   // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);   // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);   // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);   // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+    return static_cast<std::uint32_t>(v);
 }
 
 // With `skip` given, the scan kernels return at once while *skip is 0 (a

@@ -36,6 +36,7 @@
 #include "../../include/tcc_spmm_cnic.h"
 #include "../../include/tcc_swtcf.h"
 #include "common.hpp"
+#include "scratch.hpp"
 #include "gather_ops.hpp"
 #include "primitives.hpp"
 #include "swtcf_plan.hpp"
@@ -514,6 +515,7 @@ int tcc_swtcf_release_plans(void) {
     std::lock_guard<std::mutex> lock(C.mu);
     for (auto& p : C.plans) p.release();
     C.plans.clear();
+    release_scratch();
     return TCC_OK;
 }
 
