@@ -120,14 +120,6 @@ __device__ __forceinline__ std::uint32_t grouped_window(const Coo& c, const std:
     else return c.a[i] >> 3;  // in range, and one phase: checked before
 }
 
-__device__ __forceinline__ void raise_flag(std::uint32_t* flag, bool mine) {
-    // one atomic per wave, and none once the flag is seen set
-    if (__ballot(mine) == 0) return;
-    if (__lane_id() == static_cast<unsigned>(__builtin_ctzll(__ballot(mine))) &&
-        __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u)
-        atomicOr(flag, 1u);
-}
-
 // Window starts: the thread of edge i writes i to every window after its
 // predecessor's up to its own (thread E: to all that are left), so
 // winStart[w] is the first edge of window w or of the next one with edges.
@@ -179,12 +171,12 @@ __global__ void __launch_bounds__(kThreads) window_starts_kernel(Coo c, const st
 
 // ---------------------------------------------------------------- partition
 
-// Stable partition of the elements by one digit of the window, in tiles of
-// 4096 (primitives.hpp).  FIRST reads the COO and checks its ranges.
-template <bool FIRST>
-__device__ __forceinline__ void load_elements(const Coo& c, const std::uint64_t* __restrict__ in, std::uint64_t first,
-                                              std::uint64_t (&k)[kPrimRounds], bool& bad) {
-    if constexpr (FIRST) {
+// Elements of the first pass, from the COO (ranges checked), for the
+// partition by the window's digits.
+struct CooLoad {
+    Coo c;
+    std::uint32_t* flags;
+    __device__ __forceinline__ void load(std::uint64_t first, std::uint64_t (&k)[kPrimRounds], bool& bad) const {
         std::uint32_t a[kPrimRounds], b[kPrimRounds];
         const std::uint64_t last = c.E - 1;
 #pragma unroll
@@ -206,126 +198,9 @@ __device__ __forceinline__ void load_elements(const Coo& c, const std::uint64_t*
                      c.windowsPerPhase;
             k[r] = pack_edge(Edge{w, b[r], a[r] & 7u}, c.bBits);
         }
-    } else {
-        prim_load(in, first, c.E, k);
     }
-}
-
-template <bool FIRST>
-__global__ void __launch_bounds__(kPrimThreads) part_hist_kernel(Coo c, const std::uint64_t* __restrict__ in,
-                                                                unsigned shift, unsigned bits,
-                                                                std::uint32_t* __restrict__ hist, unsigned tiles,
-                                                                std::uint32_t* __restrict__ flags) {
-    __shared__ std::uint32_t h[kPrimWaves][kRadixBins];
-    const unsigned lane = __lane_id(), wave = threadIdx.x / kWave;
-    for (int i = threadIdx.x; i < kPrimWaves * kRadixBins; i += kPrimThreads) (&h[0][0])[i] = 0;
-    __syncthreads();
-    const std::uint64_t base = static_cast<std::uint64_t>(blockIdx.x) * kPrimTile + wave * kWaveSpan;
-    std::uint64_t k[kPrimRounds];
-    bool bad = false;
-    load_elements<FIRST>(c, in, base + lane, k, bad);
-    const unsigned mask = (1u << bits) - 1u;
-#pragma unroll
-    for (int r = 0; r < kPrimRounds; ++r)
-        if (base + r * kWave + lane < c.E) atomicAdd(&h[wave][static_cast<unsigned>(k[r] >> shift) & mask], 1u);
-    if constexpr (FIRST) raise_flag(&flags[kFlagRange], bad);
-    __syncthreads();
-    const unsigned d = threadIdx.x;  // kPrimThreads == kRadixBins
-    if (d <= mask) {
-        std::uint32_t s = 0;
-#pragma unroll
-        for (int w = 0; w < kPrimWaves; ++w) s += h[w][d];
-        hist[static_cast<std::uint64_t>(d) * tiles + blockIdx.x] = s;
-    }
-}
-
-// hist[d][*] := its exclusive scan, total[d] := its sum; one workgroup per
-// digit, 4096 counts a step.  (One launch in place of the three of a scan
-// over all digits: the digits' bases are summed where they are used.)
-__global__ void __launch_bounds__(1024) digit_scan_kernel(std::uint32_t* __restrict__ hist, unsigned tiles,
-                                                         std::uint32_t* __restrict__ total) {
-    __shared__ std::uint32_t waveSum[16];
-    std::uint32_t* row = hist + static_cast<std::uint64_t>(blockIdx.x) * tiles;
-    const unsigned lane = __lane_id(), wave = threadIdx.x / kWave;
-    std::uint32_t run = 0;
-    for (unsigned base = 0; base < tiles; base += 4096) {
-        const unsigned i0 = base + 4 * threadIdx.x;
-        std::uint32_t v[4], s = 0;
-#pragma unroll
-        for (unsigned q = 0; q < 4; ++q) v[q] = i0 + q < tiles ? row[i0 + q] : 0u;
-#pragma unroll
-        for (unsigned q = 0; q < 4; ++q) s += v[q];
-        const std::uint32_t inc = wave_inclusive_scan(s);
-        if (lane == kWave - 1) waveSum[wave] = inc;
-        __syncthreads();
-        std::uint32_t off = run + inc - s, all = 0;
-#pragma unroll
-        for (unsigned w = 0; w < 16; ++w) {
-            if (w < wave) off += waveSum[w];
-            all += waveSum[w];
-        }
-#pragma unroll
-        for (unsigned q = 0; q < 4; ++q) {
-            if (i0 + q < tiles) row[i0 + q] = off;
-            off += v[q];
-        }
-        run += all;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) total[blockIdx.x] = run;
-}
-
-template <bool FIRST>
-__global__ void __launch_bounds__(kPrimThreads) part_scatter_kernel(Coo c, const std::uint64_t* __restrict__ in,
-                                                                   std::uint64_t* __restrict__ out, unsigned shift,
-                                                                   unsigned bits, const std::uint32_t* __restrict__ hist,
-                                                                   unsigned tiles,
-                                                                   const std::uint32_t* __restrict__ total) {
-    __shared__ std::uint32_t cnt[kPrimWaves][kRadixBins];
-    __shared__ std::uint32_t waveSum[kPrimWaves];
-    const unsigned lane = __lane_id(), wave = threadIdx.x / kWave;
-    const unsigned bins = 1u << bits, mask = bins - 1u;
-    for (int i = threadIdx.x; i < kPrimWaves * kRadixBins; i += kPrimThreads) (&cnt[0][0])[i] = 0;
-    const std::uint64_t base = static_cast<std::uint64_t>(blockIdx.x) * kPrimTile + wave * kWaveSpan;
-    const std::uint64_t lt = lanemask_lt();
-    std::uint64_t k[kPrimRounds];
-    std::uint32_t rank[kPrimRounds];
-    bool bad = false;
-    load_elements<FIRST>(c, in, base + lane, k, bad);
-    // thread d: digit d's base (the digits before it) and this tile's place in it
-    const unsigned d = threadIdx.x;
-    const std::uint32_t tot = d < bins ? total[d] : 0u;
-    const std::uint32_t inTile = d < bins ? hist[static_cast<std::uint64_t>(d) * tiles + blockIdx.x] : 0u;
-    const std::uint32_t inc = wave_inclusive_scan(tot);
-    if (lane == kWave - 1) waveSum[wave] = inc;
-    __syncthreads();
-    std::uint32_t run = inc - tot + inTile;
-    for (unsigned w = 0; w < wave; ++w) run += waveSum[w];
-#pragma unroll
-    for (int r = 0; r < kPrimRounds; ++r) {
-        const bool valid = base + r * kWave + lane < c.E;
-        const unsigned dg = static_cast<unsigned>(k[r] >> shift) & mask;
-        const std::uint64_t peers = match_peers<kRadixBits>(dg, valid);
-        const std::uint32_t seen = cnt[wave][dg];
-        rank[r] = seen + static_cast<std::uint32_t>(__popcll(peers & lt));
-        if (valid && (peers & lt) == 0) cnt[wave][dg] = seen + static_cast<std::uint32_t>(__popcll(peers));
-    }
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < kPrimWaves; ++w) {
-        const std::uint32_t n = cnt[w][d];
-        cnt[w][d] = run;  // the first position of (wave w, digit d)
-        run += n;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kPrimRounds; ++r) {
-        if (base + r * kWave + lane < c.E) {
-            const unsigned dg = static_cast<unsigned>(k[r] >> shift) & mask;
-            out[cnt[wave][dg] + rank[r]] = k[r];
-        }
-    }
-}
+    __device__ __forceinline__ void report(bool bad) const { raise_flag(&flags[kFlagRange], bad); }
+};
 
 // ---------------------------------------------------------------- lists
 
@@ -977,7 +852,7 @@ struct BlockArrays {
         const std::size_t sizes[5] = {align_up(4 * (RW + 1)), align_up(4 * (maxB + 1)), align_up(32 * std::max<std::uint64_t>(maxB, 1)),
                                       align_up(8 * std::max<std::uint64_t>(maxB, 1)),
                                       values ? align_up(4 * std::max<std::uint64_t>(E, 1)) : 0};
-        const hipError_t e = malloc_or_release(reinterpret_cast<void**>(&base),
+        const hipError_t e = pool_malloc(reinterpret_cast<void**>(&base),
                                                sizes[0] + sizes[1] + sizes[2] + sizes[3] + sizes[4]);
         if (e != hipSuccess) {
             base = nullptr;
@@ -1004,7 +879,6 @@ int build_blocks(Coo c, std::uint32_t RW, const float* val, BlockArrays& out, st
     const bool tryGrouped = !BCSC && c.phases == 1;
     const std::uint64_t E = c.E;
     const unsigned wBits = ceil_log2(RW);
-    const unsigned tiles = radix_tiles(E);
     const bool places = BCSC && val;
     std::uint64_t *keysA = nullptr, *keysB = nullptr;
     std::uint32_t *winStart, *flags, *blocks, *scanTemp, *hist, *total;
@@ -1023,7 +897,7 @@ int build_blocks(Coo c, std::uint32_t RW, const float* val, BlockArrays& out, st
         if (partition) {
             keysA = reinterpret_cast<std::uint64_t*>(take(8 * E));
             keysB = reinterpret_cast<std::uint64_t*>(take(8 * E));
-            hist = reinterpret_cast<std::uint32_t*>(take(4ull * kRadixBins * tiles));
+            hist = reinterpret_cast<std::uint32_t*>(take(4 * partition_hist_elems(E)));
             total = reinterpret_cast<std::uint32_t*>(take(4ull * kRadixBins));
             return off;
         }
@@ -1066,28 +940,9 @@ int build_blocks(Coo c, std::uint32_t RW, const float* val, BlockArrays& out, st
         // stable passes over the window's bits, the first from the COO
         TCC_HIP_CHECK(partition.take(carve(nullptr, true), st));
         carve(partition.data(), true);
-        const unsigned passes = std::max(1u, (wBits + kRadixBits - 1) / kRadixBits);
-        unsigned shift = c.bBits + 3;
-        for (unsigned p = 0; p < passes; ++p) {
-            const unsigned bits = std::max(1u, wBits / passes + (p < wBits % passes ? 1u : 0u));
-            std::uint64_t* dst = p % 2 ? keysB : keysA;
-            if (p == 0)
-                hipLaunchKernelGGL(part_hist_kernel<true>, dim3(tiles), dim3(kPrimThreads), 0, st, c, nullptr, shift,
-                                   bits, hist, tiles, flags);
-            else
-                hipLaunchKernelGGL(part_hist_kernel<false>, dim3(tiles), dim3(kPrimThreads), 0, st, c, grouped, shift,
-                                   bits, hist, tiles, flags);
-            hipLaunchKernelGGL(digit_scan_kernel, dim3(1u << bits), dim3(1024), 0, st, hist, tiles, total);
-            if (p == 0)
-                hipLaunchKernelGGL(part_scatter_kernel<true>, dim3(tiles), dim3(kPrimThreads), 0, st, c, nullptr, dst,
-                                   shift, bits, hist, tiles, total);
-            else
-                hipLaunchKernelGGL(part_scatter_kernel<false>, dim3(tiles), dim3(kPrimThreads), 0, st, c, grouped, dst,
-                                   shift, bits, hist, tiles, total);
-            TCC_LAUNCH_CHECK();
-            grouped = dst;
-            shift += bits;
-        }
+        std::uint64_t* sorted = nullptr;
+        TCC_HIP_CHECK(partition_by(CooLoad{c, flags}, keysA, keysB, E, c.bBits + 3, wBits, hist, total, &sorted, st));
+        grouped = sorted;
         hipLaunchKernelGGL(window_starts_kernel<true>, perEdge1, dim3(kThreads), 0, st, c, grouped, RW, winStart, flags);
         TCC_LAUNCH_CHECK();
     }
@@ -1153,7 +1008,7 @@ int build_blocks(Coo c, std::uint32_t RW, const float* val, BlockArrays& out, st
     }
     if (rc != TCC_OK || what != Built::Ok) {
         (void)hipStreamSynchronize(st);
-        (void)hipFree(out.base);
+        (void)pool_free(out.base);
         out.base = nullptr;
     }
     return rc;
@@ -1253,7 +1108,7 @@ extern "C" {
 
 int tcc_block_release(void* allocation) {
     clear_last_error();
-    if (allocation) TCC_HIP_CHECK(hipFree(allocation));
+    if (allocation) TCC_HIP_CHECK(pool_free(allocation));
     return TCC_OK;
 }
 
@@ -1295,7 +1150,7 @@ int tcc_coo_to_bcsr_phased(const std::uint32_t* dRow, const std::uint32_t* dCol,
         TCC_HIP_CHECK(arrays.allocate(RW, 0, 0, true));
         if (fill<std::uint32_t>(arrays.off, RW + 1ull, 0u, st) != hipSuccess ||
             fill<std::uint32_t>(arrays.tcOffset, 1, 0u, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess) {
-            (void)hipFree(arrays.base);
+            (void)pool_free(arrays.base);
             set_last_error("HIP error while building an empty BCSR");
             return TCC_ERR_HIP;
         }

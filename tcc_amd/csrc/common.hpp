@@ -135,6 +135,15 @@ __device__ inline std::uint32_t wave_lower_bound(const std::uint32_t* off, std::
     return m == 0 ? hi : lo + static_cast<std::uint32_t>(__builtin_ctzll(m));
 }
 
+// *flag = 1 if any lane's `mine` (one atomic per wave, and none once the flag
+// is seen set).
+__device__ __forceinline__ void raise_flag(std::uint32_t* flag, bool mine) {
+    if (__ballot(mine) == 0) return;
+    if (__lane_id() == static_cast<unsigned>(__builtin_ctzll(__ballot(mine))) &&
+        __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u)
+        atomicOr(flag, 1u);
+}
+
 // counter[idx] += 1 for every calling lane, one atomic per distinct index
 // in the wave: sorted inputs put many lanes of a wave on the same few
 // counters, where per-lane atomics serialise.

@@ -47,6 +47,7 @@
 #include "degree_rank.hpp"
 #include "gather_ops.hpp"
 #include "primitives.hpp"
+#include "scratch.hpp"
 
 namespace tcc {
 namespace {
@@ -162,30 +163,18 @@ __device__ __forceinline__ std::uint64_t tile_index(const std::uint64_t* keys, c
     return keys[tileStart[t]] >> 8;
 }
 
-// dense[t] = tile t holds at least minNnz entries and its step (the
-// stepTiles tiles of one group and step column, adjacent in the sorted
-// order) at least minStepNnz; the number of dense tiles; the largest step
-// column of a dense tile (+1).
+// dense[t] = tile t holds at least minNnz entries; the number of dense tiles;
+// the largest step column of a dense tile (+1).
 __global__ void dense_tiles_kernel(const std::uint64_t* __restrict__ keys, const std::uint32_t* __restrict__ tileStart,
                                    const std::uint32_t* __restrict__ numTiles, std::uint32_t E, std::uint32_t minNnz,
-                                   std::uint32_t minStepNnz, std::uint32_t colSteps, std::uint32_t stepTiles,
-                                   std::uint32_t* __restrict__ dense, std::uint32_t* __restrict__ denseCount,
-                                   std::uint32_t* __restrict__ hubBlocks) {
+                                   std::uint32_t colSteps, std::uint32_t stepTiles, std::uint32_t* __restrict__ dense,
+                                   std::uint32_t* __restrict__ denseCount, std::uint32_t* __restrict__ hubBlocks) {
     const std::uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     bool d = false;
     if (t < *numTiles) {
-        const std::uint32_t nt = *numTiles;
         const std::uint32_t s = tileStart[t];
-        const std::uint32_t e = t + 1 < nt ? tileStart[t + 1] : E;
+        const std::uint32_t e = t + 1 < *numTiles ? tileStart[t + 1] : E;
         d = e - s >= minNnz;
-        if (d && minStepNnz > e - s) {
-            // the step's entries: its tiles before and after t (at most stepTiles - 1 each way)
-            const std::uint64_t step = (keys[s] >> 8) / stepTiles;
-            std::uint32_t first = t, end = t + 1;
-            while (first > 0 && (keys[tileStart[first - 1]] >> 8) / stepTiles == step) --first;
-            while (end < nt && (keys[tileStart[end]] >> 8) / stepTiles == step) ++end;
-            d = (end < nt ? tileStart[end] : E) - tileStart[first] >= minStepNnz;
-        }
         dense[t] = d ? 1u : 0u;
         if (d) atomicMax(hubBlocks, static_cast<std::uint32_t>((keys[s] >> 8) / stepTiles % colSteps) + 1u);
     }
@@ -249,15 +238,15 @@ __global__ void units_per_group_kernel(const std::uint32_t* __restrict__ groupSt
     if (g < NG) units[g] = (groupSteps[g] + unitSteps - 1) / unitSteps;
 }
 
-// Dense tiles' entries into their slots (TF32-rounded values in the
-// A-operand order, or pattern bits), the others into the remainder COO.
+// Value tiles: dense tiles' entries into their slots (TF32-rounded values in
+// the A-operand order), the others into the remainder COO.
 __global__ void place_entries_kernel(const std::uint64_t* __restrict__ keys, const std::uint32_t* __restrict__ perm,
                                      std::uint32_t E, const std::uint32_t* __restrict__ flags,
                                      const std::uint32_t* __restrict__ pos, const std::uint32_t* __restrict__ dense,
                                      const std::uint32_t* __restrict__ slot, const std::uint32_t* __restrict__ restPos,
                                      const std::uint32_t* __restrict__ row, const std::uint32_t* __restrict__ col,
                                      const float* __restrict__ val, float* __restrict__ tileVals,
-                                     std::uint32_t format, std::uint32_t G, std::uint32_t* __restrict__ tileMasks,
+                                     std::uint32_t format,
                                      std::uint32_t* __restrict__ restRow, std::uint32_t* __restrict__ restCol,
                                      float* __restrict__ restVal) {
     const std::uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
@@ -267,14 +256,7 @@ __global__ void place_entries_kernel(const std::uint64_t* __restrict__ keys, con
     const float v = val ? val[src] : 1.0f;
     if (dense[t]) {
         const std::uint32_t i = static_cast<std::uint32_t>(keys[e] >> 4) & 15u, j = static_cast<std::uint32_t>(keys[e]) & 15u;
-        if (format == TCC_TILES_BINARY) {
-            // the step's raw bits (binary_encode_kernel's input): 32 G bytes
-            // per 16-column half h of the step, byte l*(G/2) + rb/2 with
-            // l = 16*(rb%2) + i + 32*(j/8), bit j%8
-            const std::uint32_t step = slot[t] / (2 * G), q = slot[t] % (2 * G), h = q / G, rb = q % G;
-            const std::uint64_t byte = (2ull * step + h) * G * 32 + (16 * (rb % 2) + i + 32 * (j / 8)) * (G / 2) + rb / 2;
-            atomicOr(&tileMasks[byte / 4], 1u << (8 * (byte % 4) + j % 8));
-        } else if (format == TCC_TILES_BF16X2) {
+        if (format == TCC_TILES_BF16X2) {
             // bf16 tile: hi[i][j] at 2(16i + j) bytes, lo 512 bytes further
             std::uint16_t hi, lo;
             bf16_split(tf32_rna(v), hi, lo);
@@ -291,6 +273,189 @@ __global__ void place_entries_kernel(const std::uint64_t* __restrict__ keys, con
         restCol[p] = col[src];
         if (restVal) restVal[p] = v;
     }
+}
+
+// ---- binary steps
+//
+// A binary step stores every entry once the step holds enough of them, and
+// its record has a place for each position, so its entries need no order:
+// the edges are partitioned by step alone (3 passes of u64 keys at 114M
+// edges, where the order of the valued tiles takes 5 of keys and edge
+// numbers), and a key holds its position, so that the original row and column
+// come back from the rank orders.
+//   key = step << pos | row in the group << 5 | column in the step
+// with pos = 13 bits below the step for groups of 16 row blocks, 12 for 8.
+// Kept after the partition are two counts per tile of 4096 keys, the steps
+// and, of the remainder, the edges; a wave then fills one step's raw bits
+// in LDS.  The layout of 57M edges of a 233k-node R-MAT graph, remainder
+// included: 19 -> 4.0 ms of kernels (8.9 of the 19 were degree counts with an
+// atomic per edge, 3.1 the sort, 3.3 lists and marks per 16x16 tile).
+inline unsigned pos_bits(std::uint32_t G) { return G == 16 ? 13 : 12; }
+
+struct StepKeys {
+    const std::uint32_t* row;
+    const std::uint32_t* col;
+    const std::uint32_t* rowRank;
+    const std::uint32_t* colRank;
+    std::uint32_t E, G, colSteps;
+    unsigned pos;
+};
+
+__global__ void step_keys_kernel(StepKeys a, std::uint64_t* __restrict__ keys) {
+    const std::uint64_t e = static_cast<std::uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (e >= a.E) return;
+    const std::uint32_t rr = a.rowRank[a.row[e]], cr = a.colRank[a.col[e]];
+    const std::uint32_t rows = a.G * kTile, g = rr / rows;
+    const std::uint64_t step = static_cast<std::uint64_t>(g) * a.colSteps + cr / (2 * kTile);
+    keys[e] = step << a.pos | (rr - g * rows) << 5 | (cr % (2 * kTile));
+}
+
+// Element e of the partitioned keys (one per lane, a wave's lanes
+// consecutive): whether it is its step's first and whether the step holds at
+// least minNnz entries.  The step's first element is found among the wave's,
+// or, for the step the wave's first element continues, by going back 64
+// elements at a time, at most to minNnz of them.
+struct StepOf {
+    std::uint64_t step;
+    bool head, dense;
+};
+
+__device__ __forceinline__ StepOf step_of(const std::uint64_t* __restrict__ keys, std::uint64_t e, std::uint64_t E,
+                                          std::uint32_t minNnz, unsigned pos) {
+    const unsigned lane = __lane_id();
+    const std::uint64_t w0 = e - lane;  // the wave's first element, below E
+    StepOf s;
+    s.step = keys[e < E ? e : E - 1] >> pos;
+    const std::uint64_t prev = e > 0 ? keys[(e < E ? e : E - 1) - (e < E ? 1 : 0)] >> pos : ~0ull;
+    s.head = e < E && (e == 0 || prev != s.step);
+    const std::uint64_t heads = __ballot(s.head);
+    std::uint64_t first = w0;  // of the step that the wave's first element continues
+    if ((heads & 1ull) == 0) {
+        const std::uint64_t step0 = __shfl(s.step, 0, kWave);
+        while (first > 0 && w0 - first < minNnz) {
+            const std::uint64_t b = first > kWave ? first - kWave : 0;  // elements [b, first)
+            const std::uint64_t i = b + lane;
+            const std::uint64_t other = __ballot(i < first && (keys[i < first ? i : b] >> pos) != step0);
+            if (other) {
+                first = b + 64 - static_cast<std::uint64_t>(__builtin_clzll(other));
+                break;
+            }
+            first = b;
+        }
+    }
+    const std::uint64_t upto = heads & (lane == 63 ? ~0ull : (2ull << lane) - 1ull);
+    const std::uint64_t start = upto ? w0 + (63 - static_cast<unsigned>(__builtin_clzll(upto))) : first;
+    const std::uint64_t last = start + minNnz - 1;
+    s.dense = e < E && (e - start >= minNnz || (last < E && (keys[last] >> pos) == s.step));
+    return s;
+}
+
+constexpr unsigned kStepTile = 4096;
+constexpr unsigned kStepRounds = kStepTile / kThreads;
+
+// counts[0][t] and counts[1][t]: the dense steps that start in tile t, the
+// edges of it that stay in the remainder.
+__global__ void __launch_bounds__(kThreads) step_counts_kernel(const std::uint64_t* __restrict__ keys, std::uint64_t E,
+                                                              std::uint32_t minNnz, std::uint32_t* __restrict__ counts,
+                                                              unsigned tiles, unsigned pos) {
+    __shared__ std::uint32_t sum[2][kThreads / kWave];
+    const unsigned lane = __lane_id(), wave = threadIdx.x / kWave;
+    std::uint32_t steps = 0, rest = 0;
+    for (unsigned r = 0; r < kStepRounds; ++r) {
+        const std::uint64_t w0 = static_cast<std::uint64_t>(blockIdx.x) * kStepTile + (wave * kStepRounds + r) * kWave;
+        if (w0 >= E) break;
+        const StepOf s = step_of(keys, w0 + lane, E, minNnz, pos);
+        steps += static_cast<std::uint32_t>(__popcll(__ballot(s.head && s.dense)));
+        rest += static_cast<std::uint32_t>(__popcll(__ballot(w0 + lane < E && !s.dense)));
+    }
+    if (lane == 0) {
+        sum[0][wave] = steps;
+        sum[1][wave] = rest;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        std::uint32_t t = 0;
+        for (unsigned w = 0; w < kThreads / kWave; ++w) t += sum[threadIdx.x][w];
+        counts[threadIdx.x * tiles + blockIdx.x] = t;
+    }
+}
+
+// The dense steps' first elements and the remainder's COO, at the places the
+// scanned counts give; the largest column of a dense step (+1).
+__global__ void __launch_bounds__(kThreads) step_emit_kernel(const std::uint64_t* __restrict__ keys, std::uint64_t E,
+                                                            std::uint32_t minNnz, const std::uint32_t* __restrict__ counts,
+                                                            unsigned tiles, StepKeys a,
+                                                            const std::uint32_t* __restrict__ rowOrder,
+                                                            const std::uint32_t* __restrict__ colOrder,
+                                                            std::uint32_t* __restrict__ stepStart,
+                                                            std::uint32_t* __restrict__ restRow,
+                                                            std::uint32_t* __restrict__ restCol,
+                                                            std::uint32_t* __restrict__ hubSteps) {
+    __shared__ std::uint32_t sum[2][kThreads / kWave];
+    const unsigned lane = __lane_id(), wave = threadIdx.x / kWave;
+    const std::uint64_t lt = lanemask_lt();
+    std::uint64_t key[kStepRounds];
+    std::uint32_t headBits = 0, restBits = 0, steps = 0, rest = 0, hub = 0;
+#pragma unroll
+    for (unsigned r = 0; r < kStepRounds; ++r) {
+        const std::uint64_t w0 = static_cast<std::uint64_t>(blockIdx.x) * kStepTile + (wave * kStepRounds + r) * kWave;
+        key[r] = 0;
+        if (w0 >= E) continue;
+        const StepOf s = step_of(keys, w0 + lane, E, minNnz, a.pos);
+        key[r] = keys[w0 + lane < E ? w0 + lane : E - 1];
+        const bool h = s.head && s.dense, o = w0 + lane < E && !s.dense;
+        headBits |= h ? 1u << r : 0u;
+        restBits |= o ? 1u << r : 0u;
+        steps += static_cast<std::uint32_t>(__popcll(__ballot(h)));
+        rest += static_cast<std::uint32_t>(__popcll(__ballot(o)));
+        if (h) hub = max(hub, static_cast<std::uint32_t>(s.step % a.colSteps) + 1u);
+    }
+    if (lane == 0) {
+        sum[0][wave] = steps;
+        sum[1][wave] = rest;
+    }
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) hub = max(hub, static_cast<std::uint32_t>(__shfl_xor(static_cast<int>(hub), d, kWave)));
+    // one atomic per wave, and none where the maximum is already as large
+    if (lane == 0 && hub > __hip_atomic_load(hubSteps, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(hubSteps, hub);
+    __syncthreads();
+    std::uint32_t stepAt = counts[blockIdx.x], restAt = counts[tiles + blockIdx.x];
+    for (unsigned w = 0; w < wave; ++w) {
+        stepAt += sum[0][w];
+        restAt += sum[1][w];
+    }
+    const std::uint32_t rows = a.G * kTile;
+#pragma unroll
+    for (unsigned r = 0; r < kStepRounds; ++r) {
+        const std::uint64_t e = static_cast<std::uint64_t>(blockIdx.x) * kStepTile + (wave * kStepRounds + r) * kWave + lane;
+        const bool h = (headBits >> r) & 1u, o = (restBits >> r) & 1u;
+        const std::uint64_t hb = __ballot(h), ob = __ballot(o);
+        if (h) stepStart[stepAt + static_cast<std::uint32_t>(__popcll(hb & lt))] = static_cast<std::uint32_t>(e);
+        if (o) {
+            const std::uint32_t at = restAt + static_cast<std::uint32_t>(__popcll(ob & lt));
+            const std::uint64_t step = key[r] >> a.pos;
+            const std::uint32_t g = static_cast<std::uint32_t>(step / a.colSteps);
+            const std::uint32_t cs = static_cast<std::uint32_t>(step - static_cast<std::uint64_t>(g) * a.colSteps);
+            restRow[at] = rowOrder[static_cast<std::uint64_t>(g) * rows + ((key[r] >> 5) & (rows - 1))];
+            restCol[at] = colOrder[cs * 2 * kTile + (key[r] & 31u)];
+        }
+        stepAt += static_cast<std::uint32_t>(__popcll(hb));
+        restAt += static_cast<std::uint32_t>(__popcll(ob));
+    }
+}
+
+// stepOffset[g] = the first dense step of group g or of a later one.
+__global__ void step_offsets_kernel(const std::uint64_t* __restrict__ keys, const std::uint32_t* __restrict__ stepStart,
+                                    std::uint32_t NS, std::uint32_t NG, std::uint32_t colSteps, unsigned pos,
+                                    std::uint32_t* __restrict__ stepOffset) {
+    const std::uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g > NG) return;
+    std::uint32_t lo = 0, hi = NS;
+    while (lo < hi) {
+        const std::uint32_t mid = (lo + hi) / 2;
+        if ((keys[stepStart[mid]] >> pos) < static_cast<std::uint64_t>(g) * colSteps) lo = mid + 1; else hi = mid;
+    }
+    stepOffset[g] = lo;
 }
 
 // ---- binary tiles: the pattern as operands of the 2:4 sparse MFMA
@@ -323,16 +488,76 @@ __device__ __forceinline__ bool crowded_nibble(std::uint64_t x) {
     return ((c + 0x1111111111111111ull) & 0xCCCCCCCCCCCCCCCCull) != 0;      // count + 1 >= 4
 }
 
-// layers[s] = 2 when a nibble of step s holds more than two entries, else 1
-// (one wave per step).
-__global__ void binary_layers_kernel(const std::uint32_t* __restrict__ raw, std::uint32_t NS, std::uint32_t G,
-                                     std::uint32_t* __restrict__ layers) {
-    const std::uint64_t s = (static_cast<std::uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
-    if (s >= NS) return;
-    const unsigned lane = __lane_id();
-    const bool crowded = crowded_nibble(raw_lane_bytes(raw, G, s, 0, lane)) || crowded_nibble(raw_lane_bytes(raw, G, s, 1, lane));
-    const std::uint64_t any = __ballot(crowded);
-    if (lane == 0) layers[s] = any ? 2u : 1u;
+// One wave per dense step: its entries' bits (32 G bytes per 16-column half
+// h: byte l*(G/2) + rb/2 with l = 16*(rb%2) + i + 32*(j/8), bit j%8, for row
+// i of row block rb and column j of the half) put together in LDS and
+// written out, the step's column, its layers (2 when a nibble holds more
+// than two entries, else 1), the 16x16 tiles it fills; a bit that is set
+// already is a duplicate edge.
+constexpr unsigned kRawWaves = 8;
+__global__ void __launch_bounds__(kRawWaves * kWave) step_raw_kernel(const std::uint64_t* __restrict__ keys,
+                                                                    std::uint64_t E,
+                                                                    const std::uint32_t* __restrict__ stepStart,
+                                                                    std::uint32_t NS, std::uint32_t G,
+                                                                    std::uint32_t colSteps, unsigned pos,
+                                                                    std::uint32_t* __restrict__ raw,
+                                                                    std::uint32_t* __restrict__ stepCol,
+                                                                    std::uint32_t* __restrict__ layers,
+                                                                    std::uint32_t* __restrict__ numTiles,
+                                                                    std::uint32_t* __restrict__ err) {
+    __shared__ __attribute__((aligned(16))) std::uint32_t bits[kRawWaves][256];
+    const unsigned lane = __lane_id(), wave = threadIdx.x / kWave;
+    std::uint32_t* mine = bits[wave];
+    const std::uint32_t words = 16 * G;  // of a step
+    std::uint32_t tiles = 0;
+    bool dup = false;
+    for (std::uint32_t s = blockIdx.x * kRawWaves + wave; s < NS; s += gridDim.x * kRawWaves) {
+        for (std::uint32_t i = lane; i < words; i += kWave) mine[i] = 0;
+        __builtin_amdgcn_wave_barrier();
+        const std::uint64_t e0 = stepStart[s];
+        const std::uint64_t step = keys[e0] >> pos;
+        for (std::uint64_t e = e0; e < E; e += kWave) {
+            const std::uint64_t k = keys[e + lane < E ? e + lane : E - 1];
+            const bool in = e + lane < E && (k >> pos) == step;
+            if (in) {
+                const std::uint32_t row = static_cast<std::uint32_t>(k >> 5) & (G * kTile - 1), c = static_cast<std::uint32_t>(k) & 31u;
+                const std::uint32_t rb = row / kTile, i = row % kTile, h = c / kTile, j = c % kTile;
+                const std::uint32_t byte = h * G * 32 + (16 * (rb % 2) + i + 32 * (j / 8)) * (G / 2) + rb / 2;
+                const std::uint32_t bit = 1u << (8 * (byte % 4) + j % 8);
+                dup |= (atomicOr(&mine[byte / 4], bit) & bit) != 0;
+            }
+            if (__ballot(in) != ~0ull) break;
+        }
+        __builtin_amdgcn_wave_barrier();
+        std::uint32_t* out = raw + static_cast<std::uint64_t>(s) * words;
+        for (std::uint32_t i = lane; i < words; i += kWave) out[i] = mine[i];
+        bool crowded = false;
+        for (std::uint32_t h = 0; h < 2; ++h) {
+            // this lane's G/2 bytes of the half, as raw_lane_bytes reads them
+            const std::uint32_t at = (h * G * 32 + lane * (G / 2)) / 4;
+            std::uint64_t w = mine[at];
+            if (G == 16) w |= static_cast<std::uint64_t>(mine[at + 1]) << 32;
+            crowded |= crowded_nibble(w);
+            for (std::uint32_t t = 0; t < G / 2; ++t) {
+                const std::uint64_t m = __ballot(((w >> (8 * t)) & 0xFFu) != 0);
+                tiles += ((m & 0x0000FFFF0000FFFFull) != 0) + ((m & 0xFFFF0000FFFF0000ull) != 0);
+            }
+        }
+        const std::uint64_t any = __ballot(crowded);
+        if (lane == 0) {
+            layers[s] = any ? 2u : 1u;
+            stepCol[s] = static_cast<std::uint32_t>(step % colSteps);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (__ballot(dup) && lane == 0) atomicMax(err, 2u);
+    __shared__ std::uint32_t sum[kRawWaves];
+    if (lane == 0) sum[wave] = tiles;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (unsigned w = 1; w < kRawWaves; ++w) tiles += sum[w];
+        if (tiles) atomicAdd(numTiles, tiles);
+    }
 }
 
 // subOffset[g] = first sub-step of group g (g <= NG); groupSub[g] = its
@@ -547,14 +772,6 @@ __global__ void bcsr_expand_kernel(tcc_bcsr A, const std::uint32_t* __restrict__
         ++k;
     }
 }
-
-template <typename T>
-struct DevBuf {
-    T* p = nullptr;
-    ~DevBuf() {
-        if (p) (void)hipFree(p);
-    }
-};
 
 // ---------------------------------------------------------------- SpMM
 
@@ -1584,6 +1801,8 @@ int build_hybrid(const HybridParams& P, tcc_hybrid* out, void* stream) {
     const std::uint64_t Vn = std::max<std::uint64_t>({En, rowSlots, numCols});
     const unsigned tileBits = std::max(1u, rank_bits(static_cast<std::uint64_t>(NG) * CB * G));
     TCC_REQUIRE(tileBits + 8 <= 64, TCC_ERR_UNSUPPORTED, "hybrid: tile key exceeds 64 bits");
+    const unsigned stepBits = rank_bits(static_cast<std::uint64_t>(NG) * colSteps);  // binary: no more bits than a tile key
+    const unsigned stepTileCount = static_cast<unsigned>((En + kStepTile - 1) / kStepTile);
     const std::uint64_t tempElems = std::max({radix_temp_elems(Vn), scan_temp_elems(En + 1),
                                               scan_temp_elems(static_cast<std::uint64_t>(NG) + 1)});
 
@@ -1591,7 +1810,8 @@ int build_hybrid(const HybridParams& P, tcc_hybrid* out, void* stream) {
     std::uint32_t *permA, *permB, *flags, *pos, *tileStart, *dense, *stepHead, *stepPos, *slot, *restFlag, *restPos,
         *rowDeg, *colDeg, *rowRank, *colRank, *rowOrder, *colOrder, *groupSteps, *unitCount, *temp, *small, *restRow,
         *restCol;
-    float* restVal;
+    float* restVal = nullptr;
+    std::uint32_t *stepCounts = nullptr, *stepStart = nullptr;
     auto carve = [&](char* base) {
         std::size_t off = 0;
         auto take = [&](std::size_t bytes) {
@@ -1601,58 +1821,88 @@ int build_hybrid(const HybridParams& P, tcc_hybrid* out, void* stream) {
         };
         keysA = reinterpret_cast<std::uint64_t*>(take(8 * Vn));
         keysB = reinterpret_cast<std::uint64_t*>(take(8 * Vn));
-        permA = reinterpret_cast<std::uint32_t*>(take(4 * En));
-        permB = reinterpret_cast<std::uint32_t*>(take(4 * En));
-        flags = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
-        pos = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
-        tileStart = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
-        dense = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
-        stepHead = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
-        stepPos = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
-        slot = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
-        restFlag = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
-        restPos = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
+        if (binary) {
+            stepCounts = reinterpret_cast<std::uint32_t*>(take(8ull * stepTileCount));
+            stepStart = reinterpret_cast<std::uint32_t*>(take(4 * (En / P.minStepNnz + 1)));
+        } else {
+            permA = reinterpret_cast<std::uint32_t*>(take(4 * En));
+            permB = reinterpret_cast<std::uint32_t*>(take(4 * En));
+            flags = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
+            pos = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
+            tileStart = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
+            dense = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
+            stepHead = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
+            stepPos = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
+            slot = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
+            restFlag = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
+            restPos = reinterpret_cast<std::uint32_t*>(take(4 * (En + 1)));
+            groupSteps = reinterpret_cast<std::uint32_t*>(take(4 * (NG + 1)));
+            restRow = reinterpret_cast<std::uint32_t*>(take(4 * En));
+            restCol = reinterpret_cast<std::uint32_t*>(take(4 * En));
+            restVal = reinterpret_cast<float*>(take(4 * En));
+        }
         rowDeg = reinterpret_cast<std::uint32_t*>(take(4 * (numRows + 1)));
         colDeg = reinterpret_cast<std::uint32_t*>(take(4 * (numCols + 1)));
         rowRank = reinterpret_cast<std::uint32_t*>(take(4 * (numRows + 1)));
         colRank = reinterpret_cast<std::uint32_t*>(take(4 * (numCols + 1)));
         rowOrder = reinterpret_cast<std::uint32_t*>(take(4ull * rowSlots));
         colOrder = reinterpret_cast<std::uint32_t*>(take(4 * (numCols + 1)));
-        groupSteps = reinterpret_cast<std::uint32_t*>(take(4 * (NG + 1)));
         unitCount = reinterpret_cast<std::uint32_t*>(take(4 * (NG + 1)));
-        restRow = reinterpret_cast<std::uint32_t*>(take(4 * En));
-        restCol = reinterpret_cast<std::uint32_t*>(take(4 * En));
-        restVal = reinterpret_cast<float*>(take(4 * En));
         temp = reinterpret_cast<std::uint32_t*>(take(4 * tempElems));
         // [0]=err [1]=tiles [2]=steps [3]=rest [4]=units [5]=hubBlocks [6]=dense tiles [7]=sub-steps
         small = reinterpret_cast<std::uint32_t*>(take(256));
         return off;
     };
     const std::size_t scratchBytes = carve(nullptr);
-    DevBuf<char> scratch;
-    TCC_HIP_CHECK(hipMalloc(&scratch.p, scratchBytes));
-    carve(scratch.p);
+    Scratch scratch;
+    TCC_HIP_CHECK(scratch.take(scratchBytes, st));
+    carve(scratch.data());
+    // small[0..8) on the host, after the work queued so far
+    std::uint32_t hostSmall[8] = {};
+    auto read_small = [&]() -> int {
+        TCC_HIP_CHECK(hipMemcpyAsync(scratch.mailHost(), small, sizeof(hostSmall), hipMemcpyDeviceToHost, st));
+        TCC_HIP_CHECK(scratch.wait());
+        for (unsigned i = 0; i < 8; ++i) hostSmall[i] = scratch.read()[i];
+        return TCC_OK;
+    };
 
     TCC_HIP_CHECK(fill<std::uint32_t>(small, 64, 0u, st));
     TCC_HIP_CHECK(fill<std::uint32_t>(rowDeg, numRows, 0u, st));
     TCC_HIP_CHECK(fill<std::uint32_t>(colDeg, numCols, 0u, st));
-    TCC_HIP_CHECK(fill<std::uint32_t>(groupSteps, NG + 1, 0u, st));
-    // dense[] and stepHead[] are scanned over E entries; only the first
-    // (tile count) are set below
-    TCC_HIP_CHECK(fill<std::uint32_t>(dense, En, 0u, st));
-    TCC_HIP_CHECK(fill<std::uint32_t>(stepHead, En, 0u, st));
+    if (!binary) {
+        TCC_HIP_CHECK(fill<std::uint32_t>(groupSteps, NG + 1, 0u, st));
+        // dense[] and stepHead[] are scanned over E entries; only the first
+        // (tile count) are set below
+        TCC_HIP_CHECK(fill<std::uint32_t>(dense, En, 0u, st));
+        TCC_HIP_CHECK(fill<std::uint32_t>(stepHead, En, 0u, st));
+    }
     TCC_HIP_CHECK(degree_histogram(P.row, E, numRows, rowDeg, small, st));
     TCC_HIP_CHECK(degree_histogram(P.col, E, numCols, colDeg, small, st));
-    std::uint32_t hostSmall[8] = {};
-    TCC_HIP_CHECK(hipMemcpyAsync(hostSmall, small, sizeof(hostSmall), hipMemcpyDeviceToHost, st));
-    TCC_HIP_CHECK(hipStreamSynchronize(st));
+    std::uint32_t* perm = nullptr;
+    if (const int rc = read_small()) return rc;
     TCC_REQUIRE(hostSmall[0] == 0, TCC_ERR_INVALID_ARGUMENT, "COO index out of range");
-    TCC_HIP_CHECK(degree_ranks(rowDeg, numRows, rowSlots, rowRank, rowOrder, keysA, keysB, temp, st));
-    TCC_HIP_CHECK(degree_ranks(colDeg, numCols, numCols, colRank, colOrder, keysA, keysB, temp, st));
+    TCC_HIP_CHECK(degree_ranks(rowDeg, numRows, E, rowSlots, rowRank, rowOrder, keysA, keysB, temp, st));
+    TCC_HIP_CHECK(degree_ranks(colDeg, numCols, E, numCols, colRank, colOrder, keysA, keysB, temp, st));
 
     std::uint64_t* sorted = keysA;
-    std::uint32_t* perm = permA;
-    if (E > 0) {
+    if (E > 0 && binary) {
+        // the edges partitioned by step; steps and remainder counted, then written
+        const StepKeys a{P.row, P.col, rowRank, colRank, E, G, colSteps, pos_bits(G)};
+        hipLaunchKernelGGL(step_keys_kernel, dim3(grid_for(E, kThreads)), dim3(kThreads), 0, st, a, keysB);
+        TCC_LAUNCH_CHECK();
+        TCC_HIP_CHECK(partition_by(KeyLoad{keysB, E}, keysA, keysB, E, a.pos, stepBits, temp,
+                                   temp + partition_hist_elems(E), &sorted, st));
+        // the remainder's COO over the elements that the last pass read
+        restRow = reinterpret_cast<std::uint32_t*>(sorted == keysA ? keysB : keysA);
+        restCol = restRow + E;
+        hipLaunchKernelGGL(step_counts_kernel, dim3(stepTileCount), dim3(kThreads), 0, st, sorted, E, P.minStepNnz,
+                           stepCounts, stepTileCount, a.pos);
+        hipLaunchKernelGGL(row_scan_kernel, dim3(2), dim3(1024), 0, st, stepCounts, stepTileCount, small + 2);
+        hipLaunchKernelGGL(step_emit_kernel, dim3(stepTileCount), dim3(kThreads), 0, st, sorted, E, P.minStepNnz,
+                           stepCounts, stepTileCount, a, rowOrder, colOrder, stepStart, restRow, restCol, small + 5);
+        TCC_LAUNCH_CHECK();
+    } else if (E > 0) {
+        perm = permA;
         hipLaunchKernelGGL(tile_keys_kernel, dim3(grid_for(E, kThreads)), dim3(kThreads), 0, st, P.row, P.col, E,
                            rowRank, colRank, CB, G, keysA, permA);
         TCC_LAUNCH_CHECK();
@@ -1663,7 +1913,7 @@ int build_hybrid(const HybridParams& P, tcc_hybrid* out, void* stream) {
         hipLaunchKernelGGL(tile_start_kernel, dim3(grid_for(E, kThreads)), dim3(kThreads), 0, st, flags, pos, E,
                            tileStart);
         hipLaunchKernelGGL(dense_tiles_kernel, dim3(grid_for(E, kThreads)), dim3(kThreads), 0, st, sorted, tileStart,
-                           small + 1, E, P.minTileNnz, P.minStepNnz, colSteps, stepTiles, dense, small + 6, small + 5);
+                           small + 1, E, P.minTileNnz, colSteps, stepTiles, dense, small + 6, small + 5);
         hipLaunchKernelGGL(step_heads_kernel, dim3(grid_for(E, kThreads)), dim3(kThreads), 0, st, sorted, tileStart,
                            small + 1, dense, stepTiles, colSteps, stepHead, groupSteps);
         TCC_LAUNCH_CHECK();
@@ -1680,19 +1930,17 @@ int build_hybrid(const HybridParams& P, tcc_hybrid* out, void* stream) {
         TCC_LAUNCH_CHECK();
         TCC_HIP_CHECK(exclusive_scan(unitCount, unitCount, NG, small + 4, temp, st));
     }
-    TCC_HIP_CHECK(hipMemcpyAsync(hostSmall, small, sizeof(hostSmall), hipMemcpyDeviceToHost, st));
-    TCC_HIP_CHECK(hipStreamSynchronize(st));
+    if (const int rc = read_small()) return rc;
     TCC_REQUIRE(hostSmall[0] == 0, TCC_ERR_INVALID_ARGUMENT,
                 hostSmall[0] == 2 ? "duplicate (row, col) entries in the COO input" : "COO index out of range");
     const std::uint32_t NS = E > 0 ? hostSmall[2] : 0;
     const std::uint32_t NR = E > 0 ? hostSmall[3] : 0;
-    const std::uint32_t ND = E > 0 ? hostSmall[6] : 0;
     const std::uint32_t hubCols = std::min(hostSmall[5] * (binary ? 2 * kTile : kTile), numCols);
 
     // Binary tiles: the steps' raw bits, their layers (a second one where a
     // nibble holds more than two entries) and the sub-steps the units cut.
     std::uint32_t NSS = NS;  // sub-steps
-    DevBuf<char> binScratch;
+    Scratch binScratch;
     std::uint32_t *raw = nullptr, *stepColTmp = nullptr, *subPos = nullptr, *subOffset = nullptr;
     if (binary) {
         const std::uint64_t NS1 = static_cast<std::uint64_t>(NS) + 1;
@@ -1713,23 +1961,16 @@ int build_hybrid(const HybridParams& P, tcc_hybrid* out, void* stream) {
             groupSub = take(4ull * (NG + 1));
             return off;
         };
-        TCC_HIP_CHECK(hipMalloc(&binScratch.p, carveBin(nullptr)));
-        carveBin(binScratch.p);
-        TCC_HIP_CHECK(fill<std::uint32_t>(raw, 16ull * G * NS1, 0u, st));
-        if (E > 0) {
-            hipLaunchKernelGGL(tile_slots_kernel, dim3(grid_for(E, kThreads)), dim3(kThreads), 0, st, sorted, tileStart,
-                               small + 1, dense, stepHead, stepPos, stepTiles, colSteps, slot, stepColTmp);
-            hipLaunchKernelGGL(place_entries_kernel, dim3(grid_for(E, kThreads)), dim3(kThreads), 0, st, sorted, perm,
-                               E, flags, pos, dense, slot, restPos, P.row, P.col, P.val, nullptr, P.format, G, raw,
-                               restRow, restCol, P.val ? restVal : nullptr);
-            TCC_LAUNCH_CHECK();
-        }
-        TCC_HIP_CHECK(exclusive_scan(groupSteps, stepOffset, NG, stepOffset + NG, temp, st));
+        TCC_HIP_CHECK(binScratch.take(carveBin(nullptr), st));
+        carveBin(binScratch.data());
+        hipLaunchKernelGGL(step_offsets_kernel, dim3(grid_for(NG + 1, kThreads)), dim3(kThreads), 0, st, sorted,
+                           stepStart, NS, NG, colSteps, pos_bits(G), stepOffset);
         if (NS > 0) {
-            hipLaunchKernelGGL(binary_layers_kernel, dim3(grid_for(static_cast<std::uint64_t>(NS) * kWave, kThreads)),
-                               dim3(kThreads), 0, st, raw, NS, G, layers);
-            TCC_LAUNCH_CHECK();
+            const unsigned blocks = std::min<unsigned>((NS + kRawWaves - 1) / kRawWaves, device_cus() * 4);
+            hipLaunchKernelGGL(step_raw_kernel, dim3(blocks), dim3(kRawWaves * kWave), 0, st, sorted, E, stepStart, NS, G,
+                               colSteps, pos_bits(G), raw, stepColTmp, layers, small + 6, small);
         }
+        TCC_LAUNCH_CHECK();
         TCC_HIP_CHECK(exclusive_scan(layers, subPos, NS, subPos + NS, temp, st));
         hipLaunchKernelGGL(sub_offsets_kernel, dim3(grid_for(NG + 1, kThreads)), dim3(kThreads), 0, st, stepOffset,
                            subPos, NG, subOffset, groupSub);
@@ -1738,11 +1979,12 @@ int build_hybrid(const HybridParams& P, tcc_hybrid* out, void* stream) {
         TCC_LAUNCH_CHECK();
         TCC_HIP_CHECK(exclusive_scan(unitCount, unitCount, NG, small + 4, temp, st));
         TCC_HIP_CHECK(hipMemcpyAsync(small + 7, subPos + NS, 4, hipMemcpyDeviceToDevice, st));
-        TCC_HIP_CHECK(hipMemcpyAsync(hostSmall, small, sizeof(hostSmall), hipMemcpyDeviceToHost, st));
-        TCC_HIP_CHECK(hipStreamSynchronize(st));
+        if (const int rc = read_small()) return rc;
+        TCC_REQUIRE(hostSmall[0] == 0, TCC_ERR_INVALID_ARGUMENT, "duplicate (row, col) entries in the COO input");
         NSS = hostSmall[7];
     }
     const std::uint32_t NU = hostSmall[4];
+    const std::uint32_t ND = E > 0 ? hostSmall[6] : 0;
 
     // tiles part: rowOrder[rowSlots] hubColOrder[hubCols] groupStepOffset[NG+1] unitFirst[NG+1] stepCol[NS]
     // units[3 NU] unitOrder[NU] unitPartial[NU] sharedGroups[3 NG] then the format's tiles (one more step, of
@@ -1762,7 +2004,7 @@ int build_hybrid(const HybridParams& P, tcc_hybrid* out, void* stream) {
         tilesBytes += align_up(4ull * kTileVals * G * (NS + 1));
     }
     char* o = nullptr;
-    TCC_HIP_CHECK(hipMalloc(&o, tilesBytes));
+    TCC_HIP_CHECK(pool_malloc(reinterpret_cast<void**>(&o), tilesBytes));
     char* q = o;
     auto takeOut = [&](std::size_t bytes) {
         char* p = q;
@@ -1792,7 +2034,8 @@ int build_hybrid(const HybridParams& P, tcc_hybrid* out, void* stream) {
         oTileVals = reinterpret_cast<float*>(takeOut(4ull * kTileVals * G * (NS + 1)));
     }
     auto fail = [&](int rc) {
-        (void)hipFree(o);
+        (void)hipStreamSynchronize(st);
+        (void)pool_free(o);
         return rc;
     };
     bool ok = hipMemcpyAsync(oRowOrder, rowOrder, 4ull * rowSlots, hipMemcpyDeviceToDevice, st) == hipSuccess &&
@@ -1826,27 +2069,27 @@ int build_hybrid(const HybridParams& P, tcc_hybrid* out, void* stream) {
         hipLaunchKernelGGL(tile_slots_kernel, dim3(grid_for(E, kThreads)), dim3(kThreads), 0, st, sorted, tileStart,
                            small + 1, dense, stepHead, stepPos, stepTiles, colSteps, slot, oStepCol);
         hipLaunchKernelGGL(place_entries_kernel, dim3(grid_for(E, kThreads)), dim3(kThreads), 0, st, sorted, perm, E,
-                           flags, pos, dense, slot, restPos, P.row, P.col, P.val, oTileVals, P.format, G, oTileMasks,
-                           restRow, restCol, P.val ? restVal : nullptr);
+                           flags, pos, dense, slot, restPos, P.row, P.col, P.val, oTileVals, P.format, restRow,
+                           restCol, P.val ? restVal : nullptr);
     }
     hipLaunchKernelGGL(group_units_kernel, dim3(grid_for(NG, kThreads)), dim3(kThreads), 0, st, oGroupStepOffset,
                        oUnitFirst, NG, P.unitSteps, oUnits);
     // partial-sum slots of the units of shared groups, and the shared groups
     std::uint32_t shared[2] = {};  // units with a slot, shared groups
-    DevBuf<char> slotScratch;
+    Scratch slotScratch;
     {
         const std::uint64_t n = std::max<std::uint64_t>(NU, NG) + 1;
         const std::size_t bytes = 4 * align_up(4 * n) + align_up(4 * scan_temp_elems(n)) + 256;
-        if (hipMalloc(&slotScratch.p, bytes) != hipSuccess) {
+        if (slotScratch.take(bytes, st) != hipSuccess) {
             set_last_error("out of device memory for the hub tiles' partial slots");
             return fail(TCC_ERR_NO_MEMORY);
         }
-        auto* groupShared = reinterpret_cast<std::uint32_t*>(slotScratch.p);
-        auto* groupPos = reinterpret_cast<std::uint32_t*>(slotScratch.p + align_up(4 * n));
-        auto* unitShared = reinterpret_cast<std::uint32_t*>(slotScratch.p + 2 * align_up(4 * n));
-        auto* unitPos = reinterpret_cast<std::uint32_t*>(slotScratch.p + 3 * align_up(4 * n));
-        auto* totals = reinterpret_cast<std::uint32_t*>(slotScratch.p + 4 * align_up(4 * n));
-        auto* scanTemp = reinterpret_cast<std::uint32_t*>(slotScratch.p + 4 * align_up(4 * n) + 256);
+        auto* groupShared = reinterpret_cast<std::uint32_t*>(slotScratch.data());
+        auto* groupPos = reinterpret_cast<std::uint32_t*>(slotScratch.data() + align_up(4 * n));
+        auto* unitShared = reinterpret_cast<std::uint32_t*>(slotScratch.data() + 2 * align_up(4 * n));
+        auto* unitPos = reinterpret_cast<std::uint32_t*>(slotScratch.data() + 3 * align_up(4 * n));
+        auto* totals = reinterpret_cast<std::uint32_t*>(slotScratch.data() + 4 * align_up(4 * n));
+        auto* scanTemp = reinterpret_cast<std::uint32_t*>(slotScratch.data() + 4 * align_up(4 * n) + 256);
         hipLaunchKernelGGL(shared_groups_kernel, dim3(grid_for(NG, kThreads)), dim3(kThreads), 0, st, oUnitFirst, NG,
                            groupShared);
         ok = exclusive_scan(groupShared, groupPos, NG, totals + 1, scanTemp, st) == hipSuccess;
@@ -1862,7 +2105,7 @@ int build_hybrid(const HybridParams& P, tcc_hybrid* out, void* stream) {
             ok = fill<std::uint32_t>(totals, 1, 0u, st) == hipSuccess;
         }
         ok = ok && hipGetLastError() == hipSuccess &&
-             hipMemcpyAsync(shared, totals, sizeof(shared), hipMemcpyDeviceToHost, st) == hipSuccess;
+             hipMemcpyAsync(scratch.mailHost(), totals, sizeof(shared), hipMemcpyDeviceToHost, st) == hipSuccess;
         if (!ok) {
             set_last_error("HIP error while numbering the hub tiles' partial sums");
             return fail(TCC_ERR_HIP);
@@ -1870,17 +2113,17 @@ int build_hybrid(const HybridParams& P, tcc_hybrid* out, void* stream) {
     }
     // launch order: units by the column block of their first step (stable);
     // binary tiles: the largest size bucket first
-    DevBuf<char> orderScratch;
+    Scratch orderScratch;
     if (NU > 0) {
         const std::uint64_t tempElems = radix_temp_elems(NU);
         const std::size_t bytes = align_up(16ull * NU) + align_up(4ull * NU) + align_up(4 * tempElems);
-        if (hipMalloc(&orderScratch.p, bytes) != hipSuccess) {
+        if (orderScratch.take(bytes, st) != hipSuccess) {
             set_last_error("out of device memory for the hub tiles' unit order");
             return fail(TCC_ERR_NO_MEMORY);
         }
-        auto* keys = reinterpret_cast<std::uint64_t*>(orderScratch.p);
-        auto* vals = reinterpret_cast<std::uint32_t*>(orderScratch.p + align_up(16ull * NU));
-        auto* sortTemp = reinterpret_cast<std::uint32_t*>(orderScratch.p + align_up(16ull * NU) + align_up(4ull * NU));
+        auto* keys = reinterpret_cast<std::uint64_t*>(orderScratch.data());
+        auto* vals = reinterpret_cast<std::uint32_t*>(orderScratch.data() + align_up(16ull * NU));
+        auto* sortTemp = reinterpret_cast<std::uint32_t*>(orderScratch.data() + align_up(16ull * NU) + align_up(4ull * NU));
         unsigned bits = 0;
         while (bits < 32 && (static_cast<std::uint64_t>(CB) - 1) >> bits) ++bits;
         hipLaunchKernelGGL(unit_order_keys_kernel, dim3(grid_for(NU, kThreads)), dim3(kThreads), 0, st, oUnits, oStepCol,
@@ -1897,10 +2140,16 @@ int build_hybrid(const HybridParams& P, tcc_hybrid* out, void* stream) {
             return fail(TCC_ERR_HIP);
         }
     }
-    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) {
+    if (hipGetLastError() != hipSuccess || scratch.wait() != hipSuccess) {
         set_last_error("HIP error while building the hub tiles");
         return fail(TCC_ERR_HIP);
     }
+    shared[0] = scratch.read()[0];
+    shared[1] = scratch.read()[1];
+    // nothing is queued on these any more
+    binScratch.idle();
+    slotScratch.idle();
+    orderScratch.idle();
     // the remainder: an ordinary or phased BCSR of the entries outside dense tiles
     tcc_bcsr rest{};
     void* restAlloc = nullptr;
@@ -1960,8 +2209,8 @@ extern "C" {
 int tcc_hybrid_release(tcc_hybrid* H) {
     clear_last_error();
     if (!H) return TCC_OK;
-    if (H->tilesAllocation) TCC_HIP_CHECK(hipFree(H->tilesAllocation));
-    if (H->restAllocation) TCC_HIP_CHECK(hipFree(H->restAllocation));
+    if (H->tilesAllocation) TCC_HIP_CHECK(pool_free(H->tilesAllocation));
+    if (H->restAllocation) TCC_HIP_CHECK(pool_free(H->restAllocation));
     std::memset(H, 0, sizeof(*H));
     return TCC_OK;
 }
@@ -2041,28 +2290,28 @@ int tcc_hybrid_from_bcsr(const tcc_bcsr* A, int useValues, std::uint32_t minStep
     // remainder holds 9.8% of the entries), 4 behind value tiles (35%)
     if (phases == 0) phases = A->num_rowWindows && B >= 64ull * A->num_rowWindows ? (useValues ? 4 : 2) : 1;
     // block counts, their scan, then the entries
-    DevBuf<char> scratch;
+    Scratch scratch, coo;
     const std::uint64_t Bn = std::max<std::uint32_t>(B, 1);
     const std::size_t headBytes = 2 * align_up(4 * (Bn + 1)) + align_up(4 * scan_temp_elems(Bn + 1)) + 256;
-    TCC_HIP_CHECK(hipMalloc(&scratch.p, headBytes));
-    auto* counts = reinterpret_cast<std::uint32_t*>(scratch.p);
-    auto* offset = reinterpret_cast<std::uint32_t*>(scratch.p + align_up(4 * (Bn + 1)));
-    auto* total = reinterpret_cast<std::uint32_t*>(scratch.p + 2 * align_up(4 * (Bn + 1)));
-    auto* temp = reinterpret_cast<std::uint32_t*>(scratch.p + 2 * align_up(4 * (Bn + 1)) + 256);
+    TCC_HIP_CHECK(scratch.take(headBytes, st));
+    auto* counts = reinterpret_cast<std::uint32_t*>(scratch.data());
+    auto* offset = reinterpret_cast<std::uint32_t*>(scratch.data() + align_up(4 * (Bn + 1)));
+    auto* total = reinterpret_cast<std::uint32_t*>(scratch.data() + 2 * align_up(4 * (Bn + 1)));
+    auto* temp = reinterpret_cast<std::uint32_t*>(scratch.data() + 2 * align_up(4 * (Bn + 1)) + 256);
     std::uint32_t E = 0;
     if (B > 0) {
         hipLaunchKernelGGL(bcsr_entry_counts_kernel, dim3(grid_for(B, kThreads)), dim3(kThreads), 0, st, *A, counts);
         TCC_LAUNCH_CHECK();
         TCC_HIP_CHECK(exclusive_scan(counts, offset, B, total, temp, st));
-        TCC_HIP_CHECK(hipMemcpyAsync(&E, total, 4, hipMemcpyDeviceToHost, st));
-        TCC_HIP_CHECK(hipStreamSynchronize(st));
+        TCC_HIP_CHECK(hipMemcpyAsync(scratch.mailHost(), total, 4, hipMemcpyDeviceToHost, st));
+        TCC_HIP_CHECK(scratch.wait());
+        E = scratch.read()[0];
     }
-    DevBuf<char> coo;
     const std::uint64_t En = std::max<std::uint32_t>(E, 1);
-    TCC_HIP_CHECK(hipMalloc(&coo.p, 3 * align_up(4 * En)));
-    auto* row = reinterpret_cast<std::uint32_t*>(coo.p);
-    auto* col = reinterpret_cast<std::uint32_t*>(coo.p + align_up(4 * En));
-    auto* val = reinterpret_cast<float*>(coo.p + 2 * align_up(4 * En));
+    TCC_HIP_CHECK(coo.take(3 * align_up(4 * En), st));
+    auto* row = reinterpret_cast<std::uint32_t*>(coo.data());
+    auto* col = reinterpret_cast<std::uint32_t*>(coo.data() + align_up(4 * En));
+    auto* val = reinterpret_cast<float*>(coo.data() + 2 * align_up(4 * En));
     if (E > 0) {
         hipLaunchKernelGGL(bcsr_expand_kernel, dim3(grid_for(B, kThreads)), dim3(kThreads), 0, st, *A, offset,
                            useValues != 0, row, col, val);

@@ -201,14 +201,13 @@ __global__ void __launch_bounds__(kPrimThreads) radix_hist_kernel(const std::uin
 }
 
 // Stable scatter: position = global offset of (digit, tile) + keys of the
-// same digit in earlier waves of the tile + earlier keys in this wave.  With
-// PAYLOAD, a u32 value travels with each key, and the tile is first ordered
-// by digit in LDS and then written out in that order, so that consecutive
-// threads write consecutive addresses of a digit's run: the key-value passes
-// took 2.4 ms each at 114M keys written from their lanes, 1.2 ms staged.
-// Keys alone are written from their lanes (staged: 0.77 against 0.73 ms, as
-// the 32 KB of LDS cost occupancy).
-template <bool PAYLOAD>
+// same digit in earlier waves of the tile + earlier keys in this wave.  A u32
+// value travels with each key, and the tile is first ordered by digit in LDS
+// and then written out in that order, so that consecutive threads write
+// consecutive addresses of a digit's run: the key-value passes took 2.4 ms
+// each at 114M keys written from their lanes, 1.2 ms staged.  (Keys alone,
+// partition_by below, are written from their lanes: staged 0.77 against 0.73
+// ms, as the 32 KB of LDS cost occupancy.)
 __global__ void __launch_bounds__(kPrimThreads) radix_scatter_kernel(const std::uint64_t* __restrict__ keysIn,
                                                                     std::uint64_t* __restrict__ keysOut,
                                                                     const std::uint32_t* __restrict__ valsIn,
@@ -220,8 +219,8 @@ __global__ void __launch_bounds__(kPrimThreads) radix_scatter_kernel(const std::
     __shared__ std::uint32_t gbase[kRadixBins];   // global start of (digit, this tile)
     __shared__ std::uint32_t tstart[kRadixBins];  // start of the digit's run in the tile
     __shared__ std::uint32_t waveSum[kPrimWaves];
-    __shared__ std::uint64_t skeys[PAYLOAD ? kPrimTile : 1];
-    __shared__ std::uint32_t svals[PAYLOAD ? kPrimTile : 1];
+    __shared__ std::uint64_t skeys[kPrimTile];
+    __shared__ std::uint32_t svals[kPrimTile];
     const unsigned lane = __lane_id();
     const unsigned wave = threadIdx.x / kWave;
     for (int i = threadIdx.x; i < kPrimWaves * kRadixBins; i += kPrimThreads) (&cnt[0][0])[i] = 0;
@@ -235,7 +234,7 @@ __global__ void __launch_bounds__(kPrimThreads) radix_scatter_kernel(const std::
     std::uint32_t v[kPrimRounds];
     std::uint32_t rank[kPrimRounds];
     prim_load(keysIn, base + lane, n, k);
-    if constexpr (PAYLOAD) prim_load(valsIn, base + lane, n, v);
+    prim_load(valsIn, base + lane, n, v);
 #pragma unroll
     for (int r = 0; r < kPrimRounds; ++r) {
         const std::uint64_t i = base + r * kWave + lane;
@@ -249,26 +248,6 @@ __global__ void __launch_bounds__(kPrimThreads) radix_scatter_kernel(const std::
         if (valid && (peers & lt) == 0) cnt[wave][d] = before + static_cast<std::uint32_t>(__popcll(peers));
     }
     __syncthreads();
-    if constexpr (!PAYLOAD) {
-        const unsigned d = threadIdx.x;
-        std::uint32_t run = gbase[d];
-#pragma unroll
-        for (int w = 0; w < kPrimWaves; ++w) {
-            const std::uint32_t c = cnt[w][d];
-            cnt[w][d] = run;  // becomes the absolute base of (wave w, digit d)
-            run += c;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < kPrimRounds; ++r) {
-            const std::uint64_t i = base + r * kWave + lane;
-            if (i < n) {
-                const unsigned dd = static_cast<unsigned>(k[r] >> shift) & (kRadixBins - 1);
-                keysOut[cnt[wave][dd] + rank[r]] = k[r];
-            }
-        }
-        return;
-    }
     {
         // thread d: the digit's per-wave offsets within its run, and the
         // run's start (an exclusive scan of the digits' tile counts)
@@ -300,7 +279,7 @@ __global__ void __launch_bounds__(kPrimThreads) radix_scatter_kernel(const std::
             const unsigned d = static_cast<unsigned>(k[r] >> shift) & (kRadixBins - 1);
             const std::uint32_t p = tstart[d] + cnt[wave][d] + rank[r];
             skeys[p] = k[r];
-            if constexpr (PAYLOAD) svals[p] = v[r];
+            svals[p] = v[r];
         }
     }
     __syncthreads();
@@ -310,7 +289,7 @@ __global__ void __launch_bounds__(kPrimThreads) radix_scatter_kernel(const std::
         const unsigned d = static_cast<unsigned>(key >> shift) & (kRadixBins - 1);
         const std::uint32_t dst = gbase[d] + (p - tstart[d]);
         keysOut[dst] = key;
-        if constexpr (PAYLOAD) valsOut[dst] = svals[p];
+        valsOut[dst] = svals[p];
     }
 }
 
@@ -324,14 +303,14 @@ inline std::uint64_t radix_temp_elems(std::uint64_t n) {
     return 2 * h + scan_temp_elems(h);
 }
 
-// Sorts the low `bits` bits of n keys (stable LSD, 8 bits per pass), with an
-// optional u32 payload (valsA/valsB may be null).  Data start in the A
-// buffers; *result / *resultVals point at the buffers holding the output.
+// Sorts the low `bits` bits of n keys with a u32 payload (stable LSD, 8 bits
+// per pass).  Data start in the A buffers; *result / *resultVals point at the
+// buffers holding the output.
 inline hipError_t radix_sort_pairs(std::uint64_t* bufA, std::uint64_t* bufB, std::uint32_t* valsA,
                                    std::uint32_t* valsB, std::uint64_t n, unsigned bits, std::uint32_t* temp,
                                    std::uint64_t** result, std::uint32_t** resultVals, hipStream_t stream) {
     *result = bufA;
-    if (resultVals) *resultVals = valsA;
+    *resultVals = valsA;
     if (n <= 1 || bits == 0) return hipSuccess;
     const unsigned tiles = radix_tiles(n);
     const std::uint64_t h = static_cast<std::uint64_t>(kRadixBins) * tiles;
@@ -349,26 +328,185 @@ inline hipError_t radix_sort_pairs(std::uint64_t* bufA, std::uint64_t* bufB, std
         if (e != hipSuccess) return e;
         e = exclusive_scan(hist, histScan, h, nullptr, scanTemp, stream);
         if (e != hipSuccess) return e;
-        if (vsrc) {
-            hipLaunchKernelGGL(radix_scatter_kernel<true>, dim3(tiles), dim3(kPrimThreads), 0, stream, src, dst,
-                               vsrc, vdst, n, shift, histScan, tiles);
-        } else {
-            hipLaunchKernelGGL(radix_scatter_kernel<false>, dim3(tiles), dim3(kPrimThreads), 0, stream, src, dst,
-                               nullptr, nullptr, n, shift, histScan, tiles);
-        }
+        hipLaunchKernelGGL(radix_scatter_kernel, dim3(tiles), dim3(kPrimThreads), 0, stream, src, dst, vsrc, vdst, n,
+                           shift, histScan, tiles);
         e = hipGetLastError();
         if (e != hipSuccess) return e;
         std::swap(src, dst);
         std::swap(vsrc, vdst);
     }
     *result = src;
-    if (resultVals) *resultVals = vsrc;
+    *resultVals = vsrc;
     return hipSuccess;
 }
 
-inline hipError_t radix_sort(std::uint64_t* bufA, std::uint64_t* bufB, std::uint64_t n, unsigned bits,
-                             std::uint32_t* temp, std::uint64_t** result, hipStream_t stream) {
-    return radix_sort_pairs(bufA, bufB, nullptr, nullptr, n, bits, temp, result, nullptr, stream);
+// ------------------------------------------------------------------ partition
+
+// Stable passes over one field of u64 elements, keys alone, the first pass
+// reading them from a loader: three launches a pass (counts, one scan per
+// digit, scatter) where radix_sort's scan over all digits takes three of its
+// own.  A loader has load(first, k, bad): the 16 rounds' elements first + 64 r
+// (past the end: any), and report(bad), called by every lane of the counts.
+
+struct KeyLoad {
+    const std::uint64_t* p;
+    std::uint64_t n;
+    __device__ __forceinline__ void load(std::uint64_t first, std::uint64_t (&k)[kPrimRounds], bool&) const {
+        prim_load(p, first, n, k);
+    }
+    __device__ __forceinline__ void report(bool) const {}
+};
+
+template <typename Load>
+__global__ void __launch_bounds__(kPrimThreads) part_hist_kernel(Load src, std::uint64_t n, unsigned shift, unsigned bits,
+                                                                std::uint32_t* __restrict__ hist, unsigned tiles) {
+    __shared__ std::uint32_t h[kPrimWaves][kRadixBins];
+    const unsigned lane = __lane_id(), wave = threadIdx.x / kWave;
+    for (int i = threadIdx.x; i < kPrimWaves * kRadixBins; i += kPrimThreads) (&h[0][0])[i] = 0;
+    __syncthreads();
+    const std::uint64_t base = static_cast<std::uint64_t>(blockIdx.x) * kPrimTile + wave * kWaveSpan;
+    std::uint64_t k[kPrimRounds];
+    bool bad = false;
+    src.load(base + lane, k, bad);
+    const unsigned mask = (1u << bits) - 1u;
+#pragma unroll
+    for (int r = 0; r < kPrimRounds; ++r)
+        if (base + r * kWave + lane < n) atomicAdd(&h[wave][static_cast<unsigned>(k[r] >> shift) & mask], 1u);
+    src.report(bad);
+    __syncthreads();
+    const unsigned d = threadIdx.x;  // kPrimThreads == kRadixBins
+    if (d <= mask) {
+        std::uint32_t s = 0;
+#pragma unroll
+        for (int w = 0; w < kPrimWaves; ++w) s += h[w][d];
+        hist[static_cast<std::uint64_t>(d) * tiles + blockIdx.x] = s;
+    }
+}
+
+// hist[d][*] := its exclusive scan, total[d] := its sum; one workgroup per
+// row d, 4096 counts a step.
+__global__ void __launch_bounds__(1024) row_scan_kernel(std::uint32_t* __restrict__ hist, unsigned tiles,
+                                                       std::uint32_t* __restrict__ total) {
+    __shared__ std::uint32_t waveSum[16];
+    std::uint32_t* row = hist + static_cast<std::uint64_t>(blockIdx.x) * tiles;
+    const unsigned lane = __lane_id(), wave = threadIdx.x / kWave;
+    std::uint32_t run = 0;
+    for (unsigned base = 0; base < tiles; base += 4096) {
+        const unsigned i0 = base + 4 * threadIdx.x;
+        std::uint32_t v[4], s = 0;
+#pragma unroll
+        for (unsigned q = 0; q < 4; ++q) v[q] = i0 + q < tiles ? row[i0 + q] : 0u;
+#pragma unroll
+        for (unsigned q = 0; q < 4; ++q) s += v[q];
+        const std::uint32_t inc = wave_inclusive_scan(s);
+        if (lane == kWave - 1) waveSum[wave] = inc;
+        __syncthreads();
+        std::uint32_t off = run + inc - s, all = 0;
+#pragma unroll
+        for (unsigned w = 0; w < 16; ++w) {
+            if (w < wave) off += waveSum[w];
+            all += waveSum[w];
+        }
+#pragma unroll
+        for (unsigned q = 0; q < 4; ++q) {
+            if (i0 + q < tiles) row[i0 + q] = off;
+            off += v[q];
+        }
+        run += all;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) total[blockIdx.x] = run;
+}
+
+template <typename Load>
+__global__ void __launch_bounds__(kPrimThreads) part_scatter_kernel(Load src, std::uint64_t* __restrict__ out,
+                                                                   std::uint64_t n, unsigned shift, unsigned bits,
+                                                                   const std::uint32_t* __restrict__ hist, unsigned tiles,
+                                                                   const std::uint32_t* __restrict__ total) {
+    __shared__ std::uint32_t cnt[kPrimWaves][kRadixBins];
+    __shared__ std::uint32_t waveSum[kPrimWaves];
+    const unsigned lane = __lane_id(), wave = threadIdx.x / kWave;
+    const unsigned bins = 1u << bits, mask = bins - 1u;
+    for (int i = threadIdx.x; i < kPrimWaves * kRadixBins; i += kPrimThreads) (&cnt[0][0])[i] = 0;
+    const std::uint64_t base = static_cast<std::uint64_t>(blockIdx.x) * kPrimTile + wave * kWaveSpan;
+    const std::uint64_t lt = lanemask_lt();
+    std::uint64_t k[kPrimRounds];
+    std::uint32_t rank[kPrimRounds];
+    bool bad = false;
+    src.load(base + lane, k, bad);
+    // thread d: digit d's base (the digits before it) and this tile's place in it
+    const unsigned d = threadIdx.x;
+    const std::uint32_t tot = d < bins ? total[d] : 0u;
+    const std::uint32_t inTile = d < bins ? hist[static_cast<std::uint64_t>(d) * tiles + blockIdx.x] : 0u;
+    const std::uint32_t inc = wave_inclusive_scan(tot);
+    if (lane == kWave - 1) waveSum[wave] = inc;
+    __syncthreads();
+    std::uint32_t run = inc - tot + inTile;
+    for (unsigned w = 0; w < wave; ++w) run += waveSum[w];
+#pragma unroll
+    for (int r = 0; r < kPrimRounds; ++r) {
+        const bool valid = base + r * kWave + lane < n;
+        const unsigned dg = static_cast<unsigned>(k[r] >> shift) & mask;
+        const std::uint64_t peers = match_peers<kRadixBits>(dg, valid);
+        const std::uint32_t seen = cnt[wave][dg];
+        rank[r] = seen + static_cast<std::uint32_t>(__popcll(peers & lt));
+        if (valid && (peers & lt) == 0) cnt[wave][dg] = seen + static_cast<std::uint32_t>(__popcll(peers));
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kPrimWaves; ++w) {
+        const std::uint32_t c = cnt[w][d];
+        cnt[w][d] = run;  // the first position of (wave w, digit d)
+        run += c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kPrimRounds; ++r) {
+        if (base + r * kWave + lane < n) {
+            const unsigned dg = static_cast<unsigned>(k[r] >> shift) & mask;
+            out[cnt[wave][dg] + rank[r]] = k[r];
+        }
+    }
+}
+
+// u32 scratch of partition_by's counts (its totals take kRadixBins more).
+inline std::uint64_t partition_hist_elems(std::uint64_t n) {
+    return static_cast<std::uint64_t>(kRadixBins) * std::max<std::uint64_t>(radix_tiles(n), 1);
+}
+
+// The n > 0 elements of `first` in stable order of their bits
+// [shift, shift + bits), in bufA or bufB (*result); at least one pass.  The
+// loader may read bufB, which the first pass does not write.
+template <typename Load>
+inline hipError_t partition_by(const Load& first, std::uint64_t* bufA, std::uint64_t* bufB, std::uint64_t n,
+                               unsigned shift, unsigned bits, std::uint32_t* hist, std::uint32_t* total,
+                               std::uint64_t** result, hipStream_t stream) {
+    const unsigned tiles = radix_tiles(n);
+    const unsigned passes = std::max(1u, (bits + kRadixBits - 1) / kRadixBits);
+    std::uint64_t* cur = nullptr;
+    for (unsigned p = 0; p < passes; ++p) {
+        const unsigned w = std::max(1u, bits / passes + (p < bits % passes ? 1u : 0u));
+        std::uint64_t* dst = p % 2 ? bufB : bufA;
+        if (p == 0)
+            hipLaunchKernelGGL(part_hist_kernel<Load>, dim3(tiles), dim3(kPrimThreads), 0, stream, first, n, shift, w,
+                               hist, tiles);
+        else
+            hipLaunchKernelGGL(part_hist_kernel<KeyLoad>, dim3(tiles), dim3(kPrimThreads), 0, stream, KeyLoad{cur, n}, n,
+                               shift, w, hist, tiles);
+        hipLaunchKernelGGL(row_scan_kernel, dim3(1u << w), dim3(1024), 0, stream, hist, tiles, total);
+        if (p == 0)
+            hipLaunchKernelGGL(part_scatter_kernel<Load>, dim3(tiles), dim3(kPrimThreads), 0, stream, first, dst, n,
+                               shift, w, hist, tiles, total);
+        else
+            hipLaunchKernelGGL(part_scatter_kernel<KeyLoad>, dim3(tiles), dim3(kPrimThreads), 0, stream, KeyLoad{cur, n},
+                               dst, n, shift, w, hist, tiles, total);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        cur = dst;
+        shift += w;
+    }
+    *result = cur;
+    return hipSuccess;
 }
 
 // ------------------------------------------------------------------ fills

@@ -515,7 +515,7 @@ int tcc_swtcf_release_plans(void) {
     std::lock_guard<std::mutex> lock(C.mu);
     for (auto& p : C.plans) p.release();
     C.plans.clear();
-    release_scratch();
+    pool_release();
     return TCC_OK;
 }
 

@@ -148,3 +148,49 @@ def test_duplicates_and_ranges(gpu, oracle, columns):
         swtcf.coo_to_bcsc(_u32(bad), _u32(src), None, 32, columns)
     with pytest.raises(_lib.TccError, match="out of range"):
         swtcf.coo_to_bcsr(_u32(dst), _u32(src), None, 32, int(src.max()), phases=2)
+
+
+def test_builds_from_several_threads_and_streams(gpu, oracle):
+    """Kept memory goes from one build to the next: four threads on streams of
+    their own build and release different matrices at the same time, with a
+    release of everything kept in between."""
+    import threading
+
+    from tcc_amd import _lib, swtcf
+
+    cases, errors = [], []
+    for k in range(4):
+        rng = np.random.default_rng(100 + k)
+        nr, nc = 700 + 311 * k, 900 + 17 * k
+        dst, src = _random(nr, nc, 9000 + 4000 * k, rng)
+        p = rng.permutation(dst.size)
+        rowptr = np.zeros(nr + 1, np.int64)
+        np.cumsum(np.bincount(dst, minlength=nr), out=rowptr[1:])
+        colptr = np.zeros(nc + 1, np.int64)
+        np.cumsum(np.bincount(src, minlength=nc), out=colptr[1:])
+        o = np.lexsort((dst, src))
+        cases.append((nr, nc, _u32(dst[p]), _u32(src[p]), oracle.bcsr_build(nr, nc, rowptr, src, None),
+                      oracle.bcsc_build(nr, nc, colptr, dst[o], None)))
+    torch.cuda.synchronize()
+
+    def work(k):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for i in range(12):
+                    nr, nc, d, s, want_r, want_c = cases[(k + i) % 4]
+                    A, B = swtcf.coo_to_bcsr(d, s, None, nr, nc), swtcf.coo_to_bcsc(d, s, None, nr, nc)
+                    if i == 5:
+                        _lib.check(_lib.lib().tcc_swtcf_release_plans())
+                    _same(A.to_host(), want_r, False)
+                    _same(B.to_host(), want_c, False)
+                    A.release()
+                    B.release()
+        except Exception as e:  # shown by the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
