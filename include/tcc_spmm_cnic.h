@@ -188,6 +188,20 @@ int tcc_spmm_cnic_forward_mixed(const tcc_bcsr* bcsr, const tcc_bcsc* bcsc,
                                 const tcc_feature_source* src, float* denseC,
                                 uint32_t featureDim, void* stream);
 
+/* tcc_spmm_cnic_forward_mixed with a caller-owned workspace (no reference
+ * counterpart): when the BCSC holds no blocks and the rows are fp32, the rows
+ * that the BCSR uses are first packed to exact TF32 rows in the workspace and
+ * gathered from there (the same products, fewer bytes).  It takes
+ * tcc_tf32_packed_bytes(num_cols, featureDim) + 16 + 4 * ceil(num_cols / 32)
+ * bytes, which ..._workspace_bytes gives where that pays (a table of 128 MiB
+ * whose rows are gathered 16 times each on average; else 0); a smaller or NULL
+ * workspace gathers the rows where they lie.  The workspace must not be shared with a concurrent call. */
+size_t tcc_spmm_cnic_forward_mixed_workspace_bytes(const tcc_bcsr* bcsr, const tcc_bcsc* bcsc,
+                                                   const tcc_feature_source* src, uint32_t featureDim);
+int tcc_spmm_cnic_forward_mixed_ws(const tcc_bcsr* bcsr, const tcc_bcsc* bcsc, const tcc_feature_source* src,
+                                   float* denseC, uint32_t featureDim, void* workspace, size_t workspaceBytes,
+                                   void* stream);
+
 /* The BCSR part of the mixed form alone (for hot/cold measurements). */
 int tcc_bcsr_spmm_mixed(const tcc_bcsr* A, const tcc_feature_source* src, float* Y,
                         uint32_t featureDim, int accumulate, void* stream);

@@ -106,6 +106,11 @@ SIGNATURES = {
     "tcc_spmm_cnic_forward": (ctypes.c_int, [ctypes.POINTER(BCSR), ctypes.POINTER(BCSC), vp, vp, u32, vp]),
     "tcc_spmm_cnic_forward_mixed": (ctypes.c_int, [ctypes.POINTER(BCSR), ctypes.POINTER(BCSC),
                                                    ctypes.POINTER(FeatureSource), vp, u32, vp]),
+    "tcc_spmm_cnic_forward_mixed_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(BCSR), ctypes.POINTER(BCSC),
+                                                                      ctypes.POINTER(FeatureSource), u32]),
+    "tcc_spmm_cnic_forward_mixed_ws": (ctypes.c_int, [ctypes.POINTER(BCSR), ctypes.POINTER(BCSC),
+                                                      ctypes.POINTER(FeatureSource), vp, u32, vp, ctypes.c_size_t,
+                                                      vp]),
     "tcc_coo_to_bcsr": (ctypes.c_int, [vp, vp, vp, u32, u32, u32, ctypes.POINTER(BCSR), ctypes.POINTER(vp), vp]),
     "tcc_coo_to_bcsr_phased": (ctypes.c_int, [vp, vp, vp, u32, u32, u32, u32, ctypes.POINTER(BCSR),
                                               ctypes.POINTER(vp), vp]),

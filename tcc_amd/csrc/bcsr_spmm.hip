@@ -882,17 +882,16 @@ __global__ void calibration_atomic_kernel(float* __restrict__ dst, std::uint32_t
 // one 8-byte store of their high halves and one 2-byte store of the low bits
 // of their two pairs (features past F: the high halves and pair bytes of the
 // valid ones only, as the layout's padding is left as it is).  With
-// colScale, row r is packed as TF32(colScale[r] * X[r]) (the fp32 product,
-// then rounded).  This is thread i's quad: row r, features 4 (i - r quads)
-// and on; with smax, the quad's largest finite magnitude goes into its
-// slice's LDS maximum.
-__device__ __forceinline__ void pack_quad_body(const float* __restrict__ X, std::uint32_t F, std::uint32_t quads,
-                                               unsigned char* __restrict__ out, std::uint64_t stride, bool vec2,
-                                               const float* __restrict__ colScale, std::uint32_t* smax,
-                                               std::uint32_t W, std::uint64_t i, std::uint64_t r) {
-    const std::uint32_t e = 4 * static_cast<std::uint32_t>(i - r * quads);
+// colScale, row r is packed as TF32(colScale[r] * its features) (the fp32
+// product, then rounded).  Features e.. of row r, which starts at `from`;
+// with smax, the quad's largest finite magnitude goes into its slice's LDS
+// maximum.
+__device__ __forceinline__ void pack_quad(const float* __restrict__ from, std::uint32_t F, std::uint32_t e,
+                                          unsigned char* __restrict__ out, std::uint64_t stride, bool vec2,
+                                          const float* __restrict__ colScale, std::uint32_t* smax, std::uint32_t W,
+                                          std::uint64_t r) {
     const std::uint32_t valid = min(4u, F - e);
-    const float* x = X + r * F + e;
+    const float* x = from + e;
     float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (vec2 && valid == 4) {
         const vf2 a = load_global<vf2>(x), b = load_global<vf2>(x + 2);
@@ -939,6 +938,14 @@ __device__ __forceinline__ void pack_quad_body(const float* __restrict__ X, std:
     }
 }
 
+// Thread i's quad of X's rows: row r, features 4 (i - r quads) and on.
+__device__ __forceinline__ void pack_quad_body(const float* __restrict__ X, std::uint32_t F, std::uint32_t quads,
+                                               unsigned char* __restrict__ out, std::uint64_t stride, bool vec2,
+                                               const float* __restrict__ colScale, std::uint32_t* smax,
+                                               std::uint32_t W, std::uint64_t i, std::uint64_t r) {
+    pack_quad(X + r * F, F, 4 * static_cast<std::uint32_t>(i - r * quads), out, stride, vec2, colScale, smax, W, r);
+}
+
 // With sliceMax (non-null, zeroed by the caller), the largest finite |TF32
 // value| bits of each slice of W features (W % 4 == 0) over all rows go to
 // sliceMax[(blockIdx.x % kPackSliceMaxRows) * slices + s] through atomicMax:
@@ -960,6 +967,96 @@ __global__ void tf32_pack_kernel(const float* __restrict__ X, std::uint32_t rows
         for (std::uint32_t s = threadIdx.x; s < slices; s += blockDim.x)
             if (smax[s]) atomicMax(&sliceMax[(blockIdx.x % kPackSliceMaxRows) * slices + s], smax[s]);
     }
+}
+
+// Bit c of `used` for every column c in a block matrix's slots (its padding
+// skipped), gathered in LDS a slice of kMarkColumns columns at a time, each
+// slice by its own workgroups over all slots, and joined by one OR a word
+// that is not yet complete.  2.45M columns in 55M slots: 131 us
+// (432 with one byte a column in memory, checked and stored by every slot:
+// each check fills a 128-byte L1 line).  Past kMarkSlices slices the re-reading costs
+// more than that, and `slices` 0 checks and sets the bits in memory.
+constexpr std::uint32_t kMarkColumns = 32u * 32768u;  // 128 KiB of bits
+constexpr std::uint32_t kMarkSlices = 8;
+__global__ void __launch_bounds__(1024) mark_columns_kernel(const std::uint32_t* __restrict__ idx, std::uint64_t n,
+                                                            std::uint32_t numIn, std::uint32_t slices,
+                                                            std::uint32_t* __restrict__ used) {
+    extern __shared__ std::uint32_t bits[];  // [kMarkColumns / 32] where slices != 0
+    if (slices == 0) {
+        const std::uint64_t stride = static_cast<std::uint64_t>(gridDim.x) * 1024;
+        for (std::uint64_t i = static_cast<std::uint64_t>(blockIdx.x) * 1024 + threadIdx.x; i < n; i += stride) {
+            const std::uint32_t in = idx[i];
+            if (in < numIn && ((used[in / 32] >> (in % 32)) & 1u) == 0) atomicOr(&used[in / 32], 1u << (in % 32));
+        }
+        return;
+    }
+    const std::uint32_t base = blockIdx.x % slices * kMarkColumns;
+    const std::uint32_t span = min(kMarkColumns, numIn - base);
+    const std::uint32_t words = (span + 31) / 32;
+    for (unsigned i = threadIdx.x; i < words; i += 1024) bits[i] = 0;
+    __syncthreads();
+    // the slots are whole blocks of 8: two 16-byte loads each, where aligned;
+    // their words are read together, and only bits not yet set are added
+    auto mark = [&](const std::uint32_t (&in)[8]) {
+        std::uint32_t x[8], w[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            x[k] = in[k] - base;  // wraps below the slice
+            w[k] = x[k] < span ? bits[x[k] / 32] : ~0u;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (((w[k] >> (x[k] % 32)) & 1u) == 0) atomicOr(&bits[x[k] / 32], 1u << (x[k] % 32));
+    };
+    const std::uint64_t stride = static_cast<std::uint64_t>(gridDim.x / slices) * 1024;
+    const std::uint64_t first = static_cast<std::uint64_t>(blockIdx.x / slices) * 1024 + threadIdx.x;
+    const bool aligned = (reinterpret_cast<std::uintptr_t>(idx) & 15u) == 0;
+    for (std::uint64_t i = first; i < n / 8; i += stride) {
+        std::uint32_t in[8];
+        if (aligned) {
+            const vu4 u = load_global<vu4>(idx + 8 * i), v = load_global<vu4>(idx + 8 * i + 4);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                in[k] = u[k];
+                in[4 + k] = v[k];
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) in[k] = idx[8 * i + k];
+        }
+        mark(in);
+    }
+    __syncthreads();
+    // from a different word each: one address takes an atomic every 12 ns
+    const std::uint32_t turn = blockIdx.x / slices * 1024u % words;
+    for (unsigned i = threadIdx.x; i < words; i += 1024) {
+        const unsigned j = i + turn < words ? i + turn : i + turn - words;
+        const std::uint32_t w = bits[j];
+        if (w & ~used[base / 32 + j]) atomicOr(&used[base / 32 + j], w);
+    }
+}
+
+// tf32_pack_kernel over the feature source's fp32 rows: row c of `out` is the
+// packed row of column c, wherever it lies (zeros for none), for the columns
+// in use.
+__global__ void __launch_bounds__(kThreads) mixed_pack_kernel(MixedArgs m, const std::uint32_t* __restrict__ used,
+                                                             std::uint32_t rows, std::uint32_t F, std::uint32_t quads,
+                                                             unsigned char* __restrict__ out, std::uint64_t stride) {
+    const std::uint64_t i = static_cast<std::uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
+    const std::uint64_t r = i / quads;
+    if (r >= rows || ((used[r / 32] >> (r % 32)) & 1u) == 0) return;
+    const std::uint32_t e = 4 * static_cast<std::uint32_t>(i - r * quads);
+    const float* row = mixed_row(m, F, static_cast<std::uint32_t>(r));
+    if (row == nullptr) {
+        unsigned char* p = out + r * stride;
+        const PackedAt at = packed_at(F, e);
+        const std::uint32_t valid = min(4u, F - e);
+        for (std::uint32_t k = 0; k < valid; ++k) *reinterpret_cast<std::uint16_t*>(p + at.hi + 2 * k) = 0;
+        p[at.lo] = 0;
+        if (valid > 2) p[at.lo + 1] = 0;
+        return;
+    }
+    pack_quad(row, F, e, out, stride, (reinterpret_cast<std::uintptr_t>(row) & 7u) == 0, nullptr, nullptr, 0, r);
 }
 
 struct ScatterArgs {
@@ -1465,6 +1562,26 @@ int mixed_vec(const tcc_feature_source* src, std::uint32_t F, const float* Y) {
     return pick_vec(F, {Y, src->cpu_features});
 }
 
+// Whether the first layer's rows are packed before the gather: rows read
+// often (as kPackMinGathers), of more than 16 features, and a table larger
+// than about half the Infinity Cache, past which the gather runs at memory's
+// rate for the lines it touches.  Edges of a skewed graph, direct against
+// packed, us: 2.45M rows 2010 : 2018 at F = 17, 2540 : 2124 at 64,
+// 4911 : 2784 at 100, 9337 : 5957 at 256; 200k rows 217 : 246 at F = 64
+// (51 MB), 306 : 317 at 128 (102 MB), 590 : 472 at 200 (160 MB); 20k rows
+// 56 : 65 at F = 100 (8 MB).
+constexpr std::uint32_t kMixedPackMinF = 17;
+constexpr std::uint64_t kMixedPackMinTable = 128ull << 20;
+bool mixed_pack_pays(const tcc_bcsr* A, std::uint32_t F) {
+    return 8ull * A->num_TCBlocks >= kPackMinGathers * A->num_cols && F >= kMixedPackMinF &&
+           4ull * F * A->num_cols >= kMixedPackMinTable;
+}
+
+// Packed rows (16-byte aligned in the workspace) and the columns' bits.
+size_t mixed_pack_bytes(const tcc_bcsr* A, std::uint32_t F) {
+    return tcc_tf32_packed_bytes(A->num_cols, F) + 16 + 4 * ((A->num_cols + 31ull) / 32);
+}
+
 // The window offsets are read whenever there are windows (a gather writes
 // every window, empty or not), the block arrays only when there are blocks:
 // a matrix without blocks may come with empty (null) block tensors.
@@ -1786,6 +1903,20 @@ int tcc_spmm_cnic_forward_ws(const tcc_bcsr* bcsr, const tcc_bcsc* bcsc, const f
 
 int tcc_spmm_cnic_forward_mixed(const tcc_bcsr* bcsr, const tcc_bcsc* bcsc, const tcc_feature_source* src,
                                 float* denseC, std::uint32_t featureDim, void* stream) {
+    return tcc_spmm_cnic_forward_mixed_ws(bcsr, bcsc, src, denseC, featureDim, nullptr, 0, stream);
+}
+
+size_t tcc_spmm_cnic_forward_mixed_workspace_bytes(const tcc_bcsr* bcsr, const tcc_bcsc* bcsc,
+                                                   const tcc_feature_source* src, std::uint32_t featureDim) {
+    if (!bcsr || !src || src->row_format != TCC_ROWS_FP32 || bcsr->num_cols == 0 || !feature_dim_ok(featureDim)) return 0;
+    if (bcsc && bcsc->num_TCBlocks != 0) return 0;  // beside the scatter the host link sets the time
+    if (!mixed_pack_pays(bcsr, featureDim)) return 0;
+    return mixed_pack_bytes(bcsr, featureDim);
+}
+
+int tcc_spmm_cnic_forward_mixed_ws(const tcc_bcsr* bcsr, const tcc_bcsc* bcsc, const tcc_feature_source* src,
+                                   float* denseC, std::uint32_t featureDim, void* workspace, size_t workspaceBytes,
+                                   void* stream) {
     clear_last_error();
     TCC_REQUIRE(bcsr_ok(bcsr) && bcsc_ok(bcsc) && src && denseC && feature_dim_ok(featureDim), TCC_ERR_INVALID_ARGUMENT,
                 "invalid spmm_cnic mixed forward arguments");
@@ -1793,6 +1924,35 @@ int tcc_spmm_cnic_forward_mixed(const tcc_bcsr* bcsr, const tcc_bcsc* bcsc, cons
     TCC_REQUIRE(bcsr->phases <= 1, TCC_ERR_UNSUPPORTED, "spmm_cnic forward takes an ordinary (unphased) BCSR");
     const hipStream_t st = as_stream(stream);
     const std::uint64_t F = featureDim;
+    if (bcsc->num_TCBlocks == 0 || bcsc->num_colWindows == 0) {
+        // No scatter: the gather alone stores every row of the windows it
+        // covers (no zero fill, atomics only where units share a window).
+        // 2.45M nodes, 61.9M edges, F = 100, all rows on the device: 5.30 ms
+        // with the zero fill and every window added; 4.91 from fp32 rows,
+        // 2.82 with the rows packed first.
+        TCC_HIP_CHECK(fill<float>(denseC + static_cast<std::uint64_t>(bcsr->num_rowWindows) * 8 * F, 8 * F, 0.0f, st));
+        if (src->row_format != TCC_ROWS_FP32 || bcsr->num_cols == 0 || bcsr->num_TCBlocks == 0 ||
+            workspace == nullptr || workspaceBytes < mixed_pack_bytes(bcsr, featureDim))
+            return tcc_bcsr_spmm_mixed(bcsr, src, denseC, featureDim, 0, stream);
+        const std::uint32_t rows = bcsr->num_cols;
+        auto* packed = reinterpret_cast<unsigned char*>((reinterpret_cast<std::uintptr_t>(workspace) + 15) & ~std::uintptr_t(15));
+        auto* used = reinterpret_cast<std::uint32_t*>(packed + tcc_tf32_packed_bytes(rows, featureDim));
+        TCC_HIP_CHECK(fill<std::uint32_t>(used, (rows + 31ull) / 32, 0u, st));
+        const std::uint64_t n = 8ull * bcsr->num_TCBlocks;
+        std::uint32_t slices = (rows - 1) / kMarkColumns + 1;
+        if (slices > kMarkSlices) slices = 0;
+        // one workgroup a compute unit (its LDS holds one), no more than there are slots for
+        const std::uint64_t markers = std::min<std::uint64_t>((n + 8191) / 8192, device_cus() / std::max(1u, slices));
+        hipLaunchKernelGGL(mark_columns_kernel, dim3(static_cast<unsigned>(std::max(1u, slices) * std::max<std::uint64_t>(1, markers) * (slices ? 1 : 2))),
+                           dim3(1024), slices ? kMarkColumns / 8 : 0, st, bcsr->sparseA2B, n, rows, slices, used);
+        const std::uint32_t quads = (featureDim + 3) / 4;
+        const std::uint64_t threads = static_cast<std::uint64_t>(rows) * quads;
+        TCC_REQUIRE(threads <= 0xFFFFFFFFull * kThreads, TCC_ERR_UNSUPPORTED, "TF32 pack too large");
+        hipLaunchKernelGGL(mixed_pack_kernel, dim3(grid_for(threads, kThreads)), dim3(kThreads), 0, st,
+                           mixed_args(src, featureDim), used, rows, featureDim, quads, packed, packed_stride(featureDim));
+        TCC_LAUNCH_CHECK();
+        return bcsr_spmm_packed_scaled(bcsr, packed, denseC, featureDim, 0, nullptr, st);
+    }
     // denseC = 0 over its (num_rowWindows+1)*8 rows, then both parts add in.
     TCC_HIP_CHECK(fill<float>(denseC, (static_cast<std::uint64_t>(bcsr->num_rowWindows) + 1) * 8 * F, 0.0f, st));
     const int V = mixed_vec(src, featureDim, denseC);

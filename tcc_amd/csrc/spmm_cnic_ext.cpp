@@ -363,6 +363,21 @@ void forward(const tcc_bcsr& A, const tcc_bcsc& B, const torch::Tensor& x, float
                                    st));
 }
 
+// denseC of the first layer, its rows packed in a buffer of the current
+// stream where that pays and memory has room for it.
+void forward_mixed(const tcc_bcsr& A, const tcc_bcsc& B, const tcc_feature_source& s, float* C, std::int32_t F,
+                   int device) {
+    std::size_t need = tcc_spmm_cnic_forward_mixed_workspace_bytes(&A, &B, &s, static_cast<std::uint32_t>(F));
+    torch::Tensor ws;
+    try {
+        if (need) ws = device_bytes(need, device);
+    } catch (const c10::OutOfMemoryError&) {
+        need = 0;
+    }
+    check(tcc_spmm_cnic_forward_mixed_ws(&A, &B, &s, C, static_cast<std::uint32_t>(F), need ? ws.data_ptr() : nullptr,
+                                         need, stream_of(device)));
+}
+
 // ---------------------------------------------------------------- compiled form
 
 torch::Tensor fwd_mixed_bound(std::uint32_t r_rows, std::uint32_t r_cols, std::uint32_t r_nnz, std::uint32_t r_blk,
@@ -381,7 +396,7 @@ torch::Tensor fwd_mixed_bound(std::uint32_t r_rows, std::uint32_t r_cols, std::u
         forward(A, B, x, C, F, device_id);
     } else {
         const tcc_feature_source s = feature_source(id_map, cpu_ptr, csm, gpu_ptr, cap);
-        check(tcc_spmm_cnic_forward_mixed(&A, &B, &s, C, F, stream_of(device_id)));
+        forward_mixed(A, B, s, C, F, device_id);
     }
     return view_of(C, r_rows, F, current_device());
 }
@@ -437,8 +452,7 @@ torch::Tensor fwd_mixed_py(std::uint32_t r_rows, std::uint32_t r_cols, std::uint
     tcc_bcsc B = make_bcsc(c_rows, c_cols, c_nnz, c_blk, c_win, c_cwo, c_tco, c_a2c, c_bits, &c_data);
     const tcc_feature_source s = feature_source(id_map, cpu_ptr, csm, gpu_ptr, cap);
     torch::Tensor out = alloc_output(r_win, F);
-    void* st = stream_of(current_device());
-    check(tcc_spmm_cnic_forward_mixed(&A, &B, &s, out.data_ptr<float>(), F, st));
+    forward_mixed(A, B, s, out.data_ptr<float>(), F, current_device());
     return out.narrow(0, 0, static_cast<std::int64_t>(r_rows) * F);
 }
 

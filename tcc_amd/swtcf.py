@@ -618,8 +618,19 @@ def feature_source(id_map: torch.Tensor, cache_search_map: torch.Tensor, gpu_cac
 
 def spmm_cnic_forward_mixed(bcsr: BlockMatrix, bcsc: BlockMatrix, src: FeatureSourceHandle, denseC: torch.Tensor,
                             F: int, stream=None) -> torch.Tensor:
-    check(_lib.lib().tcc_spmm_cnic_forward_mixed(ctypes.byref(bcsr.view), ctypes.byref(bcsc.view),
-                                                 ctypes.byref(src.struct), denseC.data_ptr(), F, _stream(stream)))
+    """denseC = the first layer's product (tcc_spmm_cnic_forward_mixed_ws),
+    with a workspace of the launch's stream where packing the rows pays and
+    memory has room for it."""
+    args = (ctypes.byref(bcsr.view), ctypes.byref(bcsc.view), ctypes.byref(src.struct))
+    need = int(_lib.lib().tcc_spmm_cnic_forward_mixed_workspace_bytes(*args, F))
+    ws = None
+    if need:
+        try:
+            with torch.cuda.stream(stream):  # None: the current stream
+                ws = torch.empty(need, dtype=torch.uint8, device=denseC.device)
+        except torch.cuda.OutOfMemoryError:
+            need = 0
+    check(_lib.lib().tcc_spmm_cnic_forward_mixed_ws(*args, denseC.data_ptr(), F, _ptr(ws), need, _stream(stream)))
     return denseC
 
 

@@ -1,0 +1,123 @@
+"""The first layer without a scatter: the gather alone, from the rows where
+they lie and from rows packed into a workspace, over widths around the packed
+layout's edges, with rows in several device caches, in host memory, missing
+and refused, against the oracle."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _table(nc, F, rng, refused):
+    """Rows in two device caches, in host memory and missing; (source, X as it
+    is read, what to keep)."""
+    from tcc_amd import swtcf
+    from tcc_amd.hostmem import PinnedArray
+
+    X = rng.standard_normal((nc, F)).astype(np.float32)
+    kind = rng.integers(0, 4, nc)  # 0, 1: device caches; 2: host; 3: none
+    cap = nc
+    csm = np.full(nc, -1, np.int32)
+    caches = []
+    for d in range(2):
+        ids = np.flatnonzero(kind == d)
+        csm[ids] = d * cap + np.arange(ids.size)
+        caches.append(torch.from_numpy(np.ascontiguousarray(X[ids])).cuda())
+    host = PinnedArray((nc, F))
+    order = rng.permutation(nc)
+    host.array[order] = X  # row j lies at order[j]
+    ids = np.where(kind == 3, -1, order).astype(np.int32)
+    seen = X.copy()
+    seen[kind == 3] = 0.0
+    csm[7] = 2 * cap + 5
+    if refused:  # one cache entry past the table
+        j = int(np.flatnonzero((kind == 0) & (np.arange(nc) != 7))[0])
+        csm[j] = 2 * cap + 1
+        seen[j] = 0.0
+    ptrs = torch.tensor([c.data_ptr() for c in caches], dtype=torch.int64, device="cuda")
+    err = torch.zeros(1, dtype=torch.int32, device="cuda")
+    src = swtcf.feature_source(torch.from_numpy(ids).cuda(), torch.from_numpy(csm).cuda(), ptrs, cap, host.device_ptr,
+                               nc * F, device_error=err)
+    return src, seen, err, (caches, host)
+
+
+@pytest.mark.parametrize("refused", [False, True])
+@pytest.mark.parametrize("F", [17, 63, 64, 100, 129, 256, 257, 300, 602])
+def test_mixed_without_scatter(gpu, oracle, F, refused):
+    from tcc_amd import _lib, swtcf
+    from tcc_amd.gcn import _EMPTY_BCSC
+
+    nr, nc, nnz = 203, 150, 9000
+    rng = np.random.default_rng(F)
+    key = np.sort(rng.choice(nr * nc, size=nnz, replace=False))
+    key = key[(key // nc < 40) | (key // nc >= 70)]  # rows without an entry, and windows
+    key = key[key % nc != 7]  # a column that no row uses: its entry is not looked at
+    dst, col = (key // nc).astype(np.uint32), (key % nc).astype(np.uint32)
+    src, seen, err, keep = _table(nc, F, rng, refused)
+    A = swtcf.coo_to_bcsr(torch.from_numpy(dst.view(np.int32)).cuda(), torch.from_numpy(col.view(np.int32)).cuda(), None,
+                          nr, nc)
+    rowptr = np.zeros(nr + 1, np.int64)
+    np.cumsum(np.bincount(dst, minlength=nr), out=rowptr[1:])
+    want = oracle.csr_spmm(rowptr, col, None, seen, use_tf32=True)
+    L = _lib.lib()
+    args = (ctypes.byref(A.view), ctypes.byref(_EMPTY_BCSC.view), ctypes.byref(src.struct))
+    # what packing takes; the query names it only for tables where packing pays
+    need = L.tcc_tf32_packed_bytes(nc, F) + 16 + 4 * ((nc + 31) // 32)
+    assert L.tcc_spmm_cnic_forward_mixed_workspace_bytes(*args, F) == 0
+    rows = (A.view.num_rowWindows + 1) * 8
+    for ws_bytes in (0, need - 1, need):
+        ws = torch.full((need + 64,), 255, dtype=torch.uint8, device="cuda")
+        denseC = torch.full((rows, F), float("nan"), device="cuda")
+        err.zero_()
+        _lib.check(L.tcc_spmm_cnic_forward_mixed_ws(*args, denseC.data_ptr(), F, ws.data_ptr() if ws_bytes else None,
+                                                    ws_bytes, torch.cuda.current_stream().cuda_stream))
+        got = denseC.cpu().numpy()
+        # fp32 sums of at most 150 TF32 products a row
+        assert np.linalg.norm(got[:nr] - want) <= 150 * 2.0**-24 * np.linalg.norm(want), ws_bytes
+        assert not got[nr:].any()
+        assert int(err.item()) == (7 if refused else 0)
+        assert int((ws[need:] != 255).sum()) == 0
+    del keep
+
+
+def test_mixed_workspace_only_where_it_applies(gpu):
+    """A workspace for a table of 128 MiB whose rows are gathered 16 times
+    each, and none beside a scatter, for packed tables, smaller ones or rows
+    gathered too seldom; a launch on another stream packs on that stream."""
+    from tcc_amd import gcn, graphs, swtcf, _lib
+
+    n, F = 70_000, 480  # 134.4 MB
+    rows, cols = graphs.rmat_graph(n, 2_000_000, 3, device="cuda")
+    X = torch.randn((n, F), generator=torch.Generator().manual_seed(3))
+    L = _lib.lib()
+
+    def need(table, g, F=F):
+        b = g.bcsc if g.bcsc is not None else gcn._EMPTY_BCSC
+        return L.tcc_spmm_cnic_forward_mixed_workspace_bytes(ctypes.byref(g.bcsr.view), ctypes.byref(b.view),
+                                                             ctypes.byref(table.source.struct), F)
+
+    hot = gcn.FeatureTable(X, cols, hot_fraction=1.0)
+    g = gcn.LayerGraph(rows, cols, n, n, hot_src=hot.hot)
+    assert need(hot, g) == L.tcc_tf32_packed_bytes(n, F) + 16 + 4 * ((n + 31) // 32)
+    assert need(hot, g, F=479) == 0  # 134,120,000 bytes
+    half = gcn.FeatureTable(X, cols, hot_fraction=0.5)
+    assert need(half, gcn.LayerGraph(rows, cols, n, n, hot_src=half.hot)) == 0
+    assert need(gcn.FeatureTable(X, cols, hot_fraction=1.0, packed=True), g) == 0
+    assert need(hot, gcn.LayerGraph(rows[::8], cols[::8], n, n, hot_src=hot.hot)) == 0
+    # every partial sum of whole numbers is exact: any order gives one result
+    hot.cache.random_(-3, 4, generator=torch.Generator(device="cuda").manual_seed(4))
+    out = torch.empty(((g.bcsr.view.num_rowWindows + 1) * 8, F), device="cuda")
+    direct = torch.empty_like(out)
+    _lib.check(L.tcc_spmm_cnic_forward_mixed(ctypes.byref(g.bcsr.view), ctypes.byref(gcn._EMPTY_BCSC.view),
+                                             ctypes.byref(hot.source.struct), direct.data_ptr(), F,
+                                             torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(g.aggregate(F, source=hot.source), direct[:n])
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(3):  # a freed workspace goes to that stream's next call
+        swtcf.spmm_cnic_forward_mixed(g.bcsr, gcn._EMPTY_BCSC, hot.source, out, F, stream=s)
+    s.synchronize()
+    assert torch.equal(out, direct)
