@@ -4,9 +4,10 @@
 //
 // A [K x M] and B [K x N] are row-major with K = graph nodes (millions) and
 // M, N = layer widths (hundreds or less).  K is split over workgroups; each
-// accumulates the product of its rows for one block of C with
-// v_mfma_f32_16x16x4f32 (fp32 products and sums) and writes it to a partial
-// buffer, and a second kernel sums the partials in a fixed order.
+// accumulates the product of its rows for one block of C with MFMA (fp32
+// ones, or for wide outputs bf16 ones of the operands' exact parts) and
+// writes it to a partial buffer, and a second kernel sums the partials in a
+// fixed order.
 //
 // MFMA operand layout (16x16x4, fp32): lane l supplies A(i = l%16, k = l/16)
 // and B(k = l/16, j = l%16), and holds D(4*(l/16) + v, l%16) in accumulator
@@ -27,7 +28,10 @@
 namespace tcc {
 namespace {
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 struct TnArgs {
     const float* A;
@@ -37,7 +41,9 @@ struct TnArgs {
     std::uint32_t K, M, N;
     std::uint32_t rowsPerSplit;
     std::uint32_t blocksM;  // blocks of C along M
-    // Relu-gradient form only (see tn_partial_kernel): G [K x C] with row
+    // Wide outputs only (tn_split_kernel)
+    std::uint32_t blocksN, splits;
+    // Relu-gradient form only (see tn_split_kernel): G [K x C] with row
     // stride ldg, W2 [N x C], and the H^T G partials [splits][N][C].
     const float* G;
     const float* W2;
@@ -49,22 +55,14 @@ __device__ __forceinline__ std::uint32_t tn_uniform(std::uint32_t v) {
     return static_cast<std::uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
 }
 
+// Narrow outputs (M or N of 16 and less), bound by reading the rows.
 // Workgroup = WM x WN waves; a wave owns TM x TN tiles of 16x16, so a
 // workgroup covers a (16*TM*WM) x (16*TN*WN) block of C.  Each iteration
 // takes U steps of 4 rows; the next iteration's operands are loaded while
 // the current one is multiplied.
-//
-// CT > 0 is the GCN relu-gradient form: B holds H (the relu output of the
-// layer, [K x N]) and the B operand is formed in registers as
-// (G W2^T) (.) [H > 0] from G [K x C] and W2 [N x C] (C <= CT), while H^T G
-// is summed beside it into partial2 -- the layer-1 weight gradient and the
-// layer-2 weight gradient of a two-layer GCN in one pass over its rows.
-template <int TM, int TN, int WM, int WN, int U, int CT, bool VB = false, bool VA = false>
+template <int TM, int TN, int WM, int WN, int U>
 __global__ void __launch_bounds__(kWave * WM * WN) tn_partial_kernel(TnArgs a) {
-    static_assert(!VB || TN % 4 == 0, "a float4 of B feeds four N tiles");
-    constexpr int TA = VA ? TM / 4 : 0;  // groups of four M tiles fed by one float4 of A
     constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
-    constexpr int GC = CT > 0 ? CT : 1;  // G columns held per row
     constexpr std::uint32_t kStep = 4 * U;
     const unsigned lane = __lane_id();
     const unsigned wave = tn_uniform(threadIdx.x / kWave);
@@ -74,44 +72,13 @@ __global__ void __launch_bounds__(kWave * WM * WN) tn_partial_kernel(TnArgs a) {
     const std::uint32_t k0 = blockIdx.x * a.rowsPerSplit;
     const std::uint32_t k1 = min(a.K, k0 + a.rowsPerSplit);
     const unsigned li = lane & 15u, lk = lane >> 4;
-    // Column of N tile u on this lane: 16u + l%16; with VB, tile u = 4g + t
-    // takes column 64g + 4(l%16) + t, so that one float4 load from a row of B
-    // feeds four tiles (a quarter of the load instructions, each costing the
-    // same address-processing time whatever its width).
-    const auto ncol = [&](int u) -> std::uint32_t {
-        return VB ? n0 + 64 * (u / 4) + 4 * li + (u % 4) : n0 + 16 * u + li;
-    };
-    // Row r of M tile t: 16t + r, or with VA, for the first 4*TA tiles
-    // (t = 4h + e), 64h + 4r + e (one float4 of an A row feeds four tiles).
-    const auto mrow = [&](int t, unsigned r) -> std::uint32_t {
-        return t < 4 * TA ? m0 + 64 * (t / 4) + 4 * r + (t % 4) : m0 + 16 * t + r;
-    };
 
-    // Per-lane element offsets inside a 4-row step (row lk, clamped column;
-    // with VB the float4's start, clamped to the row's last 4 columns: a
-    // clamped float4 only feeds columns past N, which are never stored).
+    // Per-lane element offsets inside a 4-row step (row lk, clamped column).
     std::uint32_t offA[TM], offB[TN];
 #pragma unroll
-    for (int t = 0; t < TM; ++t)
-        offA[t] = t < 4 * TA ? lk * a.lda + min(m0 + 64 * (t / 4) + 4 * li, a.M - 4) : lk * a.lda + min(mrow(t, li), a.M - 1);
+    for (int t = 0; t < TM; ++t) offA[t] = lk * a.lda + min(m0 + 16 * t + li, a.M - 1);
 #pragma unroll
-    for (int t = 0; t < TN; ++t)
-        offB[t] = VB ? lk * a.ldb + min(n0 + 64 * (t / 4) + 4 * li, a.N - 4) : lk * a.ldb + min(ncol(t), a.N - 1);
-    // Relu-gradient form: this lane's W2 rows, G column offsets (clamped).
-    float w2[TN][GC];
-    float dw2[TN][GC];
-    std::uint32_t offG[GC];
-#pragma unroll
-    for (int j = 0; j < GC; ++j) offG[j] = CT > 0 ? lk * a.ldg + min<std::uint32_t>(j, a.C - 1) : 0u;
-#pragma unroll
-    for (int t = 0; t < TN; ++t)
-#pragma unroll
-        for (int j = 0; j < GC; ++j) {
-            dw2[t][j] = 0.0f;
-            w2[t][j] = 0.0f;
-            if (CT > 0 && static_cast<std::uint32_t>(j) < a.C)
-                w2[t][j] = a.W2[static_cast<std::uint64_t>(min(ncol(t), a.N - 1)) * a.C + j];
-        }
+    for (int t = 0; t < TN; ++t) offB[t] = lk * a.ldb + min(n0 + 16 * t + li, a.N - 1);
 
     f32x4 acc[TM][TN];
 #pragma unroll
@@ -119,67 +86,25 @@ __global__ void __launch_bounds__(kWave * WM * WN) tn_partial_kernel(TnArgs a) {
 #pragma unroll
         for (int u = 0; u < TN; ++u) acc[t][u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    auto load_full = [&](std::uint32_t k, float (&xa)[U][TM], float (&xb)[U][TN], float (&xg)[U][GC]) {
+    auto load_full = [&](std::uint32_t k, float (&xa)[U][TM], float (&xb)[U][TN]) {
 #pragma unroll
         for (int s = 0; s < U; ++s) {
             const float* ra = a.A + static_cast<std::uint64_t>(k + 4 * s) * a.lda;
             const float* rb = a.B + static_cast<std::uint64_t>(k + 4 * s) * a.ldb;
 #pragma unroll
-            for (int h = 0; h < TA; ++h) {
-                const float4 v = *reinterpret_cast<const float4*>(ra + offA[4 * h]);
-                xa[s][4 * h] = v.x;
-                xa[s][4 * h + 1] = v.y;
-                xa[s][4 * h + 2] = v.z;
-                xa[s][4 * h + 3] = v.w;
-            }
+            for (int t = 0; t < TM; ++t) xa[s][t] = ra[offA[t]];
 #pragma unroll
-            for (int t = 4 * TA; t < TM; ++t) xa[s][t] = ra[offA[t]];
-            if constexpr (VB) {
-#pragma unroll
-                for (int g = 0; g < TN / 4; ++g) {
-                    const float4 v = *reinterpret_cast<const float4*>(rb + offB[4 * g]);
-                    xb[s][4 * g] = v.x;
-                    xb[s][4 * g + 1] = v.y;
-                    xb[s][4 * g + 2] = v.z;
-                    xb[s][4 * g + 3] = v.w;
-                }
-            } else {
-#pragma unroll
-                for (int t = 0; t < TN; ++t) xb[s][t] = rb[offB[t]];
-            }
-            if constexpr (CT > 0) {
-                const float* rg = a.G + static_cast<std::uint64_t>(k + 4 * s) * a.ldg;
-#pragma unroll
-                for (int j = 0; j < GC; ++j) xg[s][j] = rg[offG[j]];
-            }
+            for (int t = 0; t < TN; ++t) xb[s][t] = rb[offB[t]];
         }
     };
-    auto multiply = [&](const float (&xa)[U][TM], const float (&xb)[U][TN], const float (&xg)[U][GC]) {
+    auto multiply = [&](const float (&xa)[U][TM], const float (&xb)[U][TN]) {
 #pragma unroll
-        for (int s = 0; s < U; ++s) {
-            float b[TN];
-#pragma unroll
-            for (int u = 0; u < TN; ++u) {
-                if constexpr (CT > 0) {
-                    // dOut1 = (G W2^T) (.) [H > 0]; dW2 += H^T G (columns past C have w2 = 0
-                    // and are never stored)
-                    float d = 0.0f;
-#pragma unroll
-                    for (int j = 0; j < GC; ++j) {
-                        d = fmaf(xg[s][j], w2[u][j], d);
-                        dw2[u][j] = fmaf(xb[s][u], xg[s][j], dw2[u][j]);
-                    }
-                    b[u] = xb[s][u] > 0.0f ? d : 0.0f;
-                } else {
-                    b[u] = xb[s][u];
-                }
-            }
+        for (int s = 0; s < U; ++s)
 #pragma unroll
             for (int t = 0; t < TM; ++t)
 #pragma unroll
                 for (int u = 0; u < TN; ++u)
-                    acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[s][t], b[u], acc[t][u], 0, 0, 0);
-        }
+                    acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[s][t], xb[s][u], acc[t][u], 0, 0, 0);
     };
 
     // Two operand buffers in turn; loads are unconditional (past the last
@@ -189,25 +114,21 @@ __global__ void __launch_bounds__(kWave * WM * WN) tn_partial_kernel(TnArgs a) {
     // uses, which it does to lower register pressure.)
     const std::uint32_t rows = k1 > k0 ? k1 - k0 : 0u;
     const std::uint32_t nFull = rows / kStep;
-    float ca[U][TM], cb[U][TN], cg[U][GC], na[U][TM], nb[U][TN], ng[U][GC];
-#pragma unroll
-    for (int s = 0; s < U; ++s)
-#pragma unroll
-        for (int j = 0; j < GC; ++j) cg[s][j] = ng[s][j] = 0.0f;
-    if (nFull > 0) load_full(k0, ca, cb, cg);
+    float ca[U][TM], cb[U][TN], na[U][TM], nb[U][TN];
+    if (nFull > 0) load_full(k0, ca, cb);
     std::uint32_t i = 0;
     for (; i + 1 < nFull; i += 2) {
         const std::uint32_t k = k0 + i * kStep;
-        load_full(k + kStep, na, nb, ng);
+        load_full(k + kStep, na, nb);
         __builtin_amdgcn_sched_barrier(0);
-        multiply(ca, cb, cg);
+        multiply(ca, cb);
         __builtin_amdgcn_sched_barrier(0);
-        load_full(i + 2 < nFull ? k + 2 * kStep : k + kStep, ca, cb, cg);
+        load_full(i + 2 < nFull ? k + 2 * kStep : k + kStep, ca, cb);
         __builtin_amdgcn_sched_barrier(0);
-        multiply(na, nb, ng);
+        multiply(na, nb);
         __builtin_amdgcn_sched_barrier(0);
     }
-    if (i < nFull) multiply(ca, cb, cg);
+    if (i < nFull) multiply(ca, cb);
     const std::uint32_t kt = k0 + nFull * kStep;
     if (kt < k1) {  // last rows of the split: zeros past k1
 #pragma unroll
@@ -216,67 +137,340 @@ __global__ void __launch_bounds__(kWave * WM * WN) tn_partial_kernel(TnArgs a) {
             const float* ra = a.A + static_cast<std::uint64_t>(kt + 4 * s) * a.lda;
             const float* rb = a.B + static_cast<std::uint64_t>(kt + 4 * s) * a.ldb;
 #pragma unroll
-            for (int h = 0; h < TA; ++h) {
-                float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (in) v = *reinterpret_cast<const float4*>(ra + offA[4 * h]);
-                ca[s][4 * h] = v.x;
-                ca[s][4 * h + 1] = v.y;
-                ca[s][4 * h + 2] = v.z;
-                ca[s][4 * h + 3] = v.w;
-            }
+            for (int t = 0; t < TM; ++t) ca[s][t] = in ? ra[offA[t]] : 0.0f;
 #pragma unroll
-            for (int t = 4 * TA; t < TM; ++t) ca[s][t] = in ? ra[offA[t]] : 0.0f;
-            if constexpr (VB) {
-#pragma unroll
-                for (int g = 0; g < TN / 4; ++g) {
-                    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                    if (in) v = *reinterpret_cast<const float4*>(rb + offB[4 * g]);
-                    cb[s][4 * g] = v.x;
-                    cb[s][4 * g + 1] = v.y;
-                    cb[s][4 * g + 2] = v.z;
-                    cb[s][4 * g + 3] = v.w;
-                }
-            } else {
-#pragma unroll
-                for (int t = 0; t < TN; ++t) cb[s][t] = in ? rb[offB[t]] : 0.0f;
-            }
-            if constexpr (CT > 0) {
-                const float* rg = a.G + static_cast<std::uint64_t>(kt + 4 * s) * a.ldg;
-#pragma unroll
-                for (int j = 0; j < GC; ++j) cg[s][j] = in ? rg[offG[j]] : 0.0f;
-            }
+            for (int t = 0; t < TN; ++t) cb[s][t] = in ? rb[offB[t]] : 0.0f;
         }
-        multiply(ca, cb, cg);
+        multiply(ca, cb);
     }
 
-    // Tile (t, u): accumulator v of lane l is C(mrow(t, 4*(l/16) + v), ncol(u)).
+    // Tile (t, u): accumulator v of lane l is C(16t + 4*(l/16) + v, 16u + l%16).
     float* out = a.partial + static_cast<std::uint64_t>(blockIdx.x) * a.M * a.N;
 #pragma unroll
     for (int t = 0; t < TM; ++t)
 #pragma unroll
         for (int u = 0; u < TN; ++u) {
-            const std::uint32_t n = ncol(u);
+            const std::uint32_t n = n0 + 16 * u + li;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const std::uint32_t m = mrow(t, 4 * lk + v);
+                const std::uint32_t m = m0 + 16 * t + 4 * lk + v;
                 if (m < a.M && n < a.N) out[static_cast<std::uint64_t>(m) * a.N + n] = acc[t][u][v];
             }
         }
-    if constexpr (CT > 0) {
-        // H^T G of this split: column n = ncol(u) summed over the 4 row
-        // quarters; one block row of C (cbm == 0, first wave row) writes it.
-        float* out2 = a.partial2 + static_cast<std::uint64_t>(blockIdx.x) * a.N * a.C;
+}
+
+// Two floats as three bf16 each: x = hi + mid + lo exactly (8 + 8 + 8 of the
+// 24 significant bits, each part rounded to nearest), two to a register.
+__device__ __forceinline__ void split3(float x0, float x1, std::uint32_t& hi, std::uint32_t& mid, std::uint32_t& lo) {
+    const auto pack = [](float p, float q) {
+        return __builtin_bit_cast(std::uint32_t, __builtin_convertvector(f32x2{p, q}, bf16x2));
+    };
+    hi = pack(x0, x1);
+    const float r0 = x0 - __uint_as_float(hi << 16), r1 = x1 - __uint_as_float(hi & 0xFFFF0000u);
+    mid = pack(r0, r1);
+    lo = pack(r0 - __uint_as_float(mid << 16), r1 - __uint_as_float(mid & 0xFFFF0000u));
+}
+
+// Column maxima of |x| below this (and above zero) are left to the fp32
+// products: their lowest parts would fall under bf16's smallest normal number.
+constexpr float kSplitTiny = 0x1p-96f;
+
+// Wide outputs.  fp32 MFMA runs at 1/16 of the bf16 rate, and the 100 x 256
+// and 602 x 256 products over node rows were bound by it (110 TFLOP/s).  Here
+// each operand is split into three bf16 parts (split3) and a product is the
+// six of the nine part products above 2^-26 of it, summed in fp32, smallest
+// first: every bit of the inputs is used.  The bf16 products' own additions
+// do not round to nearest: summed through all rows, 2.45M of them gave 4.5
+// times the fp32 products' error; so 32 rows are summed by themselves and
+// added to the running sum with an ordinary fma, the sign of A's rows changed
+// from one 32 to the next, which cancels what is left of that bias (1.7e-6 to
+// 3.3e-7 of the result).
+//
+// Workgroup = 2 x 4 waves, a (16*TM) x 256 block of C, one to a compute unit;
+// 32 rows an iteration.  The rows' elements are split once per workgroup:
+// waves w and w + 4 load rows 8w..8w+7 (a float of A and a float2 of B a row
+// and thread), so that a thread holds 8 rows of its columns, the 16 bytes that
+// a lane of the 16x16x32 product takes, and writes the parts to LDS as
+// [part][8-row group][position][8 rows].  The position of B's column 2c + e is
+// 128e + c, so that lanes write and read 16 consecutive bytes each, and a wave
+// takes four of B's tiles that are pairs of columns of the result.  LDS holds
+// two steps.  Waves w and w + 4 share a SIMD: the first stages the next step
+// and then multiplies this one, the other multiplies first, so that the vector
+// and the matrix pipe run side by side (509 us for 233k x 602 x 256 with two
+// workgroups of 4 waves a compute unit and one step each in LDS).
+//
+// Infinities and NaN do not survive a split (and a sum near the largest float
+// may overflow in parts only): a workgroup whose sums are not all finite, or
+// with a column too small to split, forms its block again with fp32 products.
+//
+// CT > 0 is the GCN relu-gradient form: B holds H (the relu output of the
+// layer, [K x N]) and the B operand is formed while it is staged as
+// (G W2^T) (.) [H > 0] from G [K x C] and W2 [N x C] (C <= CT), while H^T G
+// is summed beside it into partial2 -- the layer-1 weight gradient and the
+// layer-2 weight gradient of a two-layer GCN in one pass over its rows.
+//
+// 233k x 602 x 256: 0.43 ms (0.89 with fp32 products, in 3 turns of one
+// workgroup a compute unit), 1.1 PFLOP/s of bf16 part products, the rate of a
+// large bf16 matrix product here; 2.45M x 100 x 256: 1.03 ms (1.22), with the
+// relu gradient of 2 classes 1.12 ms (1.35).  Error against 64 bits 2.4e-7,
+// 3.3e-7 and 3.3e-7 of the result (8.6e-7, 1.3e-6 and 8.7e-7).
+template <int TM, int CT, bool VB>
+__global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
+    constexpr std::uint32_t BM = 16 * TM, BN = 256;
+    constexpr int TW = (TM + 1) / 2;  // tiles along M of the first four waves; TM / 2 of the others
+    constexpr int GC = CT > 0 ? CT : 1;
+    constexpr std::uint32_t kPartA = 4 * BM, kPartB = 4 * BN;  // 16-byte units of one part
+    constexpr std::uint32_t kStage = 3 * (kPartA + kPartB);
+    extern __shared__ uint4 parts[];  // [2 steps]: A's three parts, then B's
+    const unsigned lane = __lane_id();
+    const unsigned wave = tn_uniform(threadIdx.x / kWave);
+    const unsigned wm = wave >> 2, wn = wave & 3u;  // wn: also the 8 rows that it stages
+    const unsigned li = lane & 15u, lk = lane >> 4;
+    // The blocks of one split read the same rows: splits go around in eights,
+    // so that those blocks meet in one XCD's L2.
+    const std::uint32_t blocks = a.blocksM * a.blocksN;
+    const std::uint32_t g8 = blockIdx.x / (8 * blocks), in8 = blockIdx.x - g8 * 8 * blocks;
+    const std::uint32_t n8 = min(8u, a.splits - 8 * g8);
+    const std::uint32_t split = 8 * g8 + in8 % n8, block = in8 / n8;
+    const std::uint32_t cbm = block % a.blocksM, cbn = block / a.blocksM;
+    const std::uint32_t m0 = cbm * BM, n0 = cbn * BN;
+    const std::uint32_t k0 = split * a.rowsPerSplit;
+    const std::uint32_t k1 = min(a.K, k0 + a.rowsPerSplit);
+
+    // This thread's columns (clamped: what they feed past M and N is not stored).
+    const unsigned at = 64 * wm + lane;  // A's column, B's pair of columns
+    const std::uint32_t colA = min(m0 + at, a.M - 1);
+    std::uint32_t colB[2];
 #pragma unroll
-        for (int u = 0; u < TN; ++u)
+    for (int e = 0; e < 2; ++e) colB[e] = VB ? min(n0 + 2 * at, a.N - 2) + e : min(n0 + 2 * at + e, a.N - 1);
+    float w2[2][GC], dw2[2][GC];
 #pragma unroll
-            for (int j = 0; j < GC; ++j) {
-                float v = dw2[u][j];
-                v += __shfl_xor(v, 16);
-                v += __shfl_xor(v, 32);
-                const std::uint32_t n = ncol(u);
-                if (cbm == 0 && wm == 0 && lk == 0 && n < a.N && static_cast<std::uint32_t>(j) < a.C)
-                    out2[static_cast<std::uint64_t>(n) * a.C + j] = v;
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int j = 0; j < GC; ++j) {
+            dw2[e][j] = 0.0f;
+            w2[e][j] = CT > 0 && static_cast<std::uint32_t>(j) < a.C
+                           ? a.W2[static_cast<std::uint64_t>(colB[e]) * a.C + j] : 0.0f;
+        }
+    float maxA = 0.0f, maxB[2] = {0.0f, 0.0f};
+
+    f32x4 acc[TW][4];
+#pragma unroll
+    for (int t = 0; t < TW; ++t)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc[t][u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    // G's rows, of the relu-gradient form: lane CT r + j holds G(row r, j), read
+    // back lane by lane.
+    float xa[8], xb[8][2], xg = 0.0f;
+    const std::uint32_t gr = CT > 0 ? lane / GC % 8 : 0u, gj = CT > 0 ? lane % GC : 0u;
+    auto load = [&](std::uint32_t k) {  // rows k + 8 wn ..+7, the last row again past k1
+#pragma unroll
+        for (std::uint32_t r = 0; r < 8; ++r) {
+            const std::uint64_t row = min(k + 8 * wn + r, k1 - 1);
+            const float* rb = a.B + row * a.ldb;
+            if constexpr (VB) {
+                const float2 v = *reinterpret_cast<const float2*>(rb + colB[0]);
+                xb[r][0] = v.x, xb[r][1] = v.y;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 2; ++e) xb[r][e] = rb[colB[e]];
             }
+            xa[r] = a.A[row * a.lda + colA];
+        }
+        if constexpr (CT > 0) {
+            const std::uint32_t row = k + 8 * wn + gr;
+            xg = a.G[static_cast<std::uint64_t>(min(row, k1 - 1)) * a.ldg + min(gj, a.C - 1)];
+        }
+    };
+    auto put = [&](uint4* to, std::uint32_t part, const float (&x)[8], float& top) {
+        std::uint32_t h[4], m[4], l[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            split3(x[2 * q], x[2 * q + 1], h[q], m[q], l[q]);
+            top = fmaxf(top, fmaxf(fabsf(x[2 * q]), fabsf(x[2 * q + 1])));
+        }
+        to[0] = make_uint4(h[0], h[1], h[2], h[3]);
+        to[part] = make_uint4(m[0], m[1], m[2], m[3]);
+        to[2 * part] = make_uint4(l[0], l[1], l[2], l[3]);
+    };
+    auto stage = [&](uint4* to, std::uint32_t k, float sign) {
+        // Rows past the split's last (its row again) count zero times, by
+        // their factor of A: what 0 makes of an infinity is summed again.
+        float f[8];
+#pragma unroll
+        for (std::uint32_t r = 0; r < 8; ++r) f[r] = k + 8 * wn + r < k1 ? sign : 0.0f;
+        const float gl = k + 8 * wn + gr < k1 && gj < a.C ? xg : 0.0f;
+        if (BM == 128 || at < BM) {
+            float x[8];
+#pragma unroll
+            for (int r = 0; r < 8; ++r) x[r] = f[r] * xa[r];
+            put(to + wn * BM + at, kPartA, x, maxA);
+        }
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            float x[8];
+            float part[GC];  // of dW2, these 8 rows
+#pragma unroll
+            for (int j = 0; j < GC; ++j) part[j] = 0.0f;
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                x[r] = xb[r][e];
+                if constexpr (CT > 0) {
+                    if (k + 8 * wn + r >= k1) x[r] = 0.0f;
+                    // dOut1 = (G W2^T) (.) [H > 0]; dW2 += H^T G
+                    float d = 0.0f;
+#pragma unroll
+                    for (int j = 0; j < GC; ++j) {
+                        const float g = __uint_as_float(static_cast<std::uint32_t>(
+                            __builtin_amdgcn_readlane(static_cast<int>(__float_as_uint(gl)), GC * r + j)));
+                        d = fmaf(g, w2[e][j], d);
+                        part[j] = fmaf(x[r], g, part[j]);
+                    }
+                    x[r] = x[r] > 0.0f ? d : 0.0f;
+                }
+            }
+            if constexpr (CT > 0) {
+#pragma unroll
+                for (int j = 0; j < GC; ++j) dw2[e][j] += part[j];
+            }
+            put(to + 3 * kPartA + wn * BN + 128 * e + at, kPartB, x, maxB[e]);
+        }
+    };
+    // B's tile u of this wave: positions 128 (u / 2) + 32 wn + 16 (u % 2) + l%16.
+    auto multiply = [&](const uint4* from, float sign) {
+        bf16x8 b[4][3];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int s = 0; s < 3; ++s)
+                b[u][s] = __builtin_bit_cast(
+                    bf16x8, from[3 * kPartA + s * kPartB + lk * BN + 128 * (u / 2) + 32 * wn + 16 * (u % 2) + li]);
+#pragma unroll
+        for (int t = 0; t < TW; ++t) {
+            if (TM % 2 != 0 && t == TW - 1 && wm != 0) break;
+            bf16x8 x[3];
+#pragma unroll
+            for (int s = 0; s < 3; ++s)
+                x[s] = __builtin_bit_cast(bf16x8, from[s * kPartA + lk * BM + 16 * (TW * wm + t) + li]);
+            constexpr int kX[6] = {2, 0, 1, 1, 0, 0}, kB[6] = {0, 2, 1, 0, 1, 0};
+            f32x4 sum[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) sum[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int s = 0; s < 6; ++s)
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    sum[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[kX[s]], b[u][kB[s]], sum[u], 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[t][u][v] = fmaf(sign, sum[u][v], acc[t][u][v]);
+        }
+    };
+
+    load(k0);
+    float sign = 1.0f;
+    stage(parts, k0, sign);
+    load(k0 + 32);
+    __syncthreads();
+    std::uint32_t cur = 0;
+    for (std::uint32_t k = k0; k < k1; k += 32, sign = -sign, cur = kStage - cur) {
+        if (wm != 0) multiply(parts + cur, sign);
+        __builtin_amdgcn_sched_barrier(0);
+        // past the last row too (zeros, and its row again): under a branch the
+        // loaded registers would be copied, and waited for, where it ends
+        stage(parts + (kStage - cur), k + 32, -sign);
+        load(k + 64);
+        __builtin_amdgcn_sched_barrier(0);
+        if (wm == 0) multiply(parts + cur, sign);
+        __syncthreads();
+    }
+
+    // Row r of tile t is column m of A, tile u's lane column n(u) of B.
+    const auto mcol = [&](int t, unsigned r) { return m0 + 16 * (TW * wm + t) + r; };
+    const auto ncol = [&](int u) { return n0 + 2 * (32 * wn + 16 * (u % 2) + li) + u / 2; };
+    const int tiles = wm == 0 ? TW : TM / 2;
+
+    bool redo = false;
+    auto tiny = [&](float top) { return top != 0.0f && top < kSplitTiny; };
+    redo |= tiny(maxA) || tiny(maxB[0]) || tiny(maxB[1]);
+#pragma unroll
+    for (int t = 0; t < TW; ++t)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) redo |= !(fabsf(acc[t][u][v]) <= 0x1.fffffep127f);
+    if (__syncthreads_or(redo)) {
+#pragma unroll
+        for (int t = 0; t < TW; ++t)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) acc[t][u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (std::uint32_t k = k0; k < k1; k += 4) {
+            const bool in = k + lk < k1;
+            const std::uint64_t row = min(k + lk, k1 - 1);
+            float y[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const std::uint32_t c = min(ncol(u), a.N - 1);
+                y[u] = in ? a.B[row * a.ldb + c] : 0.0f;
+                if constexpr (CT > 0) {
+                    float d = 0.0f;
+                    for (std::uint32_t j = 0; j < a.C; ++j)
+                        d = fmaf(in ? a.G[row * a.ldg + j] : 0.0f, a.W2[static_cast<std::uint64_t>(c) * a.C + j], d);
+                    y[u] = y[u] > 0.0f ? d : 0.0f;
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < TW; ++t) {
+                const float x = in ? a.A[row * a.lda + min(mcol(t, li), a.M - 1)] : 0.0f;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, y[u], acc[t][u], 0, 0, 0);
+            }
+        }
+    }
+
+    // Tile (t, u): accumulator v of lane l is C(mcol(t, 4*(l/16) + v), ncol(u)).
+    float* out = a.partial + static_cast<std::uint64_t>(split) * a.M * a.N;
+    const bool vec = a.N % 2 == 0 && (reinterpret_cast<std::uintptr_t>(a.partial) & 7u) == 0;
+#pragma unroll
+    for (int t = 0; t < TW; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const std::uint32_t m = mcol(t, 4 * lk + v);
+            if (t >= tiles || m >= a.M) continue;
+            float* o = out + static_cast<std::uint64_t>(m) * a.N;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const std::uint32_t n = ncol(u);
+                if (vec) {
+                    if (n < a.N) *reinterpret_cast<float2*>(o + n) = make_float2(acc[t][u][v], acc[t][u + 2][v]);
+                } else {
+                    if (n < a.N) o[n] = acc[t][u][v];
+                    if (n + 1 < a.N) o[n + 1] = acc[t][u + 2][v];
+                }
+            }
+        }
+    if constexpr (CT > 0) {
+        // H^T G of this split: a column's four groups of rows, added in order;
+        // the first block row of C writes it.
+        if (cbm != 0) return;
+        float* part = reinterpret_cast<float*>(parts);  // [4][256][CT]
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int j = 0; j < GC; ++j) part[(wn * 256 + 2 * at + e) * GC + j] = dw2[e][j];
+        __syncthreads();
+        float* out2 = a.partial2 + static_cast<std::uint64_t>(split) * a.N * a.C;
+        const std::uint32_t c = n0 + threadIdx.x;
+        if (threadIdx.x >= 256 || c >= a.N) return;
+        for (std::uint32_t j = 0; j < a.C; ++j) {
+            float v = 0.0f;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) v += part[(w * 256 + threadIdx.x) * GC + j];
+            out2[static_cast<std::uint64_t>(c) * a.C + j] = v;
+        }
     }
 }
 
@@ -468,16 +662,9 @@ __global__ void __launch_bounds__(256) tn_reduce_kernel(const float* __restrict_
     }
 }
 
-// Wave shapes by output shape (measured on MI355X, K = 2.45M rows):
-//  - anything wide: 4 waves side by side along N, each with TM x 4 tiles
-//    (TM = 4, 7 or 8, the fewest that cover M, so that a 100-wide layer does
-//    not multiply a 128-wide tile column); 4 tiles along N reuse each A
-//    operand 4 times from registers: 100x256 runs at ~110 TFLOP/s, against
-//    ~50 with 8 waves of 7x2 tiles.  These waves hold ~340 registers (one
-//    wave per SIMD); limiting them to 256 for two waves per SIMD measured
-//    1.6-1.9x slower.  Six 4-row steps per buffer (24 rows in flight ahead
-//    of the multiply) measured 1.14 ms against 1.23-1.32 with four; the
-//    relu-gradient form, at 256 VGPRs, keeps four;
+// Shapes by output shape:
+//  - anything wide: tn_split_kernel, TM = 4, 7 or 8 tiles along M, the fewest
+//    that cover M, so that a 100-wide layer does not multiply 128 columns;
 //  - N <= 16 (a class-width gradient): 4 waves along M with 4 x 1 tiles,
 //    eight workgroups per CU for memory parallelism (~5 TB/s for 256x2);
 //    M <= 16 the same along N.
@@ -491,10 +678,9 @@ struct TnPlan {
     std::uint32_t splits, rowsPerSplit;
 };
 
-// Shape chosen from (M, N); block counts from (realM, realN) and the rows per
-// iteration from `step` when given.
+// Shape chosen from (M, N); block counts from (realM, realN) when given.
 TnPlan tn_plan(std::uint32_t K, std::uint32_t M, std::uint32_t N, std::uint32_t realM = 0, std::uint32_t realN = 0,
-               std::uint32_t step = 0, std::uint64_t splitCap = 0) {
+               std::uint64_t splitCap = 0) {
     TnPlan p{};
     if (N <= 16) {
         p.shape = TnShape::NarrowN;  // TM=4, TN=1, WM=4, WN=1, U=8
@@ -503,22 +689,21 @@ TnPlan tn_plan(std::uint32_t K, std::uint32_t M, std::uint32_t N, std::uint32_t 
         p.shape = TnShape::NarrowM;  // TM=1, TN=4, WM=1, WN=4, U=8
         p.step = 32, p.BM = 16, p.BN = 256;
     } else {
-        // TM in {4, 7, 8}, TN=4, WM=1, WN=4, U=6 (U=4 for the relu-gradient form)
         p.shape = M <= 64 ? TnShape::Wide4 : M <= 112 ? TnShape::Wide7 : TnShape::Wide8;
-        p.step = 24, p.BN = 256;
+        p.step = 32, p.BN = 256;
         p.BM = p.shape == TnShape::Wide4 ? 64 : p.shape == TnShape::Wide7 ? 112 : 128;
     }
     if (realM != 0) M = realM;
     if (realN != 0) N = realN;
-    if (step != 0) p.step = step;
     p.blocksM = (M + p.BM - 1) / p.BM;
     p.blocksN = (N + p.BN - 1) / p.BN;
     const std::uint64_t blocks = static_cast<std::uint64_t>(p.blocksM) * p.blocksN;
-    // About two (Wide*) or eight workgroups per compute unit in all.
+    // One (Wide*: what fits, so that none is left for a second turn) or about
+    // eight workgroups per compute unit in all.
     const bool narrow = p.shape == TnShape::NarrowN || p.shape == TnShape::NarrowM;
-    const std::uint64_t target = static_cast<std::uint64_t>(device_cus()) * (narrow ? 8 : 2);
+    const std::uint64_t target = static_cast<std::uint64_t>(device_cus()) * (narrow ? 8 : 1);
     const std::uint64_t maxSplits = std::max<std::uint64_t>(1, (K + p.step - 1) / p.step);
-    std::uint64_t splits = std::min<std::uint64_t>(maxSplits, std::max<std::uint64_t>(1, (target + blocks - 1) / blocks));
+    std::uint64_t splits = std::min<std::uint64_t>(maxSplits, std::max<std::uint64_t>(1, (target + (narrow ? blocks - 1 : 0)) / blocks));
     if (splitCap != 0) splits = std::min(splits, splitCap);
     std::uint64_t rps = (K + splits - 1) / splits;
     rps = std::max<std::uint64_t>(p.step, (rps + p.step - 1) / p.step * p.step);
@@ -534,16 +719,25 @@ TnPlan tn_plan(std::uint32_t K, std::uint32_t M, std::uint32_t N, std::uint32_t 
 // as C, 2.5x torch.mm).
 inline bool tn_swapped(std::uint32_t M, std::uint32_t N) { return M > 16 && N > 16 && N <= 128 && N < M; }
 
-template <int TM, int TN, int WM, int WN, int U, int CT = 0, bool VB = false, bool VA = false>
+template <int TM, int TN, int WM, int WN, int U>
 void tn_launch(const TnArgs& a, const TnPlan& p, hipStream_t st) {
-    hipLaunchKernelGGL((tn_partial_kernel<TM, TN, WM, WN, U, CT, VB, VA>), dim3(p.splits, p.blocksM * p.blocksN),
+    hipLaunchKernelGGL((tn_partial_kernel<TM, TN, WM, WN, U>), dim3(p.splits, p.blocksM * p.blocksN),
                        dim3(kWave * WM * WN), 0, st, a);
 }
 
-// The relu-gradient form always takes the wide shapes (N is the hidden width)
-// with 16 rows per iteration (4 steps of 4; 8-class tiles take 2 x 4).
+// Pairs of B's columns in one load a row where they allow it.
+template <int TM, int CT>
+void tn_split_launch(const TnArgs& a, const TnPlan& p, hipStream_t st) {
+    const bool vb = a.N % 2 == 0 && a.ldb % 2 == 0 && reinterpret_cast<std::uintptr_t>(a.B) % 8 == 0;
+    const dim3 grid(p.splits * p.blocksM * p.blocksN);
+    constexpr std::uint32_t lds = 2 * 3 * 4 * 16 * (16 * TM + 256);
+    if (vb) hipLaunchKernelGGL((tn_split_kernel<TM, CT, true>), grid, dim3(512), lds, st, a);
+    else hipLaunchKernelGGL((tn_split_kernel<TM, CT, false>), grid, dim3(512), lds, st, a);
+}
+
+// The relu-gradient form always takes the wide shapes (N is the hidden width).
 TnPlan relu_grad_plan(std::uint32_t K, std::uint32_t F, std::uint32_t Hd) {
-    return tn_plan(K, std::max<std::uint32_t>(F, 17), std::max<std::uint32_t>(Hd, 17), F, Hd, 16);
+    return tn_plan(K, std::max<std::uint32_t>(F, 17), std::max<std::uint32_t>(Hd, 17), F, Hd);
 }
 
 }  // namespace
@@ -587,7 +781,7 @@ int dense_tn_impl(const float* A, std::uint32_t lda, const float* B, std::uint32
         std::swap(M, N);
     }
     const std::uint64_t splitBytes = static_cast<std::uint64_t>(M) * N * sizeof(float);
-    const TnPlan p = tn_plan(K, M, N, 0, 0, 0, splitCapBytes ? splitCapBytes / splitBytes : 0);
+    const TnPlan p = tn_plan(K, M, N, 0, 0, splitCapBytes ? splitCapBytes / splitBytes : 0);
     TCC_REQUIRE(workspaceBytes >= static_cast<size_t>(p.splits) * M * N * sizeof(float), TCC_ERR_INVALID_ARGUMENT,
                 "dense A^T B workspace too small (tcc_dense_tn_workspace_bytes)");
     TCC_REQUIRE(static_cast<std::uint64_t>(p.blocksM) * p.blocksN <= 65535, TCC_ERR_UNSUPPORTED,
@@ -603,26 +797,14 @@ int dense_tn_impl(const float* A, std::uint32_t lda, const float* B, std::uint32
     a.N = N;
     a.rowsPerSplit = p.rowsPerSplit;
     a.blocksM = p.blocksM;
-    // B rows as float4 feeding four interleaved N tiles (as the relu-gradient
-    // form) when they allow 16-byte loads
-    const bool vb = N % 4 == 0 && ldb % 4 == 0 && reinterpret_cast<std::uintptr_t>(B) % 16 == 0;
-    // and A rows likewise feeding four interleaved M tiles
-    const bool va = vb && M % 4 == 0 && lda % 4 == 0 && reinterpret_cast<std::uintptr_t>(A) % 16 == 0;
+    a.blocksN = p.blocksN;
+    a.splits = p.splits;
     switch (p.shape) {
         case TnShape::NarrowN: tn_launch<4, 1, 4, 1, 8>(a, p, st); break;
         case TnShape::NarrowM: tn_launch<1, 4, 1, 4, 8>(a, p, st); break;
-        case TnShape::Wide4:
-            if (va) tn_launch<4, 4, 1, 4, 6, 0, true, true>(a, p, st);
-            else vb ? tn_launch<4, 4, 1, 4, 6, 0, true>(a, p, st) : tn_launch<4, 4, 1, 4, 6>(a, p, st);
-            break;
-        case TnShape::Wide7:
-            if (va) tn_launch<7, 4, 1, 4, 6, 0, true, true>(a, p, st);
-            else vb ? tn_launch<7, 4, 1, 4, 6, 0, true>(a, p, st) : tn_launch<7, 4, 1, 4, 6>(a, p, st);
-            break;
-        default:
-            if (va) tn_launch<8, 4, 1, 4, 6, 0, true, true>(a, p, st);
-            else vb ? tn_launch<8, 4, 1, 4, 6, 0, true>(a, p, st) : tn_launch<8, 4, 1, 4, 6>(a, p, st);
-            break;
+        case TnShape::Wide4: tn_split_launch<4, 0>(a, p, st); break;
+        case TnShape::Wide7: tn_split_launch<7, 0>(a, p, st); break;
+        default: tn_split_launch<8, 0>(a, p, st); break;
     }
     TCC_LAUNCH_CHECK();
     const std::uint64_t MN = static_cast<std::uint64_t>(M) * N;
@@ -765,28 +947,13 @@ int tcc_gcn_relu_grad(const float* AX, std::uint32_t ldax, const float* H, std::
     a.partial2 = reinterpret_cast<float*>(static_cast<char*>(workspace) + need1);
     a.ldg = ldg;
     a.C = C;
-    // C <= 2: the wide tiles; up to 8 classes: 8 waves of TM x 2 tiles and 2
-    // steps per iteration, to hold the G rows in registers (same blocks).
+    a.blocksN = p.blocksN;
+    a.splits = p.splits;
     const bool two = C <= 2;
-    // H rows as float4 when they allow 16-byte loads (4 | Hd, 4 | ldh, H aligned)
-    const bool vb = Hd % 4 == 0 && ldh % 4 == 0 && reinterpret_cast<std::uintptr_t>(H) % 16 == 0;
-    const bool va = two && vb && F % 4 == 0 && ldax % 4 == 0 && reinterpret_cast<std::uintptr_t>(AX) % 16 == 0;
     switch (p.shape) {
-        case TnShape::Wide4:
-            if (va) tn_launch<4, 4, 1, 4, 4, 2, true, true>(a, p, st);
-            else if (two && vb) tn_launch<4, 4, 1, 4, 4, 2, true>(a, p, st);
-            else two ? tn_launch<4, 4, 1, 4, 4, 2>(a, p, st) : tn_launch<4, 2, 1, 8, 2, 8>(a, p, st);
-            break;
-        case TnShape::Wide7:
-            if (va) tn_launch<7, 4, 1, 4, 4, 2, true, true>(a, p, st);
-            else if (two && vb) tn_launch<7, 4, 1, 4, 4, 2, true>(a, p, st);
-            else two ? tn_launch<7, 4, 1, 4, 4, 2>(a, p, st) : tn_launch<7, 2, 1, 8, 2, 8>(a, p, st);
-            break;
-        default:
-            if (va) tn_launch<8, 4, 1, 4, 4, 2, true, true>(a, p, st);
-            else if (two && vb) tn_launch<8, 4, 1, 4, 4, 2, true>(a, p, st);
-            else two ? tn_launch<8, 4, 1, 4, 4, 2>(a, p, st) : tn_launch<8, 2, 1, 8, 2, 8>(a, p, st);
-            break;
+        case TnShape::Wide4: two ? tn_split_launch<4, 2>(a, p, st) : tn_split_launch<4, 8>(a, p, st); break;
+        case TnShape::Wide7: two ? tn_split_launch<7, 2>(a, p, st) : tn_split_launch<7, 8>(a, p, st); break;
+        default: two ? tn_split_launch<8, 2>(a, p, st) : tn_split_launch<8, 8>(a, p, st); break;
     }
     TCC_LAUNCH_CHECK();
     hipLaunchKernelGGL(tn_reduce_kernel, dim3(grid_for(static_cast<std::uint64_t>(F) * Hd, 16)), dim3(256), 0, st,

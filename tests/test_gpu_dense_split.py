@@ -1,0 +1,118 @@
+"""The wide A^T B products of three bf16 parts (tcc_dense_tn, tcc_gcn_relu_grad):
+the edges of the blocks and of the 32-row steps, values that do not survive a
+split, and whole numbers, against float64.
+
+An element's error is bounded by its sum of |a b|: the parts dropped are below
+2^-25 of each product, a step's six additions of 32 products each lose at most
+one unit in the last place, 2^-23, of it, and the additions of steps and
+splits (at most 35 steps here) half a unit: below 2^-18 in all."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+BOUND = 2.0**-18
+
+
+def _check(C, A, B):
+    A, B = A.double().cpu(), B.double().cpu()
+    want, mag = A.t() @ B, A.abs().t() @ B.abs()
+    assert ((C.double().cpu() - want).abs() <= BOUND * mag).all()
+
+
+@pytest.mark.parametrize("K", [1, 31, 32, 33, 65, 1100])
+@pytest.mark.parametrize("M,N", [(17, 300), (64, 129), (65, 256), (112, 257), (113, 255), (129, 130), (300, 200),
+                                 (200, 40)])
+def test_edges(gpu, K, M, N):
+    from tcc_amd import swtcf
+
+    g = torch.Generator(device="cuda").manual_seed(K + M)
+    A = torch.randn(K, M, generator=g, device="cuda")
+    B = torch.randn(K, N, generator=g, device="cuda")
+    C = swtcf.dense_tn(A, B)
+    _check(C, A, B)
+    assert torch.equal(swtcf.dense_tn(A, B), C)
+    # rows of another stride and alignment
+    Aw = torch.randn(K, M + 3, generator=g, device="cuda")
+    Bw = torch.randn(K, N + 5, generator=g, device="cuda")
+    _check(swtcf.dense_tn(Aw[:, 1: M + 1], Bw[:, 3: N + 3]), Aw[:, 1: M + 1], Bw[:, 3: N + 3])
+    # whole numbers are exact
+    Ai = torch.randint(-60, 61, (K, M), generator=g, device="cuda").float()
+    Bi = torch.randint(-200, 201, (K, N), generator=g, device="cuda").float()
+    assert torch.equal(swtcf.dense_tn(Ai, Bi).double(), Ai.double().t() @ Bi.double())
+
+
+def _special(kind, A, B):
+    K = A.shape[0]
+    if kind == "inf":
+        A[K // 2, 3] = float("inf")
+    elif kind == "inf in the last row":
+        B[K - 1, 5] = float("-inf")
+    elif kind == "nan":
+        B[K // 3, 40] = float("nan")
+    elif kind == "nan of low bits":  # rounds to an infinity if its bits are only cut
+        A.view(torch.int32)[K // 3, 7] = 0x7F800001
+    elif kind == "largest":  # rounds up to an infinity in 8 bits
+        A[::7] = torch.finfo(torch.float32).max * torch.sign(A[::7])
+        B *= 1e-30
+    elif kind == "tiny":
+        A *= 1e-36
+        B *= 1e10
+    elif kind == "tiny columns":
+        A[:, 5] *= 1e-37
+        B[:, 9] *= 1e-38
+
+
+KINDS = ["inf", "inf in the last row", "nan", "nan of low bits", "largest", "tiny", "tiny columns"]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_values_past_a_split(gpu, kind):
+    from tcc_amd import swtcf
+
+    K, M, N = 77, 100, 70
+    g = torch.Generator().manual_seed(5)
+    A, B = torch.randn(K, M, generator=g), torch.randn(K, N, generator=g)
+    _special(kind, A, B)
+    got = swtcf.dense_tn(A.cuda(), B.cuda()).double().cpu()
+    A, B = A.double(), B.double()
+    want = A.t() @ B
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(torch.isinf(got), torch.isinf(want))
+    inf = torch.isinf(want)
+    assert torch.equal(got[inf], want[inf])
+    mag = A.abs().t() @ B.abs()
+    ok = torch.isfinite(want)
+    # subnormal products lose at most half of the smallest number each
+    assert ((got - want)[ok].abs() <= BOUND * mag[ok] + K * 2.0**-126).all()
+
+
+@pytest.mark.parametrize("C", [1, 2, 3, 8])
+@pytest.mark.parametrize("K", [33, 1100])
+def test_relu_gradient_edges(gpu, K, C):
+    """dW1 and dW2 with an infinity in G's and H's last row, and without."""
+    from tcc_amd import swtcf
+
+    F, Hd = 113, 258
+    g = torch.Generator().manual_seed(K + C)
+    AX, G, W2 = (torch.randn(s, generator=g) for s in ((K, F), (K, C), (Hd, C)))
+    H = torch.randn(K, Hd, generator=g).relu_()
+    for special in (False, True):
+        if special:
+            G[K - 1, C - 1] = float("inf")
+            H[K - 1, 2] = float("inf")
+            H[K - 1, 3:] += 0.5
+            H[K - 1, :2] = 0.25
+        dW1, dW2 = swtcf.gcn_relu_grad(AX.cuda(), H.cuda(), G.cuda(), W2.cuda())
+        d = (G.double() @ W2.double().t()).where(H > 0, torch.zeros((), dtype=torch.float64))
+        dmag = (G.double().abs() @ W2.double().abs().t()).where(H > 0, torch.zeros((), dtype=torch.float64))
+        for got, want, mag in ((dW1, AX.double().t() @ d, AX.double().abs().t() @ dmag),
+                               (dW2, H.double().t() @ G.double(), H.double().abs().t() @ G.double().abs())):
+            got = got.double().cpu()
+            fin = torch.isfinite(want)
+            assert torch.equal(torch.isfinite(got), fin)
+            assert torch.equal(torch.isinf(got), torch.isinf(want))
+            # d itself is a sum of C rounded products
+            assert ((got - want)[fin].abs() <= 2 * BOUND * mag[fin]).all()
+        assert special or bool(torch.isfinite(dW1).all())
