@@ -133,6 +133,42 @@ __global__ void __launch_bounds__(kPrimThreads) scan_tiles_kernel(const std::uin
     }
 }
 
+// The scan of a few tiles in one workgroup, a tile a step: up to kScanSteps
+// tiles it takes less than three launches' cost on the host (3.6 us each).
+constexpr std::uint64_t kScanSteps = 4;
+__global__ void __launch_bounds__(1024) scan_steps_kernel(const std::uint32_t* in, std::uint32_t* out, std::uint64_t n,
+                                                          std::uint32_t* total, const std::uint32_t* skip) {
+    __shared__ std::uint32_t waveSum[16];
+    if (skip != nullptr && *skip == 0u) return;
+    const unsigned lane = __lane_id(), wave = threadIdx.x / kWave;
+    std::uint32_t run = 0;
+    for (std::uint64_t base = 0; base < n; base += 4096) {
+        const std::uint64_t i0 = base + 4 * threadIdx.x;
+        std::uint32_t v[4], s = 0;
+#pragma unroll
+        for (unsigned q = 0; q < 4; ++q) v[q] = i0 + q < n ? in[i0 + q] : 0u;
+#pragma unroll
+        for (unsigned q = 0; q < 4; ++q) s += v[q];
+        const std::uint32_t inc = wave_inclusive_scan(s);
+        if (lane == kWave - 1) waveSum[wave] = inc;
+        __syncthreads();
+        std::uint32_t off = run + inc - s;
+#pragma unroll
+        for (unsigned w = 0; w < 16; ++w) {
+            const std::uint32_t x = waveSum[w];
+            if (w < wave) off += x;
+            run += x;
+        }
+#pragma unroll
+        for (unsigned q = 0; q < 4; ++q) {
+            if (i0 + q < n) out[i0 + q] = off;
+            off += v[q];
+        }
+        __syncthreads();
+    }
+    if (total != nullptr && threadIdx.x == 0) *total = run;
+}
+
 // Scratch (u32 elements) needed by exclusive_scan for n items.
 inline std::uint64_t scan_temp_elems(std::uint64_t n) {
     std::uint64_t t = 0;
@@ -152,6 +188,10 @@ inline hipError_t exclusive_scan(const std::uint32_t* in, std::uint32_t* out, st
     if (n <= static_cast<std::uint64_t>(kPrimTile)) {
         hipLaunchKernelGGL(scan_tiles_kernel, dim3(1), dim3(kPrimThreads), 0, stream, in, out, n,
                            nullptr, total, skip);
+        return hipGetLastError();
+    }
+    if (n <= kScanSteps * kPrimTile) {
+        hipLaunchKernelGGL(scan_steps_kernel, dim3(1), dim3(1024), 0, stream, in, out, n, total, skip);
         return hipGetLastError();
     }
     const std::uint64_t tiles = (n + kPrimTile - 1) / kPrimTile;

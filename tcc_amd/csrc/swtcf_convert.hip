@@ -43,6 +43,11 @@ constexpr unsigned kWaves = kThreads / kWave;  // 4
 constexpr unsigned kRounds = 16;
 constexpr unsigned kTile = kThreads * kRounds;  // elements per sort tile and per segment tile
 constexpr unsigned kSpan = kWave * kRounds;     // consecutive elements of one wave
+// Where there are no more tiles than compute units, a tile's workgroup has
+// kWideThreads threads: with a quarter of the rounds a wave, its serial chain
+// is as much shorter, and no other workgroup waits for the room (16 tiles:
+// the counts 12 -> 7 us, the scatter 14.7 -> 10.2).
+constexpr unsigned kWideThreads = 1024;
 constexpr unsigned kMaxLowDigit = 9;            // bits per pass over dst/lo
 constexpr unsigned kMaxTopDigit = 8;            // bits per pass over sw
 constexpr unsigned kMaxBins = 1u << kMaxLowDigit;
@@ -351,16 +356,17 @@ struct ScatterArgs {
     unsigned w0;                  // bits of the first pass's digit
 };
 
-// The 16 rounds' elements of a lane (element first + 64 r), all loads
+// The R rounds' elements of a lane (element first + 64 r), all loads
 // issued before any is used: indices past the end are clamped to the last
 // element (those lanes take no part in what follows).
+template <unsigned R>
 __device__ __forceinline__ void load_elems(const ScatterArgs& a, bool coo, std::uint64_t first,
-                                           std::uint64_t (&k)[kRounds], const std::uint32_t* d0s) {
+                                           std::uint64_t (&k)[R], const std::uint32_t* d0s) {
     const std::uint64_t last = a.n - 1;
     if (a.source == 3) {
-        std::uint32_t e[kRounds];
+        std::uint32_t e[R];
 #pragma unroll
-        for (unsigned r = 0; r < kRounds; ++r) e[r] = a.in32[clamp_to(first + r * kWave, last)];
+        for (unsigned r = 0; r < R; ++r) e[r] = a.in32[clamp_to(first + r * kWave, last)];
         const unsigned kb = a.ep.kb;
         const std::uint32_t keyMask = static_cast<std::uint32_t>(a.keyMask);
         const unsigned runs = 1u << a.w0;
@@ -378,7 +384,7 @@ __device__ __forceinline__ void load_elems(const ScatterArgs& a, bool coo, std::
         }
         unsigned d = lo;
 #pragma unroll
-        for (unsigned r = 0; r < kRounds; ++r) {
+        for (unsigned r = 0; r < R; ++r) {
             const std::uint32_t i = static_cast<std::uint32_t>(clamp_to(first + r * kWave, last));
             while (d + 1 < runs && d0s[d + 1] <= i) ++d;
             const std::uint64_t sw = (static_cast<std::uint64_t>(e[r] >> kb) << a.w0) | d;
@@ -386,18 +392,18 @@ __device__ __forceinline__ void load_elems(const ScatterArgs& a, bool coo, std::
             d = static_cast<unsigned>(__builtin_amdgcn_readlane(static_cast<int>(d), kWave - 1));
         }
     } else if (coo) {
-        std::uint32_t d[kRounds], s[kRounds];
+        std::uint32_t d[R], s[R];
 #pragma unroll
-        for (unsigned r = 0; r < kRounds; ++r) {
+        for (unsigned r = 0; r < R; ++r) {
             const std::uint64_t i = clamp_to(first + r * kWave, last);
             d[r] = a.dst[i];
             s[r] = a.src[i];
         }
 #pragma unroll
-        for (unsigned r = 0; r < kRounds; ++r) k[r] = make_elem(d[r], s[r], a.ep);
+        for (unsigned r = 0; r < R; ++r) k[r] = make_elem(d[r], s[r], a.ep);
     } else {
 #pragma unroll
-        for (unsigned r = 0; r < kRounds; ++r) k[r] = a.in[clamp_to(first + r * kWave, last)];
+        for (unsigned r = 0; r < R; ++r) k[r] = a.in[clamp_to(first + r * kWave, last)];
     }
 }
 
@@ -416,8 +422,9 @@ __device__ __forceinline__ void load_elems(const ScatterArgs& a, bool coo, std::
 // so four workgroups fit a compute unit instead of three.  The super-window
 // of a staged element is (digit << w0) | low bits for source 3, and the digit
 // itself for a single pass over all of sw's bits (source 1).
-template <bool S32>
-__global__ void __launch_bounds__(kThreads) elem_scatter_kernel(ScatterArgs a) {
+template <bool S32, unsigned T = kThreads>
+__global__ void __launch_bounds__(T) elem_scatter_kernel(ScatterArgs a) {
+    constexpr unsigned kThreads = T, kWaves = T / kWave, kRounds = kTile / T, kSpan = kWave * kRounds;
     constexpr unsigned kB = S32 ? (1u << kMaxTopDigit) : kMaxBins;
     __shared__ std::uint32_t cnt[kWaves][kB];
     __shared__ std::uint32_t gbase[kB];   // global start of (digit, this tile)
@@ -943,6 +950,12 @@ struct Head {
     unsigned occ;    // row: groups in the row
 };
 
+// The 32 bits from bit i on.
+__device__ __forceinline__ std::uint32_t window32(const std::uint64_t* w, unsigned i) {
+    const auto* h = reinterpret_cast<const std::uint32_t*>(w);
+    return __builtin_amdgcn_alignbit(h[i / 32 + 1], h[i / 32], i % 32);
+}
+
 // Bits [i, i + 64) of a bitmap.
 __device__ __forceinline__ std::uint64_t window64(const std::uint64_t* w, unsigned i) {
     const unsigned k = i >> 6, sh = i & 63;
@@ -960,22 +973,26 @@ __device__ __forceinline__ Head head_at(const TileKeys<K>& tk, unsigned i, unsig
     h.gh = bit_at(tk.group, i);
     h.rh = bit_at(tk.row, i);
     if (h.gh) {
-        const std::uint64_t after = window64(tk.group, i + 1) | (1ull << 8);
-        h.count = min(static_cast<unsigned>(__builtin_ctzll(after)) + 1, avail - i);
+        const std::uint32_t after = window32(tk.group, i + 1) | (1u << 8);
+        h.count = min(static_cast<unsigned>(__builtin_ctz(after)) + 1, avail - i);
         const unsigned deg = min(h.count, 8u);
         // eight unconditional reads (slots past the loaded elements are in
         // the array and masked), so they issue together
         unsigned bits = 0;
 #pragma unroll
-        for (unsigned q = 0; q < 8; ++q) {
-            const unsigned b = 1u << static_cast<unsigned>(tk.key[i + 1 + q] & 7u);
-            bits |= q < deg ? b : 0u;
-        }
+        for (unsigned q = 0; q < 8; ++q)
+            bits |= (q < deg ? 1u : 0u) << (static_cast<unsigned>(tk.key[i + 1 + q]) & 7u);
         h.bits = bits;
     }
     if (h.rh) {
-        const std::uint64_t after = window64(tk.row, i + 1);
-        if (after != 0 && static_cast<unsigned>(__builtin_ctzll(after)) + 1 <= avail - i) {
+        // most rows end within 32 elements: one 32-bit window, then one of
+        // 64 bits, then a walk
+        const std::uint32_t near = window32(tk.row, i + 1);
+        const unsigned len32 = static_cast<unsigned>(__builtin_ctz(near | 0x80000000u)) + 1;  // <= 32
+        const std::uint64_t after = near != 0 ? near : window64(tk.row, i + 1);
+        if (near != 0 && len32 <= avail - i) {
+            h.occ = static_cast<unsigned>(__popc(window32(tk.group, i) & ~(0xFFFFFFFEu << (len32 - 1))));
+        } else if (after != 0 && static_cast<unsigned>(__builtin_ctzll(after)) + 1 <= avail - i) {
             const unsigned len = static_cast<unsigned>(__builtin_ctzll(after)) + 1;  // <= 64
             const std::uint64_t mask = len == 64 ? ~0ull : (1ull << len) - 1ull;
             h.occ = static_cast<unsigned>(__popcll(window64(tk.group, i) & mask));
@@ -987,9 +1004,11 @@ __device__ __forceinline__ Head head_at(const TileKeys<K>& tk, unsigned i, unsig
 }
 
 // countWindowDegreesKernel (:147-213) and the occurrence counts of
-// buildRepeatCacheMetadataKernel (:699-895), per segment tile.
-template <typename K>
-__global__ void __launch_bounds__(kThreads) tile_count_kernel(TileArgs a) {
+// buildRepeatCacheMetadataKernel (:699-895), per segment tile.  Bound by vector
+// instructions (62M edges: 564 us with 64-bit windows of the head bits and
+// every thread's totals added to one LDS address, 449 as here).
+template <typename K, unsigned T>
+__global__ void __launch_bounds__(T) tile_count_kernel(TileArgs a) {
     __shared__ TileKeys<K> tk;
     __shared__ std::uint32_t hist[8 * kMaxS + 33];
     const unsigned t = blockIdx.x;
@@ -998,17 +1017,17 @@ __global__ void __launch_bounds__(kThreads) tile_count_kernel(TileArgs a) {
     const std::uint32_t numTiles = a.firstTile[a.SW];
     const TileInfo ti = a.tileInfo[t];
     if (t >= numTiles) {  // past the last tile: empty columns of the scan
-        for (unsigned b = threadIdx.x; b < nb; b += kThreads) a.counters[static_cast<std::uint64_t>(b) * a.TM + t] = 0;
+        for (unsigned b = threadIdx.x; b < nb; b += T) a.counters[static_cast<std::uint64_t>(b) * a.TM + t] = 0;
         return;
     }
-    for (unsigned b = threadIdx.x; b < nb; b += kThreads) hist[b] = 0;
-    const TileRange r = load_tile<kThreads>(a, t, ti, tk);
+    for (unsigned b = threadIdx.x; b < nb; b += T) hist[b] = 0;
+    const TileRange r = load_tile<T>(a, t, ti, tk);
     std::uint32_t* facts = a.facts();
     const std::uint32_t loMask = (1u << a.loBits) - 1u;
     const unsigned rowBin = 8 * a.S, groupBin = 8 * a.S + 32;
     std::uint32_t groups = 0, rows = 0;
     bool degErr = false, occErr = false;
-    for (unsigned i = threadIdx.x; i < r.n; i += kThreads) {
+    for (unsigned i = threadIdx.x; i < r.n; i += T) {
         const Head h = head_at(tk, i, r.avail);
         const unsigned deg = h.gh ? min(h.count, 8u) : 1u;
         const unsigned wi = (static_cast<std::uint32_t>(tk.key[i + 1]) & loMask) >> 3;
@@ -1029,10 +1048,15 @@ __global__ void __launch_bounds__(kThreads) tile_count_kernel(TileArgs a) {
     }
     if (degErr) atomicMax(a.err, static_cast<std::uint32_t>(TCC_DEVERR_DEGREE));
     if (occErr) atomicMax(a.err, static_cast<std::uint32_t>(TCC_DEVERR_OCCURRENCE));
-    if (groups) atomicAdd(&hist[groupBin], groups);
-    if (rows) atomicAdd(&hist[rowBin], rows);
+    // one add a wave (every lane's, to one address, would queue): at most
+    // 1024 of each in a wave's elements
+    const std::uint32_t both = wave_inclusive_scan(groups | rows << 16);
+    if (__lane_id() == kWave - 1) {
+        atomicAdd(&hist[groupBin], both & 0xFFFFu);
+        atomicAdd(&hist[rowBin], both >> 16);
+    }
     __syncthreads();
-    for (unsigned b = threadIdx.x; b < nb; b += kThreads) a.counters[static_cast<std::uint64_t>(b) * a.TM + t] = hist[b];
+    for (unsigned b = threadIdx.x; b < nb; b += T) a.counters[static_cast<std::uint64_t>(b) * a.TM + t] = hist[b];
 }
 
 // buildWindowMetadataKernel (:216-265): per window, the degree-bucket bases
@@ -1394,6 +1418,12 @@ int tcc_swtcf_convert(const std::uint32_t* dDst, const std::uint32_t* dSrc, std:
         next ^= 1;
         return TCC_OK;
     };
+    auto scatter32 = [&](const ScatterArgs& a) {
+        if (tiles <= device_cus())
+            hipLaunchKernelGGL((elem_scatter_kernel<true, kWideThreads>), dim3(tiles), dim3(kWideThreads), 0, st, a);
+        else
+            hipLaunchKernelGGL((elem_scatter_kernel<true>), dim3(tiles), dim3(kThreads), 0, st, a);
+    };
     if (flow32) {
         // sw pass 0 from the COO (counts from the input pass): the keys and
         // segment heads if it is the only one, else sw >> w0 << kb | key
@@ -1401,7 +1431,7 @@ int tcc_swtcf_convert(const std::uint32_t* dDst, const std::uint32_t* dSrc, std:
         TCC_HIP_CHECK(exclusive_scan(c.histTop, c.histTop, (1ull << w0) * tiles, nullptr, c.temp, st));
         ScatterArgs a0{nullptr, nullptr, dDst, dSrc, plan.ep, E, plan.top[0], c.histTop, tiles, unsorted, 0, 1,
                        one ? B32 : A32, one ? 1 : 2, one ? c.segStart : nullptr, keyMask, nullptr, nullptr, w0};
-        hipLaunchKernelGGL(elem_scatter_kernel<true>, dim3(tiles), dim3(kThreads), 0, st, a0);
+        scatter32(a0);
         TCC_LAUNCH_CHECK();
         if (!one) {
             // sw pass 1: sw's low w0 bits from the position in pass 0's output
@@ -1412,7 +1442,7 @@ int tcc_swtcf_convert(const std::uint32_t* dDst, const std::uint32_t* dSrc, std:
             TCC_HIP_CHECK(exclusive_scan(c.histLow, c.histLow, (1ull << d1.bits) * tiles, nullptr, c.temp, st));
             ScatterArgs a1{nullptr, nullptr, dDst, dSrc, plan.ep, E, plan.top[1], c.histLow, tiles, unsorted, 0, 3,
                            B32, 1, c.segStart, keyMask, A32, c.histTop, w0};
-            hipLaunchKernelGGL(elem_scatter_kernel<true>, dim3(tiles), dim3(kThreads), 0, st, a1);
+            scatter32(a1);
             TCC_LAUNCH_CHECK();
         }
     } else {
@@ -1489,8 +1519,11 @@ int tcc_swtcf_convert(const std::uint32_t* dDst, const std::uint32_t* dSrc, std:
     ta.cachedRowSlot = m->superWindowCachedRowSlot;
 
     // 3. counts, their scan, window and super-window bases
-    if (narrow) hipLaunchKernelGGL(tile_count_kernel<std::uint32_t>, dim3(TM), dim3(kThreads), 0, st, ta);
-    else hipLaunchKernelGGL(tile_count_kernel<std::uint64_t>, dim3(TM), dim3(kThreads), 0, st, ta);
+    if (narrow && TM <= device_cus())
+        hipLaunchKernelGGL((tile_count_kernel<std::uint32_t, kWideThreads>), dim3(TM), dim3(kWideThreads), 0, st, ta);
+    else if (narrow)
+        hipLaunchKernelGGL((tile_count_kernel<std::uint32_t, kThreads>), dim3(TM), dim3(kThreads), 0, st, ta);
+    else hipLaunchKernelGGL((tile_count_kernel<std::uint64_t, kThreads>), dim3(TM), dim3(kThreads), 0, st, ta);
     TCC_LAUNCH_CHECK();
     TCC_HIP_CHECK(exclusive_scan(c.counters, c.counters, nCounters, c.counters + nCounters, c.temp, st));
     hipLaunchKernelGGL(window_meta_kernel, dim3(grid_for(CW, kThreads)), dim3(kThreads), 0, st, c.counters, TM,
