@@ -161,7 +161,7 @@ int tcc_swtcf_spmm_mfma(const tcc_swtcf_matrix* m, const float* X, float* Y, uin
  * 0.5 GB at 233k rows and 114M edges) or its BCSR, and a workspace (or
  * packed X) for the last feature width. */
 int tcc_swtcf_set_plans(uint32_t maxPlans);
-/* Releases every kept plan. */
+/* Releases every kept plan, and the device memory kept for the builders. */
 int tcc_swtcf_release_plans(void);
 /* Plans built since the process started. */
 uint32_t tcc_swtcf_plans_built(void);
