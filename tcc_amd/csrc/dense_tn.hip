@@ -479,19 +479,25 @@ __global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
 // of AX (the first layer's transform, its activation and the second layer's
 // transform of a two-layer GCN; tcgnn_conv_release.py:134 and :243-247).
 //
-// A wave computes 16 rows x 256 hidden units (16 tiles of 16x16) over
-// F <= 16*KB inputs with v_mfma_f32_16x16x4f32.  Lane (q = l/16, i = l%16)
-// loads AX[row0 + i][16b + 4q .. +3] as one float4 per block b of 16 inputs,
-// and MFMA step s of block b takes input 16b + 4q + s on lane quarter q: the
-// sum over the 16 inputs is the same in any order, so the four steps come
-// from one float4 instead of four strided loads.  The matching B operands,
-// W1[16b + 4q + s][16u + i] for s = 0..3, are one ds_read_b128 from W1^T
-// held in LDS (row pitch 16*KB + 4 floats: conflict-free b128 reads).
-// Relu, the store of H and the row sums of H W2 (a 16-lane butterfly) follow
-// in registers.  Workgroups (one per CU for the LDS copy of W1^T, 12 waves:
-// 1.44 ms for 2.45M x 100 x 256 against 1.59-1.68 ms with 8, before the
-// interleaved MFMA steps below) are persistent
-// over 16-row tiles.
+// fp32 MFMA held this at 1.40 ms for 2.45M x 100 x 256; as tn_split_kernel, the
+// operands are three bf16 parts each (split3) and a product is six part
+// products: 1.03 ms, against 0.74 for AX and H at the rate of a large copy
+// (200k rows 162 -> 102 us, 2000 rows 37 -> 13).  H's error against 64 bits
+// 1.8e-7 -> 5.5e-8 of it.
+//
+// Workgroup = 8 waves, one to a compute unit, persistent over steps of 64 rows.
+// Wave w holds the parts of W1's columns 32w .. 32w+31 in registers (first
+// operand: lane l%16 is the hidden unit, 8 inputs from 8 (l/16) + 32 ks on),
+// split once.  A step's rows are split once per workgroup: thread t takes
+// inputs 8 (t%16) ..+7 of rows t/16 and t/16 + 32, and writes their parts to
+// LDS as [part][8 inputs][row], 65 rows apart so that the 16 threads of a row
+// meet different banks.  LDS holds two steps, and of the two waves of a SIMD one
+// stages the next step first and the other multiplies first.  A lane ends with 4
+// consecutive hidden units of a row: relu, a float4 store of H, and the sum over
+// a wave's units, by lane and then over the waves through LDS, for H W2.
+//
+// A wave whose sums are not all finite, whose part of W1 has a column too small
+// to split or whose step has such a row forms its block with fp32 products.
 struct ReluFwdArgs {
     const float* AX;
     const float* W1;  // [F x Hd]
@@ -500,139 +506,220 @@ struct ReluFwdArgs {
     float* XW;
     std::uint32_t ldax, ldh, ldxw;
     std::uint32_t K, F, Hd, C;
-    std::uint32_t tiles;  // ceil(K / 16)
-    int vec;              // AX rows allow float4 loads
+    std::uint32_t steps;  // ceil(K / 64)
+    int vecH;             // H rows allow float4 stores
 };
 
-constexpr unsigned kFwdWaves = 12;  // waves per workgroup (one workgroup per CU: the LDS copy of W1^T)
-constexpr int kFwdTiles = 16;       // 16 tiles of 16 hidden units per wave
-
-template <int KB>
-__device__ __forceinline__ void fwd_load_rows(const ReluFwdArgs& a, std::uint32_t tile, float4 (&x)[KB]) {
+template <int KS, int CT, bool VEC>
+__global__ void __launch_bounds__(512) gcn_relu_forward_kernel(ReluFwdArgs a) {
+    constexpr std::uint32_t kPitch = 65;                      // rows of a group of inputs, in 16 bytes
+    constexpr std::uint32_t kPart = 4 * KS * kPitch, kStage = 3 * kPart;
+    extern __shared__ uint4 parts[];                          // [2 steps][3 parts][4 KS groups][65]
+    __shared__ float red[2][8][64][CT];                       // a step's H W2, by wave
+    // a step has had a row too small to split; kept for its half's later steps
+    // (cleared, it would take another barrier)
+    __shared__ std::uint32_t small[2];
     const unsigned lane = __lane_id();
-    const std::uint32_t row = tile * 16 + (lane & 15u);
-    const unsigned q = lane >> 4;
-#pragma unroll
-    for (int b = 0; b < KB; ++b) {
-        const std::uint32_t k = 16 * b + 4 * q;
-        x[b] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (row >= a.K || tile >= a.tiles) continue;
-        const float* p = a.AX + static_cast<std::uint64_t>(row) * a.ldax + k;
-        if (a.vec && k + 3 < a.F) {
-            x[b] = *reinterpret_cast<const float4*>(p);
-        } else {
-            if (k < a.F) x[b].x = p[0];
-            if (k + 1 < a.F) x[b].y = p[1];
-            if (k + 2 < a.F) x[b].z = p[2];
-            if (k + 3 < a.F) x[b].w = p[3];
-        }
-    }
-}
-
-// PF: load the next tile's rows during the current tile's products (with 12
-// waves per CU measured no faster than without, 1.44-1.57 ms for
-// 2.45M x 100 x 256, and 28 VGPRs more).
-template <int KB, int CT, unsigned W = kFwdWaves, bool PF = false>
-__global__ void __launch_bounds__(kWave * W) gcn_relu_forward_kernel(ReluFwdArgs a) {
-    constexpr int KP = 16 * KB + 4;  // LDS row pitch of W1^T (floats)
-    extern __shared__ float w1t[];   // [256][KP], then W2 [256][CT]
-    const unsigned lane = __lane_id();
-    const unsigned i = lane & 15u, q = lane >> 4;
+    const unsigned li = lane & 15u, lk = lane >> 4;
     const unsigned wave = tn_uniform(threadIdx.x / kWave);
+    const bool first = wave < 4;  // waves w and w + 4 share a SIMD
 
-    // W1^T into LDS, zeros past F and Hd.
-    for (std::uint32_t e = threadIdx.x; e < 256u * KP; e += blockDim.x) {
-        const std::uint32_t n = e / KP, k = e - n * KP;
-        w1t[e] = (n < a.Hd && k < a.F) ? a.W1[static_cast<std::uint64_t>(k) * a.Hd + n] : 0.0f;
-    }
-    // W2 [256][CT] after it, zeros past Hd and C.
-    float* w2 = w1t + 256 * KP;
-    for (std::uint32_t e = threadIdx.x; e < 256u * CT; e += blockDim.x) {
-        const std::uint32_t n = e / CT, j = e - n * CT;
-        w2[e] = (n < a.Hd && j < a.C) ? a.W2[static_cast<std::uint64_t>(n) * a.C + j] : 0.0f;
-    }
-    __syncthreads();
-
-    const std::uint32_t stride = gridDim.x * W;
-    std::uint32_t tile = blockIdx.x * W + wave;
-    float4 x[KB];
-    if (PF) fwd_load_rows<KB>(a, tile, x);
-    for (; tile < a.tiles; tile += stride) {
-        float4 nx[KB];
-        if (PF) {
-            fwd_load_rows<KB>(a, tile + stride, nx);  // past the last tile: zeros, no loads
-        } else {
-            fwd_load_rows<KB>(a, tile, x);
+    // The wave's part of W1 and this lane's of W2.
+    bf16x8 w[2][KS][3];
+    bool redoAll = false;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const std::uint32_t n = 32 * wave + 16 * u + li;
+        float top = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            std::uint32_t part[3][4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float x[2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const std::uint32_t k = 32 * ks + 8 * lk + 2 * q + e;
+                    x[e] = n < a.Hd && k < a.F ? a.W1[static_cast<std::uint64_t>(k) * a.Hd + n] : 0.0f;
+                    top = fmaxf(top, fabsf(x[e]));
+                }
+                split3(x[0], x[1], part[0][q], part[1][q], part[2][q]);
+            }
+#pragma unroll
+            for (int s = 0; s < 3; ++s)
+                w[u][ks][s] = __builtin_bit_cast(bf16x8, make_uint4(part[s][0], part[s][1], part[s][2], part[s][3]));
         }
-        __builtin_amdgcn_sched_barrier(0);
-        f32x4 acc[kFwdTiles];
+        top = fmaxf(top, __shfl_xor(top, 16));
+        top = fmaxf(top, __shfl_xor(top, 32));
+        redoAll |= __ballot(top != 0.0f && top < kSplitTiny) != 0;
+    }
+    float w2[2][4][CT];
 #pragma unroll
-        for (int u = 0; u < kFwdTiles; ++u) acc[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        // W1^T rows as float4 (KP % 4 == 0): ds_read_b128.  Each step s runs
-        // over 8 accumulators before the next, so no MFMA waits on the one
-        // before it.
-        const float4* w1t4 = reinterpret_cast<const float4*>(w1t);
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int b = 0; b < KB; ++b) {
+        for (int v = 0; v < 4; ++v) {
+            const std::uint32_t n = 32 * wave + 16 * u + 4 * lk + v;
 #pragma unroll
-            for (int h = 0; h < kFwdTiles; h += 8) {
-                float4 w[8];
+            for (int j = 0; j < CT; ++j)
+                w2[u][v][j] = n < a.Hd && static_cast<std::uint32_t>(j) < a.C
+                                  ? a.W2[static_cast<std::uint64_t>(n) * a.C + j] : 0.0f;
+        }
+
+    // This thread's inputs (clamped loads, zeros past F when staged).
+    const std::uint32_t kg = threadIdx.x & 15u, row0 = threadIdx.x >> 4;
+    const bool mine = kg < 4 * KS;
+    float x[2][8];
+    auto load = [&](std::uint32_t step) {
 #pragma unroll
-                for (int t = 0; t < 8; ++t) w[t] = w1t4[(16 * (h + t) + i) * (KP / 4) + 4 * b + q];
+        for (std::uint32_t h = 0; h < 2; ++h) {
+            const std::uint64_t at = static_cast<std::uint64_t>(step) * 64 + row0 + 32 * h;
+            const float* r = a.AX + (at < a.K ? at : a.K - 1) * a.ldax;
+            if constexpr (VEC) {
 #pragma unroll
-                for (int t = 0; t < 8; ++t) acc[h + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[b].x, w[t].x, acc[h + t], 0, 0, 0);
+                for (std::uint32_t q = 0; q < 2; ++q) {
+                    const float4 v = *reinterpret_cast<const float4*>(r + min(8 * kg + 4 * q, a.F - 4));
+                    x[h][4 * q] = v.x, x[h][4 * q + 1] = v.y, x[h][4 * q + 2] = v.z, x[h][4 * q + 3] = v.w;
+                }
+            } else {
 #pragma unroll
-                for (int t = 0; t < 8; ++t) acc[h + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[b].y, w[t].y, acc[h + t], 0, 0, 0);
-#pragma unroll
-                for (int t = 0; t < 8; ++t) acc[h + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[b].z, w[t].z, acc[h + t], 0, 0, 0);
-#pragma unroll
-                for (int t = 0; t < 8; ++t) acc[h + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[b].w, w[t].w, acc[h + t], 0, 0, 0);
+                for (std::uint32_t e = 0; e < 8; ++e) x[h][e] = r[min(8 * kg + e, a.F - 1)];
             }
         }
-        // Lane holds H(row0 + 4q + v, 16u + i): relu (NaN kept, as clamp_min),
-        // store, and this lane's part of the row sums of H W2.
-        const std::uint32_t row0 = tile * 16 + 4 * q;
-        float xw[4][CT];
+    };
+    auto stage = [&](unsigned buf) {
+        uint4* const to = parts + buf * kStage;
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
+        for (std::uint32_t h = 0; h < 2; ++h) {
+            std::uint32_t hi[4], mid[4], lo[4];
+            float top = 0.0f;
 #pragma unroll
-            for (int j = 0; j < CT; ++j) xw[v][j] = 0.0f;
-#pragma unroll
-        for (int u = 0; u < kFwdTiles; ++u) {
-            const std::uint32_t n = 16 * u + i;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const float h = acc[u][v] < 0.0f ? 0.0f : acc[u][v];
-                if (row0 + v < a.K && n < a.Hd) a.H[static_cast<std::uint64_t>(row0 + v) * a.ldh + n] = h;
-#pragma unroll
-                for (int j = 0; j < CT; ++j) xw[v][j] = fmaf(h, w2[n * CT + j], xw[v][j]);
+            for (std::uint32_t q = 0; q < 4; ++q) {
+                const float p = 8 * kg + 2 * q < a.F ? x[h][2 * q] : 0.0f;
+                const float r = 8 * kg + 2 * q + 1 < a.F ? x[h][2 * q + 1] : 0.0f;
+                top = fmaxf(top, fmaxf(fabsf(p), fabsf(r)));
+                split3(p, r, hi[q], mid[q], lo[q]);
             }
-        }
+            if (mine) {
+                uint4* const at = to + kg * kPitch + row0 + 32 * h;
+                at[0] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+                at[kPart] = make_uint4(mid[0], mid[1], mid[2], mid[3]);
+                at[2 * kPart] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+            }
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
+            for (unsigned d = 1; d < 16; d *= 2) top = fmaxf(top, __shfl_xor(top, d));
+            if (top != 0.0f && top < kSplitTiny) small[buf] = 1;
+        }
+    };
+    auto multiply = [&](std::uint32_t step, unsigned buf) {
+        const uint4* const from = parts + buf * kStage;
+        const bool redoStep = redoAll || small[buf] != 0;
+#pragma unroll
+        for (std::uint32_t rt = 0; rt < 4; ++rt) {
+            f32x4 acc[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
+            constexpr int kW[6] = {2, 0, 1, 1, 0, 0}, kX[6] = {0, 2, 1, 0, 1, 0};
+            bf16x8 b[KS][3];
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int s = 0; s < 3; ++s)
+                    b[ks][s] = __builtin_bit_cast(bf16x8, from[s * kPart + (4 * ks + lk) * kPitch + 16 * rt + li]);
+            // the smallest part products of all inputs first
+#pragma unroll
+            for (int s = 0; s < 6; ++s)
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                    for (int u = 0; u < 2; ++u)
+                        acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][ks][kW[s]], b[ks][kX[s]], acc[u], 0, 0, 0);
+            bool redo = redoStep;
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) redo |= !(fabsf(acc[u][v]) <= 0x1.fffffep127f);
+            const std::uint64_t row = static_cast<std::uint64_t>(step) * 64 + 16 * rt + li;
+            if (__ballot(redo)) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u) acc[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                const float* r = a.AX + (row < a.K ? row : a.K - 1) * a.ldax;
+                for (std::uint32_t k = 0; k < a.F; k += 4) {
+                    const std::uint32_t kk = k + lk;
+                    const float xv = kk < a.F ? r[kk] : 0.0f;
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const std::uint32_t n = 32 * wave + 16 * u + li;
+                        const float wv = kk < a.F && n < a.Hd ? a.W1[static_cast<std::uint64_t>(kk) * a.Hd + n] : 0.0f;
+                        acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv, xv, acc[u], 0, 0, 0);
+                    }
+                }
+            }
+            // Lane holds H(row, 32 wave + 16 u + 4 lk + v): relu (NaN kept, as clamp_min).
+            float xw[CT];
+#pragma unroll
+            for (int j = 0; j < CT; ++j) xw[j] = 0.0f;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                float h[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    // units past Hd are 0 times the row: NaN for an infinity
+                    h[v] = acc[u][v] < 0.0f || 32 * wave + 16 * u + 4 * lk + v >= a.Hd ? 0.0f : acc[u][v];
+#pragma unroll
+                    for (int j = 0; j < CT; ++j) xw[j] = fmaf(h[v], w2[u][v][j], xw[j]);
+                }
+                const std::uint32_t n = 32 * wave + 16 * u + 4 * lk;
+                float* o = a.H + row * a.ldh + n;
+                if (row < a.K && a.vecH) {
+                    if (n < a.Hd) *reinterpret_cast<float4*>(o) = make_float4(h[0], h[1], h[2], h[3]);
+                } else if (row < a.K) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        if (n + v < a.Hd) o[v] = h[v];
+                }
+            }
 #pragma unroll
             for (int j = 0; j < CT; ++j) {
-                float t = xw[v][j];
-                t += __shfl_xor(t, 1);
-                t += __shfl_xor(t, 2);
-                t += __shfl_xor(t, 4);
-                t += __shfl_xor(t, 8);
-                if (i == 0 && row0 + v < a.K && static_cast<std::uint32_t>(j) < a.C)
-                    a.XW[static_cast<std::uint64_t>(row0 + v) * a.ldxw + j] = t;
+                xw[j] += __shfl_xor(xw[j], 16);
+                xw[j] += __shfl_xor(xw[j], 32);
+                if (lk == 0) red[buf][wave][16 * rt + li][j] = xw[j];
             }
-        if (PF) {
+        }
+    };
+
+    std::uint32_t step = blockIdx.x;
+    if (threadIdx.x < 2) small[threadIdx.x] = 0;
+    __syncthreads();
+    load(step);
+    stage(0);
+    load(step + gridDim.x);  // past the last: the last row again
+    __syncthreads();
+    for (unsigned buf = 0; step < a.steps; step += gridDim.x, buf ^= 1u) {
+        if (!first) multiply(step, buf);
+        __builtin_amdgcn_sched_barrier(0);
+        stage(buf ^ 1u);
+        load(step + 2 * gridDim.x);
+        __builtin_amdgcn_sched_barrier(0);
+        if (first) multiply(step, buf);
+        __syncthreads();
+        // this step's H W2, its waves' sums in order; the next step's go to the
+        // other half of `red`
+        if (threadIdx.x < 64 * CT) {
+            const std::uint32_t r = threadIdx.x / CT, j = threadIdx.x % CT;
+            const std::uint64_t row = static_cast<std::uint64_t>(step) * 64 + r;
+            float t = 0.0f;
 #pragma unroll
-            for (int b = 0; b < KB; ++b) x[b] = nx[b];
+            for (int v = 0; v < 8; ++v) t += red[buf][v][r][j];
+            if (row < a.K && j < a.C) a.XW[row * a.ldxw + j] = t;
         }
     }
 }
 
-template <int KB, int CT, unsigned W = kFwdWaves>
+template <int KS, int CT>
 void relu_forward_launch(const ReluFwdArgs& a, hipStream_t st) {
-    const std::uint32_t lds = 256u * (16 * KB + 4 + CT) * sizeof(float);
-    const std::uint32_t grid = std::min<std::uint32_t>(device_cus(), (a.tiles + W - 1) / W);
-    hipLaunchKernelGGL((gcn_relu_forward_kernel<KB, CT, W>), dim3(std::max<std::uint32_t>(grid, 1)), dim3(kWave * W),
-                       lds, st, a);
+    constexpr std::uint32_t lds = 2 * 3 * 4 * KS * 65 * 16;
+    const bool vec = a.F % 4 == 0 && a.ldax % 4 == 0 && reinterpret_cast<std::uintptr_t>(a.AX) % 16 == 0;
+    const dim3 grid(std::max<std::uint32_t>(1, std::min<std::uint32_t>(device_cus(), a.steps)));
+    if (vec) hipLaunchKernelGGL((gcn_relu_forward_kernel<KS, CT, true>), grid, dim3(512), lds, st, a);
+    else hipLaunchKernelGGL((gcn_relu_forward_kernel<KS, CT, false>), grid, dim3(512), lds, st, a);
 }
 
 // C[m][n] (=|+=) sum over splits of partial[s][m][n], splits added in a fixed
@@ -890,13 +977,14 @@ int tcc_gcn_relu_forward(const float* AX, std::uint32_t ldax, const float* W1, c
     a.F = F;
     a.Hd = Hd;
     a.C = C;
-    a.tiles = (K + 15) / 16;
-    a.vec = (ldax % 4 == 0) && (reinterpret_cast<std::uintptr_t>(AX) % 16 == 0);
+    a.steps = static_cast<std::uint32_t>((static_cast<std::uint64_t>(K) + 63) / 64);
+    a.vecH = Hd % 4 == 0 && ldh % 4 == 0 && reinterpret_cast<std::uintptr_t>(H) % 16 == 0;
     const hipStream_t st = as_stream(stream);
     const bool two = C <= 2;
-    if (F <= 64) two ? relu_forward_launch<4, 2>(a, st) : relu_forward_launch<4, 4>(a, st);
-    else if (F <= 112) two ? relu_forward_launch<7, 2>(a, st) : relu_forward_launch<7, 4>(a, st);
-    else two ? relu_forward_launch<8, 2>(a, st) : relu_forward_launch<8, 4>(a, st);
+    if (F <= 32) two ? relu_forward_launch<1, 2>(a, st) : relu_forward_launch<1, 4>(a, st);
+    else if (F <= 64) two ? relu_forward_launch<2, 2>(a, st) : relu_forward_launch<2, 4>(a, st);
+    else if (F <= 96) two ? relu_forward_launch<3, 2>(a, st) : relu_forward_launch<3, 4>(a, st);
+    else two ? relu_forward_launch<4, 2>(a, st) : relu_forward_launch<4, 4>(a, st);
     TCC_LAUNCH_CHECK();
     return TCC_OK;
 }

@@ -116,3 +116,35 @@ def test_relu_gradient_edges(gpu, K, C):
             # d itself is a sum of C rounded products
             assert ((got - want)[fin].abs() <= 2 * BOUND * mag[fin]).all()
         assert special or bool(torch.isfinite(dW1).all())
+
+
+@pytest.mark.parametrize("C", [1, 2, 4])
+@pytest.mark.parametrize("K", [1, 63, 64, 65, 20_000])
+@pytest.mark.parametrize("F,Hd", [(3, 5), (32, 256), (33, 255), (64, 32), (65, 33), (97, 130), (100, 256), (128, 100)])
+def test_relu_forward_edges(gpu, K, F, Hd, C):
+    """H and H W2 at the edges of the forward's steps and blocks, with rows and
+    columns too small to split and (in the last pass) an infinity and a NaN."""
+    from tcc_amd import swtcf
+
+    g = torch.Generator(device="cuda").manual_seed(K + F + C)
+    for special in range(3):
+        AX = torch.randn(K, F + 1, generator=g, device="cuda")[:, :F] if special == 1 else \
+            torch.randn(K, F, generator=g, device="cuda")
+        W1, W2 = torch.randn(F, Hd, generator=g, device="cuda"), torch.randn(Hd, C, generator=g, device="cuda")
+        if special == 1:
+            AX[K // 2] *= 1e-33
+            W1[:, Hd // 2] *= 1e-34
+        if special == 2:
+            AX[K - 1, F // 2] = float("inf")
+            AX[0, 0] = float("nan")
+        H, XW = swtcf.gcn_relu_forward(AX, W1, W2)
+        pre = AX.double() @ W1.double()
+        want = torch.where(pre < 0, torch.zeros_like(pre), pre)
+        fin = torch.isfinite(want)
+        assert torch.equal(torch.isnan(H), torch.isnan(want)) and torch.equal(torch.isinf(H), torch.isinf(want))
+        mag = AX.double().abs() @ W1.double().abs()
+        assert ((H.double() - want)[fin].abs() <= BOUND * mag[fin] + F * 2.0**-126).all()
+        xw, xmag = H.double() @ W2.double(), H.double().abs() @ W2.double().abs()
+        ok = torch.isfinite(xw)
+        assert torch.equal(torch.isfinite(XW), ok)
+        assert ((XW.double() - xw)[ok].abs() <= Hd * 2.0**-23 * xmag[ok] + Hd * 2.0**-126).all()
