@@ -62,8 +62,9 @@ int tcc_dense_tn_noalloc(const float* A, uint32_t lda, const float* B, uint32_t 
  * second layer's transform of a two-layer GCN, which the reference runs as
  * X_gat = torch.mm(X_out, weights) (train/tcgnn_conv_release.py:134),
  * self.relu (:231-238) and the last layer's torch.mm (:134 again) with H
- * written and read back in between.  fp32 MFMA products and sums; relu
- * keeps NaN (clamp_min).  F <= 128, Hd <= 256, C <= 4 (TCC_ERR_UNSUPPORTED
+ * written and read back in between.  Products of exact bf16 parts of the fp32
+ * operands, summed in fp32 (no less accurate than fp32 MFMA); relu keeps NaN
+ * (clamp_min).  F <= 128, Hd <= 256, C <= 4 (TCC_ERR_UNSUPPORTED
  * above).  No workspace. */
 int tcc_gcn_relu_forward(const float* AX, uint32_t ldax, const float* W1, const float* W2, float* H, uint32_t ldh,
                          float* XW, uint32_t ldxw, uint32_t K, uint32_t F, uint32_t Hd, uint32_t C, void* stream);

@@ -7,7 +7,7 @@ CNICSPMMFunction mirrors the reference's autograd function
             spmm_launcher.cu:30-271), out = AX·W                (:130-134)
   backward: dW = AXᵀ·dY, G = Aᵀ·dY, dX = G·Wᵀ                    (:147-154)
 The weight gradients AXᵀ·dY and Xᵀ·G are tall-skinny products over all nodes
-(tcc_dense_tn: K split over workgroups on fp32 MFMA), where library GEMMs
+(tcc_dense_tn: K split over workgroups on MFMA, of fp32 accuracy), where library GEMMs
 reach a fraction of the GPU on this shape.
 The reference's G = torch.sparse.mm(Aᵀ, dY) over unit values (:139-142, :152)
 is the block-sparse transposed gather over a BCSC of the whole A

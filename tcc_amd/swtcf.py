@@ -515,7 +515,8 @@ def dense_tn(A: torch.Tensor, B: torch.Tensor, C: torch.Tensor | None = None, ac
              stream=None) -> torch.Tensor:
     """C[M x N] (=|+=) A^T B for A [K x M], B [K x N] (tcc_dense_tn): the
     weight gradient torch.mm(X_out.T, d_output) of the GCN layer backward
-    (train/tcgnn_conv_release.py:150), split over K on fp32 MFMA."""
+    (train/tcgnn_conv_release.py:150), split over K on MFMA, of fp32
+    accuracy."""
     A, B = _rows(A, "A"), _rows(B, "B")
     K, M = A.shape
     if B.shape[0] != K:
