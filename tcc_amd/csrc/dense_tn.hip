@@ -171,9 +171,18 @@ __device__ __forceinline__ void split3(float x0, float x1, std::uint32_t& hi, st
     lo = pack(r0 - __uint_as_float(mid << 16), r1 - __uint_as_float(mid & 0xFFFF0000u));
 }
 
-// Column maxima of |x| below this (and above zero) are left to the fp32
-// products: their lowest parts would fall under bf16's smallest normal number.
-constexpr float kSplitTiny = 0x1p-96f;
+// A split is exact from 2^-110 on; parts of a smaller element go below bf16's
+// smallest number, 2^-133 (the MFMA keeps subnormal operands and sums), and up
+// to 2^-134 of it is lost.  Whether that counts depends on what the element
+// meets: 2^-120 beside ones is nothing, against 2^119 it is most of the result.
+// So a block is formed again with fp32 products where a loss in each of `rows`
+// products, by the largest element of the other operand's column, comes to more
+// than 2^-24 of an element of the result.
+__device__ __forceinline__ float split_loss(std::uint32_t rows) { return 0x1p-109f * static_cast<float>(rows); }
+
+// Smaller for smaller |x|, zero (which a split keeps) the largest.
+__device__ __forceinline__ std::uint32_t smallness(float x) { return (__float_as_uint(x) << 1) - 1u; }
+constexpr std::uint32_t kSplitExactBits = ((127u - 110u) << 24) - 1u;  // of 2^-110
 
 // Wide outputs.  fp32 MFMA runs at 1/16 of the bf16 rate, and the 100 x 256
 // and 602 x 256 products over node rows were bound by it (110 TFLOP/s).  Here
@@ -201,7 +210,8 @@ constexpr float kSplitTiny = 0x1p-96f;
 //
 // Infinities and NaN do not survive a split (and a sum near the largest float
 // may overflow in parts only): a workgroup whose sums are not all finite, or
-// with a column too small to split, forms its block again with fp32 products.
+// with elements too small to split that count, forms its block again with fp32
+// products.
 //
 // CT > 0 is the GCN relu-gradient form: B holds H (the relu output of the
 // layer, [K x N]) and the B operand is formed while it is staged as
@@ -252,7 +262,8 @@ __global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
             w2[e][j] = CT > 0 && static_cast<std::uint32_t>(j) < a.C
                            ? a.W2[static_cast<std::uint64_t>(colB[e]) * a.C + j] : 0.0f;
         }
-    float maxA = 0.0f, maxB[2] = {0.0f, 0.0f};
+    float maxA = 0.0f, maxB[2] = {0.0f, 0.0f};  // of the columns' magnitudes
+    std::uint32_t lowA = ~0u, lowB[2] = {~0u, ~0u};
 
     f32x4 acc[TW][4];
 #pragma unroll
@@ -283,12 +294,13 @@ __global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
             xg = a.G[static_cast<std::uint64_t>(min(row, k1 - 1)) * a.ldg + min(gj, a.C - 1)];
         }
     };
-    auto put = [&](uint4* to, std::uint32_t part, const float (&x)[8], float& top) {
+    auto put = [&](uint4* to, std::uint32_t part, const float (&x)[8], float& top, std::uint32_t& low) {
         std::uint32_t h[4], m[4], l[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             split3(x[2 * q], x[2 * q + 1], h[q], m[q], l[q]);
-            top = fmaxf(top, fmaxf(fabsf(x[2 * q]), fabsf(x[2 * q + 1])));
+            if constexpr (CT > 0) top = fmaxf(top, fmaxf(fabsf(x[2 * q]), fabsf(x[2 * q + 1])));
+            low = min(low, min(smallness(x[2 * q]), smallness(x[2 * q + 1])));
         }
         to[0] = make_uint4(h[0], h[1], h[2], h[3]);
         to[part] = make_uint4(m[0], m[1], m[2], m[3]);
@@ -305,7 +317,7 @@ __global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
             float x[8];
 #pragma unroll
             for (int r = 0; r < 8; ++r) x[r] = f[r] * xa[r];
-            put(to + wn * BM + at, kPartA, x, maxA);
+            put(to + wn * BM + at, kPartA, x, maxA, lowA);
         }
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
@@ -334,7 +346,7 @@ __global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
 #pragma unroll
                 for (int j = 0; j < GC; ++j) dw2[e][j] += part[j];
             }
-            put(to + 3 * kPartA + wn * BN + 128 * e + at, kPartB, x, maxB[e]);
+            put(to + 3 * kPartA + wn * BN + 128 * e + at, kPartB, x, maxB[e], lowB[e]);
         }
     };
     // B's tile u of this wave: positions 128 (u / 2) + 32 wn + 16 (u % 2) + l%16.
@@ -393,8 +405,53 @@ __global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
     const int tiles = wm == 0 ? TW : TM / 2;
 
     bool redo = false;
-    auto tiny = [&](float top) { return top != 0.0f && top < kSplitTiny; };
-    redo |= tiny(maxA) || tiny(maxB[0]) || tiny(maxB[1]);
+    const bool tinyA = lowA < kSplitExactBits, tinyB[2] = {lowB[0] < kSplitExactBits, lowB[1] < kSplitExactBits};
+    if (__syncthreads_or(tinyA || tinyB[0] || tinyB[1])) {
+        // the columns' maxima and losses, of the four waves' rows: [4][BM] and
+        // [4][BN] of each
+        float* const topA = reinterpret_cast<float*>(parts);
+        float* const lossA = topA + 4 * BM;
+        float* const topB = lossA + 4 * BM;
+        float* const lossB = topB + 4 * BN;
+        const float loss = split_loss(k1 - k0);
+        if constexpr (CT == 0) {  // the maxima, here alone: the products' loop is full without them
+            for (std::uint32_t k = k0; k < k1; k += 32) {
+                load(k);
+#pragma unroll
+                for (int r = 0; r < 8; ++r) {
+                    maxA = fmaxf(maxA, fabsf(xa[r]));
+                    maxB[0] = fmaxf(maxB[0], fabsf(xb[r][0]));
+                    maxB[1] = fmaxf(maxB[1], fabsf(xb[r][1]));
+                }
+            }
+        }
+        if (at < BM) {
+            topA[wn * BM + at] = maxA;
+            lossA[wn * BM + at] = tinyA ? loss : 0.0f;
+        }
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            topB[wn * BN + 2 * at + e] = maxB[e];
+            lossB[wn * BN + 2 * at + e] = tinyB[e] ? loss : 0.0f;
+        }
+        __syncthreads();
+        const auto most = [](const float* x, std::uint32_t i, std::uint32_t n) {
+            return fmaxf(fmaxf(x[i], x[n + i]), fmaxf(x[2 * n + i], x[3 * n + i]));
+        };
+#pragma unroll
+        for (int t = 0; t < TW; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                if (t >= tiles) continue;
+                const std::uint32_t m = mcol(t, 4 * lk + v) - m0;
+                const float am = most(topA, m, BM), al = most(lossA, m, BM);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const std::uint32_t n = ncol(u) - n0;
+                    redo |= !(fabsf(acc[t][u][v]) >= al * most(topB, n, BN) + am * most(lossB, n, BN));
+                }
+            }
+    }
 #pragma unroll
     for (int t = 0; t < TW; ++t)
 #pragma unroll
@@ -496,8 +553,9 @@ __global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
 // consecutive hidden units of a row: relu, a float4 store of H, and the sum over
 // a wave's units, by lane and then over the waves through LDS, for H W2.
 //
-// A wave whose sums are not all finite, whose part of W1 has a column too small
-// to split or whose step has such a row forms its block with fp32 products.
+// A wave whose sums are not all finite forms its block with fp32 products, and
+// so does one where elements too small to split count (a step or a part of W1
+// that holds such an element is looked at closer).
 struct ReluFwdArgs {
     const float* AX;
     const float* W1;  // [F x Hd]
@@ -516,9 +574,10 @@ __global__ void __launch_bounds__(512) gcn_relu_forward_kernel(ReluFwdArgs a) {
     constexpr std::uint32_t kPart = 4 * KS * kPitch, kStage = 3 * kPart;
     extern __shared__ uint4 parts[];                          // [2 steps][3 parts][4 KS groups][65]
     __shared__ float red[2][8][64][CT];                       // a step's H W2, by wave
-    // a step has had a row too small to split; kept for its half's later steps
-    // (cleared, it would take another barrier)
-    __shared__ std::uint32_t small[2];
+    __shared__ std::uint32_t small[2];                        // 1 + the last step with an element too small to split
+    // largest magnitude of W1's columns and of a step's rows (where either
+    // holds one), negative with elements too small to split
+    __shared__ float rowTop[2][64], colTop[256];
     const unsigned lane = __lane_id();
     const unsigned li = lane & 15u, lk = lane >> 4;
     const unsigned wave = tn_uniform(threadIdx.x / kWave);
@@ -526,11 +585,12 @@ __global__ void __launch_bounds__(512) gcn_relu_forward_kernel(ReluFwdArgs a) {
 
     // The wave's part of W1 and this lane's of W2.
     bf16x8 w[2][KS][3];
-    bool redoAll = false;
+    bool smallW = false;  // an element of the wave's part
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
         const std::uint32_t n = 32 * wave + 16 * u + li;
         float top = 0.0f;
+        std::uint32_t low = ~0u;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             std::uint32_t part[3][4];
@@ -542,6 +602,7 @@ __global__ void __launch_bounds__(512) gcn_relu_forward_kernel(ReluFwdArgs a) {
                     const std::uint32_t k = 32 * ks + 8 * lk + 2 * q + e;
                     x[e] = n < a.Hd && k < a.F ? a.W1[static_cast<std::uint64_t>(k) * a.Hd + n] : 0.0f;
                     top = fmaxf(top, fabsf(x[e]));
+                    low = min(low, smallness(x[e]));
                 }
                 split3(x[0], x[1], part[0][q], part[1][q], part[2][q]);
             }
@@ -551,7 +612,9 @@ __global__ void __launch_bounds__(512) gcn_relu_forward_kernel(ReluFwdArgs a) {
         }
         top = fmaxf(top, __shfl_xor(top, 16));
         top = fmaxf(top, __shfl_xor(top, 32));
-        redoAll |= __ballot(top != 0.0f && top < kSplitTiny) != 0;
+        const std::uint64_t tiny = __ballot(low < kSplitExactBits);
+        smallW |= tiny != 0;
+        if (lk == 0) colTop[32 * wave + 16 * u + li] = ((tiny >> li) & 0x0001000100010001ull) != 0 ? -top : top;
     }
     float w2[2][4][CT];
 #pragma unroll
@@ -564,6 +627,9 @@ __global__ void __launch_bounds__(512) gcn_relu_forward_kernel(ReluFwdArgs a) {
                 w2[u][v][j] = n < a.Hd && static_cast<std::uint32_t>(j) < a.C
                                   ? a.W2[static_cast<std::uint64_t>(n) * a.C + j] : 0.0f;
         }
+
+    if (threadIdx.x < 2) small[threadIdx.x] = 0;
+    const bool colsToo = __syncthreads_or(smallW) != 0;  // any wave's
 
     // This thread's inputs (clamped loads, zeros past F when staged).
     const std::uint32_t kg = threadIdx.x & 15u, row0 = threadIdx.x >> 4;
@@ -586,17 +652,16 @@ __global__ void __launch_bounds__(512) gcn_relu_forward_kernel(ReluFwdArgs a) {
             }
         }
     };
-    auto stage = [&](unsigned buf) {
+    auto stage = [&](std::uint32_t step, unsigned buf) {
         uint4* const to = parts + buf * kStage;
 #pragma unroll
         for (std::uint32_t h = 0; h < 2; ++h) {
-            std::uint32_t hi[4], mid[4], lo[4];
-            float top = 0.0f;
+            std::uint32_t hi[4], mid[4], lo[4], low = ~0u;
 #pragma unroll
             for (std::uint32_t q = 0; q < 4; ++q) {
                 const float p = 8 * kg + 2 * q < a.F ? x[h][2 * q] : 0.0f;
                 const float r = 8 * kg + 2 * q + 1 < a.F ? x[h][2 * q + 1] : 0.0f;
-                top = fmaxf(top, fmaxf(fabsf(p), fabsf(r)));
+                low = min(low, min(smallness(p), smallness(r)));
                 split3(p, r, hi[q], mid[q], lo[q]);
             }
             if (mine) {
@@ -605,14 +670,22 @@ __global__ void __launch_bounds__(512) gcn_relu_forward_kernel(ReluFwdArgs a) {
                 at[kPart] = make_uint4(mid[0], mid[1], mid[2], mid[3]);
                 at[2 * kPart] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
             }
+            const std::uint64_t tiny = __ballot(low < kSplitExactBits);
+            if (tiny) small[buf] = step + 1;
+            float top = 0.0f;
+            if (tiny || colsToo) {
 #pragma unroll
-            for (unsigned d = 1; d < 16; d *= 2) top = fmaxf(top, __shfl_xor(top, d));
-            if (top != 0.0f && top < kSplitTiny) small[buf] = 1;
+                for (std::uint32_t e = 0; e < 8; ++e)
+                    if (8 * kg + e < a.F) top = fmaxf(top, fabsf(x[h][e]));
+#pragma unroll
+                for (unsigned d = 1; d < 16; d *= 2) top = fmaxf(top, __shfl_xor(top, d));
+            }
+            if (kg == 0) rowTop[buf][row0 + 32 * h] = (tiny >> (lane & 48u) & 0xFFFFull) != 0 ? -top : top;
         }
     };
     auto multiply = [&](std::uint32_t step, unsigned buf) {
         const uint4* const from = parts + buf * kStage;
-        const bool redoStep = redoAll || small[buf] != 0;
+        const bool look = smallW || small[buf] == step + 1;
 #pragma unroll
         for (std::uint32_t rt = 0; rt < 4; ++rt) {
             f32x4 acc[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
@@ -631,11 +704,21 @@ __global__ void __launch_bounds__(512) gcn_relu_forward_kernel(ReluFwdArgs a) {
 #pragma unroll
                     for (int u = 0; u < 2; ++u)
                         acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][ks][kW[s]], b[ks][kX[s]], acc[u], 0, 0, 0);
-            bool redo = redoStep;
+            bool redo = false;
 #pragma unroll
             for (int u = 0; u < 2; ++u)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) redo |= !(fabsf(acc[u][v]) <= 0x1.fffffep127f);
+            if (look) {
+                const float loss = split_loss(a.F), r = rowTop[buf][16 * rt + li];
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const float c = colTop[32 * wave + 16 * u + 4 * lk + v];
+                        redo |= !(fabsf(acc[u][v]) >= loss * ((r < 0.0f ? fabsf(c) : 0.0f) + (c < 0.0f ? fabsf(r) : 0.0f)));
+                    }
+            }
             const std::uint64_t row = static_cast<std::uint64_t>(step) * 64 + 16 * rt + li;
             if (__ballot(redo)) {
 #pragma unroll
@@ -686,16 +769,14 @@ __global__ void __launch_bounds__(512) gcn_relu_forward_kernel(ReluFwdArgs a) {
     };
 
     std::uint32_t step = blockIdx.x;
-    if (threadIdx.x < 2) small[threadIdx.x] = 0;
-    __syncthreads();
     load(step);
-    stage(0);
+    stage(step, 0);
     load(step + gridDim.x);  // past the last: the last row again
     __syncthreads();
     for (unsigned buf = 0; step < a.steps; step += gridDim.x, buf ^= 1u) {
         if (!first) multiply(step, buf);
         __builtin_amdgcn_sched_barrier(0);
-        stage(buf ^ 1u);
+        stage(step + gridDim.x, buf ^ 1u);
         load(step + 2 * gridDim.x);
         __builtin_amdgcn_sched_barrier(0);
         if (first) multiply(step, buf);

@@ -88,6 +88,57 @@ def test_values_past_a_split(gpu, kind):
     assert ((got - want)[ok].abs() <= BOUND * mag[ok] + K * 2.0**-126).all()
 
 
+def _hide(A, B, k, e, step):
+    """Row k of A becomes 2^e and a fraction, and in every `step`th column of B
+    only row k is left, of 2^100: there the small elements are the result,
+    though their columns hold ordinary ones too."""
+    A[k] = (1 + torch.rand(A.shape[1], generator=torch.Generator().manual_seed(1))) * 2.0**e
+    B[:, ::step] = 0.0
+    B[k, ::step] = 2.0**100 * (1 + B[k + 1, 1].abs())
+
+
+@pytest.mark.parametrize("small", ["A", "B"])
+@pytest.mark.parametrize("e", [-109, -112, -120, -133, -140])
+def test_small_elements_among_ordinary_ones(gpu, e, small):
+    from tcc_amd import swtcf
+
+    for K, M, N in ((40, 64, 257), (70, 100, 256), (1100, 300, 300)):
+        g = torch.Generator().manual_seed(K)
+        A, B = torch.randn(K, M, generator=g), torch.randn(K, N, generator=g)
+        _hide(*((A, B) if small == "A" else (B, A)), K // 2, e, 7)
+        _check(swtcf.dense_tn(A.cuda(), B.cuda()), A, B)
+
+
+@pytest.mark.parametrize("e", [-109, -115, -140])
+def test_relu_gradient_small_elements(gpu, e):
+    """One row of dOut1, and one of AX, too small to split."""
+    from tcc_amd import swtcf
+
+    K, F, Hd, C = 300, 113, 258, 2
+    for small in ("AX", "dOut1"):
+        g = torch.Generator().manual_seed(3)
+        AX, G, W2 = (torch.randn(s, generator=g) for s in ((K, F), (K, C), (Hd, C)))
+        H = torch.rand(K, Hd, generator=g) + 0.5
+        if small == "AX":
+            AX[9] = (1 + torch.rand(F, generator=g)) * 2.0**e
+            G[9] = 2.0**100
+            H[:, ::5] = 0.0  # in these columns of dOut1 only row 9 is left
+            H[9] = 1.0
+        else:
+            G[9] = (1 + torch.rand(C, generator=g)) * 2.0**e
+            W2 = W2.abs()
+            AX[:, ::5] = 0.0
+            AX[9, ::5] = 2.0**100
+        dW1, _ = swtcf.gcn_relu_grad(AX.cuda(), H.cuda(), G.cuda(), W2.cuda())
+        # the kernel's own dOut1, a sum of two rounded products
+        d = torch.where(H > 0, G.double() @ W2.double().t(), torch.zeros((), dtype=torch.float64))
+        dmag = torch.where(H > 0, G.double().abs() @ W2.double().abs().t(), torch.zeros((), dtype=torch.float64))
+        want, mag = AX.double().t() @ d, AX.double().abs().t() @ dmag
+        # below 2^-126 dOut1 is rounded to multiples of 2^-149
+        sub = AX.double().abs().sum(0).unsqueeze(1) * 2.0**-148
+        assert ((dW1.double().cpu() - want).abs() <= 2 * BOUND * mag + sub).all(), small
+
+
 @pytest.mark.parametrize("C", [1, 2, 3, 8])
 @pytest.mark.parametrize("K", [33, 1100])
 def test_relu_gradient_edges(gpu, K, C):
@@ -148,3 +199,21 @@ def test_relu_forward_edges(gpu, K, F, Hd, C):
         ok = torch.isfinite(xw)
         assert torch.equal(torch.isfinite(XW), ok)
         assert ((XW.double() - xw)[ok].abs() <= Hd * 2.0**-23 * xmag[ok] + Hd * 2.0**-126).all()
+
+
+@pytest.mark.parametrize("small", ["AX", "W1"])
+@pytest.mark.parametrize("e", [-109, -112, -120, -133, -140])
+@pytest.mark.parametrize("K,F,Hd", [(5, 20, 33), (700, 100, 256), (20_000, 128, 100)])
+def test_relu_forward_small_elements(gpu, K, F, Hd, e, small):
+    from tcc_amd import swtcf
+
+    g = torch.Generator().manual_seed(K)
+    AX, W1 = torch.randn(K, F, generator=g), torch.rand(F, Hd, generator=g) + 0.5
+    if small == "AX":
+        _hide(AX.t(), W1, F // 2, e, 7)
+    else:
+        _hide(W1, AX.t(), F // 2, e, 7)
+    H, _ = swtcf.gcn_relu_forward(AX.cuda(), W1.cuda(), torch.ones(Hd, 1).cuda())
+    want = (AX.double() @ W1.double()).clamp_min(0)
+    mag = AX.double().abs() @ W1.double().abs()
+    assert ((H.double().cpu() - want).abs() <= BOUND * mag).all()
