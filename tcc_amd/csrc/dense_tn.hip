@@ -184,6 +184,14 @@ __device__ __forceinline__ float split_loss(std::uint32_t rows) { return 0x1p-10
 __device__ __forceinline__ std::uint32_t smallness(float x) { return (__float_as_uint(x) << 1) - 1u; }
 constexpr std::uint32_t kSplitExactBits = ((127u - 110u) << 24) - 1u;  // of 2^-110
 
+// Sums of fewer products are left to the fp32 products.  The six part products
+// give a single product to 2^-23 (the three left out and the MFMA's truncation),
+// fp32 MFMA to 2^-24; sums of 1, 2, 3, 4 normal products are off by 3.5, 3.3,
+// 3.3, 3.2e-8 of the result, in fp32 by 2.5, 3.1, 3.6, 4.0e-8, and the longer
+// the sum, the further the part products are ahead (100 products: 5.6e-8
+// against 1.8e-7).
+constexpr std::uint32_t kSplitMinTerms = 4;
+
 // Wide outputs.  fp32 MFMA runs at 1/16 of the bf16 rate, and the 100 x 256
 // and 602 x 256 products over node rows were bound by it (110 TFLOP/s).  Here
 // each operand is split into three bf16 parts (split3) and a product is the
@@ -404,7 +412,7 @@ __global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
     const auto ncol = [&](int u) { return n0 + 2 * (32 * wn + 16 * (u % 2) + li) + u / 2; };
     const int tiles = wm == 0 ? TW : TM / 2;
 
-    bool redo = false;
+    bool redo = k1 - k0 < kSplitMinTerms;
     const bool tinyA = lowA < kSplitExactBits, tinyB[2] = {lowB[0] < kSplitExactBits, lowB[1] < kSplitExactBits};
     if (__syncthreads_or(tinyA || tinyB[0] || tinyB[1])) {
         // the columns' maxima and losses, of the four waves' rows: [4][BM] and
@@ -704,7 +712,7 @@ __global__ void __launch_bounds__(512) gcn_relu_forward_kernel(ReluFwdArgs a) {
 #pragma unroll
                     for (int u = 0; u < 2; ++u)
                         acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][ks][kW[s]], b[ks][kX[s]], acc[u], 0, 0, 0);
-            bool redo = false;
+            bool redo = a.F < kSplitMinTerms;
 #pragma unroll
             for (int u = 0; u < 2; ++u)
 #pragma unroll

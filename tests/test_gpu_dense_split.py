@@ -217,3 +217,19 @@ def test_relu_forward_small_elements(gpu, K, F, Hd, e, small):
     want = (AX.double() @ W1.double()).clamp_min(0)
     mag = AX.double().abs() @ W1.double().abs()
     assert ((H.double().cpu() - want).abs() <= BOUND * mag).all()
+
+
+@pytest.mark.parametrize("terms", [1, 2, 3])
+def test_few_terms_are_fp32_products(gpu, terms):
+    """Sums of one to three products are as fp32 MFMA gives them: exact
+    products, each addition rounded to nearest."""
+    from tcc_amd import swtcf
+
+    g = torch.Generator(device="cuda").manual_seed(terms)
+    A, B = torch.randn(terms, 130, generator=g, device="cuda"), torch.randn(terms, 257, generator=g, device="cuda")
+    C = swtcf.dense_tn(A, B).double()
+    assert ((C - A.double().t() @ B.double()).abs() <= terms * 2.0**-24 * (A.double().abs().t() @ B.double().abs())).all()
+    AX, W1 = torch.randn(3000, terms, generator=g, device="cuda"), torch.randn(terms, 200, generator=g, device="cuda")
+    H, _ = swtcf.gcn_relu_forward(AX, W1, torch.randn(200, 2, generator=g, device="cuda"))
+    want, mag = (AX.double() @ W1.double()).clamp_min(0), AX.double().abs() @ W1.double().abs()
+    assert ((H.double() - want).abs() <= terms * 2.0**-24 * mag).all()
