@@ -20,7 +20,9 @@
 //      takes a workgroup, which sets its masks' bits in an LDS byte per b
 //      (128K of them at a time) and reads them off in order, with no sort
 //      however long the window is.  For BCSC each list is then reordered by
-//      degree, the mask's population.
+//      degree, the mask's population.  Where one window would keep its
+//      workgroup longer than a sort of all edges takes, they are sorted and
+//      the lists read off an edge a thread.
 //   3. The lists' lengths give the block offsets (one scan), and one pass
 //      over the edges' positions writes blocks, bitmaps and value offsets.
 // The host waits once (twice where the order check decides the route), to
@@ -77,7 +79,7 @@ struct Edge {
 };
 
 // Flag words (device): what went wrong or was found.
-constexpr unsigned kFlagRange = 0, kFlagUngrouped = 1, kFlagDuplicate = 2, kNumMid = 3, kNumBig = 4;
+constexpr unsigned kFlagRange = 0, kFlagUngrouped = 1, kFlagDuplicate = 2, kNumMid = 3, kNumBig = 4, kFlagTooLong = 5;
 
 // Edge i; indices out of range become (0, 0) and set `bad`.
 __device__ __forceinline__ Edge coo_edge(const Coo& c, std::uint32_t i, bool& bad) {
@@ -221,6 +223,7 @@ struct Lists {
     std::uint32_t* sPlace;  // [E] (BCSC with values, else null)
     std::uint32_t* mid;     // windows of at most kMid edges for the second pass, flags[kNumMid] of them
     std::uint32_t* big;     // longer ones, flags[kNumBig] of them
+    std::uint32_t longest;  // edges of a window that one workgroup may take
     std::uint32_t* flags;
 };
 
@@ -422,8 +425,12 @@ __global__ void __launch_bounds__(kListWaves * kWave) short_lists_kernel(Coo c, 
         std::uint32_t before = 0;
         for (unsigned v = 0; v < wave; ++v) before += kind[v] == kind[wave];
         if (__lane_id() == 0) {
-            if (n <= kMid) L.mid[listAt[0] + before] = w;
-            else L.big[listAt[1] + before] = w;
+            if (n <= kMid) {
+                L.mid[listAt[0] + before] = w;
+            } else {
+                L.big[listAt[1] + before] = w;
+                if (n > L.longest) L.flags[kFlagTooLong] = 1;
+            }
         }
         return;
     }
@@ -467,6 +474,18 @@ constexpr unsigned kLongWaves = kLongThreads / kWave;
 constexpr unsigned kUseWords = kSlice / 32;
 constexpr unsigned kLongSteps = kUseWords / kLongThreads;  // 64 words a wave and step
 
+// A workgroup goes through a long window once for each slice (0.13 to 0.7 ns an
+// edge and slice) and no other can help it.  Where that is more for the longest
+// window than sorting the whole COO takes (0.1 ms and 0.06 ns an edge; BCSC
+// about twice that), the lists are made of the sorted COO instead.  Builds in
+// ms, a workgroup a window : all sorted: 8 x 1M with 2M edges BCSR 12.0 : 0.19,
+// 64 x 4M with 8M edges 21.4 : 0.53; 2M x 64 with 8M edges BCSC 4.7 : 0.71; a
+// 1M-node graph of 8M edges with one row and one column joined to all BCSR
+// 8.1 : 0.90, BCSC 5.0 : 1.48 (0.45 and 0.64 without them).
+inline std::uint32_t longest_window(std::uint64_t E, std::uint32_t numB) {
+    return static_cast<std::uint32_t>(((1ull << 18) + E / 4) / ((numB - 1) / kSlice + 1));
+}
+
 template <typename K>
 constexpr unsigned other_lists_lds() {
     const unsigned mid = kLongWaves * (staged(kMid) * sizeof(K) + kMid), big = kSlice + 4 * kUseWords;
@@ -483,6 +502,7 @@ __global__ void __launch_bounds__(kLongThreads) other_lists_kernel(Coo c, const 
     const unsigned lane = __lane_id(), wave = threadIdx.x / kWave;
     const std::uint64_t lt = lanemask_lt();
     const std::uint32_t numBig = L.flags[kNumBig], numMid = L.flags[kNumMid];
+    if (L.flags[kFlagTooLong]) return;
     std::uint32_t* const bytes = lds;              // [kSlice / 4] masks
     std::uint32_t* const use = lds + kSlice / 4;   // [kUseWords]
     if (blockIdx.x < numBig) {
@@ -657,6 +677,98 @@ __global__ void __launch_bounds__(kLongThreads) other_lists_kernel(Coo c, const 
     }
 }
 
+// ---------------------------------------------------------------- lists of a sorted COO
+
+// 1 where a list entry starts: the first edge of its (window, b).
+__global__ void __launch_bounds__(kThreads) entry_heads_kernel(const std::uint64_t* __restrict__ keys, std::uint32_t E,
+                                                              std::uint32_t* __restrict__ heads) {
+    const std::uint64_t i = static_cast<std::uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
+    if (i < E) heads[i] = i == 0 || (keys[i] >> 3) != (keys[i - 1] >> 3);
+}
+
+// The lists of the edges in (window, b, a % 8) order, an edge a thread (for
+// BCSC in that order still); pos: the entries that start before each edge.
+template <bool DEGREE>
+__global__ void __launch_bounds__(kThreads) sorted_lists_kernel(const std::uint64_t* __restrict__ keys,
+                                                               const std::uint32_t* __restrict__ pos, std::uint32_t E,
+                                                               unsigned bBits, Lists L) {
+    const std::uint64_t i = static_cast<std::uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
+    bool dup = false;
+    if (i < E) {
+        const std::uint64_t k = keys[i], prev = i > 0 ? keys[i - 1] : ~k;
+        const Edge e = unpack_edge(k, bBits);
+        const std::uint32_t begin = L.winStart[e.w], first = pos[begin];
+        const bool head = (k >> 3) != (prev >> 3);
+        dup = k == prev;
+        if (head) {
+            std::uint32_t mask = 1u << e.lo;
+            for (unsigned q = 1; q < 8 && i + q < E; ++q) {
+                const std::uint64_t x = keys[i + q];
+                if ((x >> 3) != (k >> 3)) break;
+                mask |= 1u << static_cast<unsigned>(x & 7u);
+            }
+            const std::uint32_t at = begin + (pos[i] - first);
+            if constexpr (DEGREE) {
+                L.sB[at] = e.b;
+                L.sMask[at] = static_cast<std::uint8_t>(mask);
+            } else {
+                L.b[at] = e.b;
+                L.mask[at] = static_cast<std::uint8_t>(mask);
+                L.before[at] = static_cast<std::uint32_t>(i) - begin;
+            }
+        }
+        if (i + 1 == L.winStart[e.w + 1]) L.length[e.w] = pos[i] + (head ? 1u : 0u) - first;
+    }
+    raise_flag(&L.flags[kFlagDuplicate], dup);
+}
+
+// BCSC: list position i's element for the order by degree, (window, 8 - degree,
+// i); the positions past a list's end stay behind its entries as degree 1.
+__global__ void __launch_bounds__(kThreads) degree_elems_kernel(const std::uint64_t* __restrict__ keys, std::uint32_t E,
+                                                               unsigned bBits, Lists L,
+                                                               std::uint64_t* __restrict__ elems) {
+    const std::uint64_t i = static_cast<std::uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
+    if (i >= E) return;
+    const std::uint32_t w = unpack_edge(keys[i], bBits).w;
+    const bool entry = static_cast<std::uint32_t>(i) - L.winStart[w] < L.length[w];
+    const unsigned d = entry ? 8u - static_cast<unsigned>(__popc(L.sMask[i])) : 7u;
+    elems[i] = (((static_cast<std::uint64_t>(w) << 3) | d) << 32) | i;
+}
+
+// The entry at each place of that order: its degree (0 past a list's end), and
+// after their scan, which counts a window's edges up to its end, the list.
+struct ByDegree {
+    std::uint32_t w, i, degree;
+};
+
+__device__ __forceinline__ ByDegree by_degree(std::uint64_t elem, const Lists& L) {
+    ByDegree r;
+    r.w = static_cast<std::uint32_t>(elem >> 35);
+    r.i = static_cast<std::uint32_t>(elem);
+    r.degree = r.i - L.winStart[r.w] < L.length[r.w] ? 8u - (static_cast<std::uint32_t>(elem >> 32) & 7u) : 0u;
+    return r;
+}
+
+__global__ void __launch_bounds__(kThreads) degrees_kernel(const std::uint64_t* __restrict__ elems, std::uint32_t E,
+                                                          Lists L, std::uint32_t* __restrict__ degree) {
+    const std::uint64_t q = static_cast<std::uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
+    if (q < E) degree[q] = by_degree(elems[q], L).degree;
+}
+
+__global__ void __launch_bounds__(kThreads) degree_lists_kernel(const std::uint64_t* __restrict__ elems,
+                                                               const std::uint32_t* __restrict__ edges, std::uint32_t E,
+                                                               Lists L) {
+    const std::uint64_t q = static_cast<std::uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
+    if (q >= E) return;
+    const ByDegree r = by_degree(elems[q], L);
+    if (r.degree == 0) return;
+    const std::uint32_t begin = L.winStart[r.w];
+    L.b[q] = L.sB[r.i];
+    L.mask[q] = L.sMask[r.i];
+    L.before[q] = edges[q] - begin;
+    if (L.sPlace) L.sPlace[r.i] = static_cast<std::uint32_t>(q) - begin;
+}
+
 // ---------------------------------------------------------------- blocks
 
 __global__ void blocks_per_window_kernel(const std::uint32_t* __restrict__ length, std::uint32_t n,
@@ -712,6 +824,16 @@ __device__ __forceinline__ std::uint64_t spread8(std::uint64_t x) {
     return (x | (x << 7)) & 0x0101010101010101ull;
 }
 
+// The block count and the flags, for the host.
+__device__ __forceinline__ void tell_host(const Lists& L, const std::uint32_t* off, std::uint32_t* mail) {
+    mail[0] = off[L.RW];
+    mail[1] = L.flags[kFlagRange];
+    mail[2] = L.flags[kFlagDuplicate];
+    mail[3] = L.flags[kFlagTooLong];
+}
+
+__global__ void tell_host_kernel(Lists L, const std::uint32_t* off, std::uint32_t* mail) { tell_host(L, off, mail); }
+
 // Entry i (at its list's position) goes to its block; the first entry of a
 // block also gathers the block's bitmap and pads it.  Thread 0 closes the
 // value offsets and tells the host the block count and the flags.
@@ -723,11 +845,8 @@ __global__ void __launch_bounds__(kThreads) emit_blocks_kernel(Coo c, const std:
                                                               std::uint64_t* __restrict__ bits, std::uint32_t* mail) {
     const std::uint64_t i64 = static_cast<std::uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (i64 == 0) {
-        const std::uint32_t B = off[L.RW];
-        tcOffset[B] = c.E;
-        mail[0] = B;
-        mail[1] = L.flags[kFlagRange];
-        mail[2] = L.flags[kFlagDuplicate];
+        tcOffset[off[L.RW]] = c.E;
+        tell_host(L, off, mail);
     }
     if (i64 >= c.E) return;
     const std::uint32_t i = static_cast<std::uint32_t>(i64);
@@ -868,7 +987,7 @@ struct BlockArrays {
     }
 };
 
-enum class Built { Ok, Range, Duplicate };
+enum class Built { Ok, Range, Duplicate, TooLong };
 
 // Builds the arrays of the COO over RW windows (E > 0).  A BCSR without
 // phases checks whether the COO is grouped by window already; the source
@@ -918,7 +1037,8 @@ int build_blocks(Coo c, std::uint32_t RW, const float* val, BlockArrays& out, st
         L.flags = flags;
         return off;
     };
-    Scratch scratch, partition;
+    L.longest = longest_window(E, c.numB);
+    Scratch scratch, partition, byDegree;
     TCC_HIP_CHECK(scratch.take(carve(nullptr, false), st));
     carve(scratch.data(), false);
     // flags and list lengths lie together
@@ -936,10 +1056,15 @@ int build_blocks(Coo c, std::uint32_t RW, const float* val, BlockArrays& out, st
         keys = scratch.read()[kFlagUngrouped] != 0;
     }
     const std::uint64_t* grouped = nullptr;
-    if (keys) {
-        // stable passes over the window's bits, the first from the COO
+    auto take_partition = [&]() -> int {
+        if (partition.data()) return TCC_OK;
         TCC_HIP_CHECK(partition.take(carve(nullptr, true), st));
         carve(partition.data(), true);
+        return TCC_OK;
+    };
+    if (keys) {
+        // stable passes over the window's bits, the first from the COO
+        if (const int rc = take_partition()) return rc;
         std::uint64_t* sorted = nullptr;
         TCC_HIP_CHECK(partition_by(CooLoad{c, flags}, keysA, keysB, E, c.bBits + 3, wBits, hist, total, &sorted, st));
         grouped = sorted;
@@ -958,7 +1083,7 @@ int build_blocks(Coo c, std::uint32_t RW, const float* val, BlockArrays& out, st
                 hipLaunchKernelGGL((other_lists_kernel<KEYS, BCSC, K>), otherGrid, dim3(kLongThreads),
                                    other_lists_lds<K>(), st, c, grouped, L);
         };
-        if (c.bBits <= 29) sorts(std::uint32_t{});  // b << 3 | a % 8, below the ~0 of no edge
+        if (c.bBits <= 29) sorts(std::uint32_t{});  // b << 3 | a % 8, at most the ~0 of no edge, which sorts last
         else sorts(std::uint64_t{});
     };
     auto emit = [&](auto fromKeys) {
@@ -976,6 +1101,7 @@ int build_blocks(Coo c, std::uint32_t RW, const float* val, BlockArrays& out, st
     // ceil(length / 8) summed over at most min(RW, E) windows with edges
     const std::uint64_t maxB = std::min<std::uint64_t>(E, (E + 7 * std::min<std::uint64_t>(RW, E)) / 8);
     TCC_HIP_CHECK(out.allocate(RW, maxB, E, val != nullptr));
+    // the blocks of the lists; mail holds their count and the flags afterwards
     auto finish = [&]() -> int {
         if (RW <= kOneScan) {
             hipLaunchKernelGGL(window_blocks_kernel, dim3(1), dim3(1024), 0, st, L.length, RW, out.off);
@@ -997,14 +1123,52 @@ int build_blocks(Coo c, std::uint32_t RW, const float* val, BlockArrays& out, st
                                out.bits, val, out.data);
             TCC_LAUNCH_CHECK();
         }
-        TCC_HIP_CHECK(scratch.finish());
-        if (keys) TCC_HIP_CHECK(partition.finish());
+        TCC_HIP_CHECK(scratch.wait());
+        B = scratch.read()[0];
+        what = scratch.read()[1] ? Built::Range : scratch.read()[2] ? Built::Duplicate
+               : scratch.read()[3] ? Built::TooLong : Built::Ok;
         return TCC_OK;
     };
-    const int rc = finish();
-    if (rc == TCC_OK) {
-        B = scratch.read()[0];
-        what = scratch.read()[1] ? Built::Range : scratch.read()[2] ? Built::Duplicate : Built::Ok;
+    // the lists again, of the whole COO sorted
+    auto sort_all = [&]() -> int {
+        if (const int rc = take_partition()) return rc;
+        std::uint64_t* sorted = nullptr;
+        TCC_HIP_CHECK(partition_by(CooLoad{c, flags}, keysA, keysB, E, 0, c.bBits + 3 + wBits, hist, total, &sorted, st));
+        grouped = sorted;
+        keys = true;
+        // the entries before each edge, over the elements that the last pass read
+        auto* pos = reinterpret_cast<std::uint32_t*>(sorted == keysA ? keysB : keysA);
+        hipLaunchKernelGGL(entry_heads_kernel, perEdge, dim3(kThreads), 0, st, grouped, c.E, pos);
+        TCC_LAUNCH_CHECK();
+        TCC_HIP_CHECK(exclusive_scan(pos, pos, E, nullptr, pos + E, st));
+        TCC_HIP_CHECK(fill<std::uint32_t>(flags + kFlagTooLong, 1, 0u, st));
+        hipLaunchKernelGGL(sorted_lists_kernel<BCSC>, perEdge, dim3(kThreads), 0, st, grouped, pos, c.E, c.bBits, L);
+        TCC_LAUNCH_CHECK();
+        if constexpr (BCSC) {
+            const std::size_t bytes = align_up(8 * E);
+            TCC_HIP_CHECK(byDegree.take(2 * bytes, st));
+            auto* elemsA = reinterpret_cast<std::uint64_t*>(byDegree.data());
+            auto* elemsB = reinterpret_cast<std::uint64_t*>(byDegree.data() + bytes);
+            hipLaunchKernelGGL(degree_elems_kernel, perEdge, dim3(kThreads), 0, st, grouped, c.E, c.bBits, L, elemsB);
+            TCC_LAUNCH_CHECK();
+            TCC_HIP_CHECK(partition_by(KeyLoad{elemsB, E}, elemsA, elemsB, E, 32, 3 + wBits, hist, total, &sorted, st));
+            hipLaunchKernelGGL(degrees_kernel, perEdge, dim3(kThreads), 0, st, sorted, c.E, L, pos);
+            TCC_LAUNCH_CHECK();
+            TCC_HIP_CHECK(exclusive_scan(pos, pos, E, nullptr, pos + E, st));
+            hipLaunchKernelGGL(degree_lists_kernel, perEdge, dim3(kThreads), 0, st, sorted, pos, c.E, L);
+            TCC_LAUNCH_CHECK();
+        }
+        return TCC_OK;
+    };
+    int rc = finish();
+    if (rc == TCC_OK && what == Built::TooLong) {
+        rc = sort_all();
+        if (rc == TCC_OK) rc = finish();
+    }
+    if (rc == TCC_OK) {  // all work waited for, and none queued after it
+        scratch.idle();
+        partition.idle();
+        byDegree.idle();
     }
     if (rc != TCC_OK || what != Built::Ok) {
         (void)hipStreamSynchronize(st);

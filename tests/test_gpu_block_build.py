@@ -1,8 +1,8 @@
 """BCSR and BCSC construction where its routes meet: grouped and shuffled
 COOs, runs of empty windows, windows around the sizes that one wave sorts
-(64 to 1024 edges), long windows over one and over several 128K slices, keys
-of more than 32 bits, every degree, phases, single edges; bit for bit against
-the oracle."""
+(64 to 1024 edges), long windows over one and over several 128K slices,
+windows too long for one workgroup, keys of more than 32 bits, every degree,
+phases, single edges; bit for bit against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -55,6 +55,13 @@ def _case(name, rng):
         src = src + 150_000 * (src % 6)
         o = np.lexsort((src, dst))
         return 900_000, nc, np.where(dst == 12, 899_999, dst).astype(np.uint32)[o], src[o]
+    if name in ("hub_row", "hub_column"):  # 10 slices of a window with 480K edges: the whole COO is sorted
+        spec = [(0, 30), (5, 400_000), (6, 80_000), (9, 1500), (30, 4)]
+        dst, src = _rows(spec, 1_200_000, rng)
+        if name == "hub_row":
+            return 64, 1_200_000, dst, src
+        o = np.lexsort((dst, src))
+        return 1_200_000, 64, src[o], dst[o]
     if name == "wide":  # keys of more than 32 bits
         nc = 600_000_000
         spec = [(0, 40), (8, 200), (17, 700), (25, 1000), (33, 1500), (41, 2100)]
@@ -82,7 +89,7 @@ def _same(got, want, values):
 
 @pytest.mark.parametrize("values", [False, True])
 @pytest.mark.parametrize("name", ["one_edge", "last_corner", "empty_runs", "sort_sizes", "long", "slices", "wide",
-                                  "dense", "sparse"])
+                                  "hub_row", "hub_column", "dense", "sparse"])
 def test_block_build_bit_exact(gpu, oracle, name, values):
     from tcc_amd import swtcf
 
@@ -106,7 +113,7 @@ def test_block_build_bit_exact(gpu, oracle, name, values):
 
 
 @pytest.mark.parametrize("phases", [2, 3, 7])
-@pytest.mark.parametrize("name", ["sort_sizes", "long", "dense", "sparse"])
+@pytest.mark.parametrize("name", ["sort_sizes", "long", "hub_row", "dense", "sparse"])
 def test_phased_build_is_the_slices_stacked(gpu, oracle, name, phases):
     from tcc_amd import swtcf
 
@@ -123,15 +130,15 @@ def test_phased_build_is_the_slices_stacked(gpu, oracle, name, phases):
         assert np.array_equal(got[k], want[k]), k
 
 
-@pytest.mark.parametrize("columns", [5000, 200_000])
-def test_duplicates_and_ranges(gpu, oracle, columns):
+@pytest.mark.parametrize("columns,hub", [(5000, 2500), (200_000, 2500), (1_200_000, 480_000)])
+def test_duplicates_and_ranges(gpu, oracle, columns, hub):
     """A repeated edge is refused for a BCSR wherever its window is built; a
     BCSC takes it (up to degree 8) as another degree, its bit set once."""
     from tcc_amd import _lib, swtcf
 
     rng = np.random.default_rng(9)
-    dst, src = _rows([(3, 40), (17, 2500), (18, 30), (31, 2)], columns, rng)
-    for at in (0, 41, 2560):  # in a short window, a long one and the last
+    dst, src = _rows([(3, 40), (17, hub), (18, 30), (31, 2)], columns, rng)
+    for at in (0, 41, hub + 60):  # in a short window, a long one and the last
         d = np.insert(dst, at, dst[at])
         s = np.insert(src, at, src[at])
         for p in (np.arange(d.size), rng.permutation(d.size)):
@@ -194,3 +201,39 @@ def test_builds_from_several_threads_and_streams(gpu, oracle):
     for t in threads:
         t.join()
     assert not errors, errors
+
+
+def test_one_row_joined_to_every_column(gpu):
+    """A window is no longer one workgroup's work however long it is: 2M edges
+    of one row or column, and 2M elsewhere, take within a few times what 4M
+    spread edges take (from 20 times it on, were that window built by one
+    workgroup)."""
+    import time
+
+    from tcc_amd import swtcf
+
+    n = 2_000_000
+    g = torch.Generator(device="cuda").manual_seed(1)
+
+    def seconds(build, hub, swap):
+        r = torch.randint(0, n, (2 * n,), generator=g, device="cuda")
+        if hub:
+            r[:n] = n // 2
+        c = torch.cat([torch.arange(n, device="cuda"), torch.randint(0, n, (n,), generator=g, device="cuda")])
+        key = torch.unique(r * n + c)
+        r, c = (key // n).int(), (key % n).int()
+        if swap:
+            r, c = c, r
+        best = float("inf")
+        for _ in range(4):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            build(r, c, None, n, n)
+            torch.cuda.synchronize()
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    for build, swap in ((swtcf.coo_to_bcsr, False), (swtcf.coo_to_bcsc, True)):
+        spread, hub = seconds(build, False, swap), seconds(build, True, swap)
+        print(f"spread {spread * 1e3:.2f} ms, with a hub {hub * 1e3:.2f} ms")
+        assert hub < 8 * spread
