@@ -527,6 +527,10 @@ __global__ void __launch_bounds__(kRawWaves * kWave) step_raw_kernel(const std::
                 dup |= (atomicOr(&mine[byte / 4], bit) & bit) != 0;
             }
             if (__ballot(in) != ~0ull) break;
+            if (e - e0 >= 512 * G) {  // more entries than places
+                dup = true;
+                break;
+            }
         }
         __builtin_amdgcn_wave_barrier();
         std::uint32_t* out = raw + static_cast<std::uint64_t>(s) * words;
@@ -1802,6 +1806,9 @@ int build_hybrid(const HybridParams& P, tcc_hybrid* out, void* stream) {
     const unsigned tileBits = std::max(1u, rank_bits(static_cast<std::uint64_t>(NG) * CB * G));
     TCC_REQUIRE(tileBits + 8 <= 64, TCC_ERR_UNSUPPORTED, "hybrid: tile key exceeds 64 bits");
     const unsigned stepBits = rank_bits(static_cast<std::uint64_t>(NG) * colSteps);  // binary: no more bits than a tile key
+    // A step has 512 G places: one that is over-full holds a duplicate, whether
+    // it is stored or left to the remainder, and the searches below may stop.
+    const std::uint32_t minStepNnz = std::min(P.minStepNnz, 512 * G + 1);
     const unsigned stepTileCount = static_cast<unsigned>((En + kStepTile - 1) / kStepTile);
     const std::uint64_t tempElems = std::max({radix_temp_elems(Vn), scan_temp_elems(En + 1),
                                               scan_temp_elems(static_cast<std::uint64_t>(NG) + 1)});
@@ -1823,7 +1830,7 @@ int build_hybrid(const HybridParams& P, tcc_hybrid* out, void* stream) {
         keysB = reinterpret_cast<std::uint64_t*>(take(8 * Vn));
         if (binary) {
             stepCounts = reinterpret_cast<std::uint32_t*>(take(8ull * stepTileCount));
-            stepStart = reinterpret_cast<std::uint32_t*>(take(4 * (En / P.minStepNnz + 1)));
+            stepStart = reinterpret_cast<std::uint32_t*>(take(4 * (En / minStepNnz + 1)));
         } else {
             permA = reinterpret_cast<std::uint32_t*>(take(4 * En));
             permB = reinterpret_cast<std::uint32_t*>(take(4 * En));
@@ -1895,10 +1902,10 @@ int build_hybrid(const HybridParams& P, tcc_hybrid* out, void* stream) {
         // the remainder's COO over the elements that the last pass read
         restRow = reinterpret_cast<std::uint32_t*>(sorted == keysA ? keysB : keysA);
         restCol = restRow + E;
-        hipLaunchKernelGGL(step_counts_kernel, dim3(stepTileCount), dim3(kThreads), 0, st, sorted, E, P.minStepNnz,
+        hipLaunchKernelGGL(step_counts_kernel, dim3(stepTileCount), dim3(kThreads), 0, st, sorted, E, minStepNnz,
                            stepCounts, stepTileCount, a.pos);
         hipLaunchKernelGGL(row_scan_kernel, dim3(2), dim3(1024), 0, st, stepCounts, stepTileCount, small + 2);
-        hipLaunchKernelGGL(step_emit_kernel, dim3(stepTileCount), dim3(kThreads), 0, st, sorted, E, P.minStepNnz,
+        hipLaunchKernelGGL(step_emit_kernel, dim3(stepTileCount), dim3(kThreads), 0, st, sorted, E, minStepNnz,
                            stepCounts, stepTileCount, a, rowOrder, colOrder, stepStart, restRow, restCol, small + 5);
         TCC_LAUNCH_CHECK();
     } else if (E > 0) {

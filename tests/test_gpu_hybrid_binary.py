@@ -460,3 +460,31 @@ def test_binary_errors(gpu):
     small = torch.empty(8, dtype=torch.uint8, device="cuda")
     with pytest.raises(_lib.TccError, match="workspace"):
         swtcf.hybrid_spmm(H, torch.ones(4, 8, device="cuda"), workspace=small)
+
+
+@pytest.mark.parametrize("groupBlocks", [8, 16])
+def test_scaled_one_edge_many_times(gpu, groupBlocks):
+    """An edge repeated past what its step has places for is refused however
+    high minStepNnz is, without a walk over all its copies; a full step with
+    none repeated is not."""
+    import time
+
+    from tcc_amd import _lib, swtcf
+
+    n = 20_000_000
+    d, s = torch.full((n,), 3, dtype=torch.int32, device="cuda"), torch.full((n,), 70, dtype=torch.int32, device="cuda")
+    for least in (0, 1, 512 * groupBlocks, 2**32 - 1):
+        t = time.perf_counter()
+        with pytest.raises(_lib.TccError, match="duplicate"):
+            swtcf.coo_to_hybrid_scaled(d, s, 300, 200, min_step_nnz=least, group_blocks=groupBlocks)
+        assert time.perf_counter() - t < 2.0
+    rows, cols = 16 * groupBlocks, 32
+    d = torch.arange(rows, dtype=torch.int32, device="cuda").repeat_interleave(cols)
+    s = torch.arange(cols, dtype=torch.int32, device="cuda").repeat(rows)
+    X = torch.randn(cols, 64, device="cuda")
+    for least in (512 * groupBlocks, 512 * groupBlocks + 1, 2**32 - 1):
+        H = swtcf.coo_to_hybrid_scaled(d, s, rows, cols, min_step_nnz=least, group_blocks=groupBlocks)
+        assert H.view.tiles.nnz == (rows * cols if least == 512 * groupBlocks else 0)
+        Y = swtcf.hybrid_spmm(H, X)[:rows].double()
+        want = X.double().sum(0).expand(rows, -1)
+        assert float((Y - want).norm()) <= 2.0**-10 * float(want.norm())  # TF32 operands, fp32 sums
