@@ -161,6 +161,11 @@ int tcc_swtcf_spmm_mfma(const tcc_swtcf_matrix* m, const float* X, float* Y, uin
  * 0.5 GB at 233k rows and 114M edges) or its BCSR, and a workspace (or
  * packed X) for the last feature width. */
 int tcc_swtcf_set_plans(uint32_t maxPlans);
+/* Frees the device memory kept for the builders (up to 2 GiB a device, given
+ * back by finished builds and released matrices, for the next build).  The
+ * library's own allocations do that by themselves when memory is short; a
+ * program whose other allocator runs out can call this and try again. */
+int tcc_release_kept_memory(void);
 /* Releases every kept plan, and the device memory kept for the builders. */
 int tcc_swtcf_release_plans(void);
 /* Plans built since the process started. */

@@ -95,6 +95,7 @@ SIGNATURES = {
     "tcc_swtcf_spmm_mfma": (ctypes.c_int, [ctypes.POINTER(SWTCFMatrix), vp, vp, u32, u32, u32, vp]),
     "tcc_swtcf_spmm_quantized": (ctypes.c_int, [ctypes.POINTER(SWTCFMatrix), vp, vp, vp, vp, u32, vp]),
     "tcc_swtcf_set_plans": (ctypes.c_int, [u32]),
+    "tcc_release_kept_memory": (ctypes.c_int, []),
     "tcc_swtcf_release_plans": (ctypes.c_int, []),
     "tcc_swtcf_plans_built": (u32, []),
     "tcc_hash_arrays": (ctypes.c_int, [vp, vp, u32, vp, vp]),

@@ -1213,7 +1213,7 @@ int bcsc_by_conversion(const std::uint32_t* dRow, const std::uint32_t* dCol, con
                                  align_up(8 * std::max(T, 1u)) + align_up(4 * nnz) + align_up(4 * std::max(U, 1u)) +
                                  align_up(4 * std::max(T, 1u)) + align_up(4 * scan_temp_elems(T + 1));
     char* o = nullptr;
-    TCC_HIP_CHECK(hipMalloc(&o, outBytes));
+    TCC_HIP_CHECK(device_malloc(&o, outBytes));
     char* q = o;
     auto takeOut = [&](std::size_t bytes) {
         char* p = q;
@@ -1349,7 +1349,7 @@ int tcc_coo_to_bcsc(const std::uint32_t* dRow, const std::uint32_t* dCol, const 
         const std::uint32_t CW = (numCols + 7) / 8;
         const std::size_t offBytes = align_up(4ull * (CW + 1));
         char* o = nullptr;
-        TCC_HIP_CHECK(hipMalloc(&o, offBytes + align_up(4) + align_up(32) + align_up(8)));
+        TCC_HIP_CHECK(device_malloc(&o, offBytes + align_up(4) + align_up(32) + align_up(8)));
         if (fill<std::uint32_t>(reinterpret_cast<std::uint32_t*>(o), (offBytes + align_up(4) + align_up(32) + align_up(8)) / 4,
                                 0u, st) != hipSuccess ||
             hipStreamSynchronize(st) != hipSuccess) {

@@ -67,7 +67,9 @@ void keep(const Block& b) {
     else (void)hipFree(b.p);
 }
 
-hipError_t fresh(void** p, std::size_t bytes) {
+}  // namespace
+
+hipError_t device_malloc(void** p, std::size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
@@ -77,8 +79,6 @@ hipError_t fresh(void** p, std::size_t bytes) {
     if (e != hipSuccess) *p = nullptr;
     return e;
 }
-
-}  // namespace
 
 void pool_release() {
     std::lock_guard<std::mutex> lock(g_mutex);
@@ -96,7 +96,7 @@ hipError_t pool_malloc(void** p, std::size_t bytes) {
         b = take_kept(bytes, bytes + bytes / 8 + 65536, dev);  // arrays may be held for long: a close fit
     }
     if (!b.p) {
-        e = fresh(reinterpret_cast<void**>(&b.p), bytes);
+        e = device_malloc(&b.p, bytes);
         if (e != hipSuccess) return e;
         b.bytes = bytes;
     }
@@ -148,8 +148,15 @@ hipError_t Scratch::take(std::size_t bytes, hipStream_t st) {
         if (e == hipSuccess) e = hipHostGetDevicePointer(reinterpret_cast<void**>(&mailDev_), mailHost_, 0);
     }
     if (e == hipSuccess && !b.p) {
-        b.bytes = bytes + (bytes < kPoolKeep / 8 ? bytes / 4 : 0);  // room for somewhat larger calls to come
-        e = fresh(reinterpret_cast<void**>(&b.p), b.bytes);
+        // room for somewhat larger calls to come, where there is room
+        b.bytes = bytes + (bytes < kPoolKeep / 8 ? bytes / 4 : 0);
+        e = hipMalloc(reinterpret_cast<void**>(&b.p), b.bytes);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            b.bytes = bytes;
+            e = device_malloc(&b.p, bytes);
+        }
+        if (e != hipSuccess) b.p = nullptr;
     }
     p_ = b.p;
     bytes_ = b.bytes;

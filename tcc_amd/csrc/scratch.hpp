@@ -8,8 +8,9 @@
 // after its call has waited for its stream, handed-out arrays after the
 // device is idle (hipFree waits for that too).  So any thread and stream can
 // take it next.  At most kPoolKeep bytes are kept per device, the blocks kept
-// longest freed first; tcc_swtcf_release_plans frees them all, and so does an
-// allocation that would otherwise fail.
+// longest freed first; tcc_release_kept_memory and tcc_swtcf_release_plans free
+// them all, and so does any allocation of the library that would otherwise fail
+// (every one goes through device_malloc, pool_malloc or Scratch).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -28,6 +29,14 @@ hipError_t pool_free(void* p);
 
 // Frees every kept block of every device.
 void pool_release();
+
+// hipMalloc that frees the kept blocks and tries again where memory is short;
+// hipFree frees its result.
+hipError_t device_malloc(void** p, std::size_t bytes);
+template <typename T>
+hipError_t device_malloc(T** p, std::size_t bytes) {
+    return device_malloc(reinterpret_cast<void**>(p), bytes);
+}
 
 // One call's scratch, with a small host-mapped mailbox that its kernels
 // write and the host reads after a wait.

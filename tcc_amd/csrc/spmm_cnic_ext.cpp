@@ -152,6 +152,13 @@ torch::Tensor view_of(float* p, std::uint32_t rows, std::int32_t F, int device) 
                             torch::TensorOptions().dtype(torch::kFloat32).device(torch::kCUDA, device));
 }
 
+hipError_t device_malloc(void** p, std::size_t bytes) {
+    if (hipMalloc(p, bytes) == hipSuccess) return hipSuccess;
+    (void)hipGetLastError();
+    (void)tcc_release_kept_memory();
+    return hipMalloc(p, bytes);
+}
+
 int current_device() {
     int d = 0;
     if (hipGetDevice(&d) != hipSuccess) throw std::runtime_error("spmm_cnic: hipGetDevice failed");
@@ -167,7 +174,7 @@ std::uint32_t* error_word(int device) {
     TORCH_CHECK(device >= 0 && device < 64, "spmm_cnic: device id out of range");
     if (g_error_word[device] == nullptr) {
         void* p = nullptr;
-        if (hipMalloc(&p, sizeof(std::uint32_t)) != hipSuccess || hipMemset(p, 0, sizeof(std::uint32_t)) != hipSuccess)
+        if (device_malloc(&p, sizeof(std::uint32_t)) != hipSuccess || hipMemset(p, 0, sizeof(std::uint32_t)) != hipSuccess)
             throw std::runtime_error("spmm_cnic: cannot allocate the feature error word");
         g_error_word[device] = static_cast<std::uint32_t*>(p);
     }
@@ -209,9 +216,20 @@ tcc_feature_source feature_source(const torch::Tensor& id_map, py::capsule cpu_p
 
 // ---------------------------------------------------------------- the non-mixed forward
 
+// A device tensor; where memory is short, what the builders keep is given back
+// first.
+torch::Tensor device_empty(std::int64_t n, torch::ScalarType type, int device) {
+    const auto options = torch::TensorOptions().dtype(type).device(torch::kCUDA, device);
+    try {
+        return torch::empty({n}, options);
+    } catch (const c10::OutOfMemoryError&) {
+        check(tcc_release_kept_memory());
+    }
+    return torch::empty({n}, options);
+}
+
 torch::Tensor device_bytes(std::size_t n, int device) {
-    return torch::empty({static_cast<std::int64_t>(n)},
-                        torch::TensorOptions().dtype(torch::kUInt8).device(torch::kCUDA, device));
+    return device_empty(static_cast<std::int64_t>(n), torch::kUInt8, device);
 }
 
 void* aligned16(const torch::Tensor& t) {
@@ -294,8 +312,7 @@ const tcc_hybrid* plan_for(const tcc_bcsr& A, int device, void* st) {
     const void* arrays[4] = {A.rowWindowOffset, A.sparseA2B, A.tcLocalBit, A.data};
     const std::uint64_t bytes[4] = {4ull * (A.num_rowWindows + 1ull), 32ull * A.num_TCBlocks, 8ull * A.num_TCBlocks,
                                     4ull * A.nnz};
-    torch::Tensor h =
-        torch::empty({TCC_HASH_WORDS}, torch::TensorOptions().dtype(torch::kInt64).device(torch::kCUDA, device));
+    torch::Tensor h = device_empty(TCC_HASH_WORDS, torch::kInt64, device);
     check(tcc_hash_arrays(arrays, bytes, values ? 4 : 3, reinterpret_cast<std::uint64_t*>(h.data_ptr()), st));
     torch::Tensor hh = torch::empty({TCC_HASH_WORDS}, torch::TensorOptions().dtype(torch::kInt64).pinned_memory(true));
     hh.copy_(h, /*non_blocking=*/true);
@@ -433,9 +450,7 @@ torch::Tensor fwd_bound(std::uint32_t r_rows, std::uint32_t r_cols, std::uint32_
 
 torch::Tensor alloc_output(std::uint32_t windows, std::int32_t F) {
     TORCH_CHECK(F >= 1, "feature_dim must be positive");
-    const int dev = current_device();
-    auto out = torch::empty({denseC_elems(windows, F)},
-                            torch::TensorOptions().dtype(torch::kFloat32).device(torch::kCUDA, dev));
+    auto out = device_empty(denseC_elems(windows, F), torch::kFloat32, current_device());
     g_outputs.push_back(out);
     return out;
 }
@@ -499,7 +514,7 @@ std::vector<py::capsule> space_malloc(int device_id, std::uint32_t denseC_size) 
     for (const char* name : {"denseC", "denseC_2"}) {
         void* p = nullptr;
         const std::size_t bytes = static_cast<std::size_t>(denseC_size) * sizeof(float);
-        if (hipMalloc(&p, bytes) != hipSuccess || hipMemset(p, 0, bytes) != hipSuccess) {
+        if (device_malloc(&p, bytes) != hipSuccess || hipMemset(p, 0, bytes) != hipSuccess) {
             throw std::runtime_error("spmm_cnic: space_malloc failed");
         }
         g_spaces.push_back(p);
@@ -516,6 +531,7 @@ void finalize(int device_id) {
     g_spaces.clear();
     g_outputs.clear();
     release_plans();
+    check(tcc_release_kept_memory());
 }
 
 void freeMatC() {
@@ -567,6 +583,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           "per-graph plans (dense tiles on MFMA + gather), found by a hash of the BCSR arrays: n > 0 keeps up to n, "
           "built by the first call on a graph; 0 turns them off; -1 restores the default (one plan, for large "
           "skewed graphs, built by the second call that finds the same arrays)");
-    m.def("release_plans", &release_plans, "release every per-graph plan");
+    m.def(
+        "release_plans",
+        [] {
+            release_plans();
+            check(tcc_release_kept_memory());
+        },
+        "release every per-graph plan");
     m.def("graph_plans", &graph_plans, "the number of per-graph plans held");
 }

@@ -33,6 +33,7 @@
 #include "../../include/tcc_swtcf.h"
 #include "common.hpp"
 #include "primitives.hpp"
+#include "scratch.hpp"
 
 namespace tcc {
 
@@ -1293,7 +1294,7 @@ int tcc_swtcf_alloc_matrix(tcc_swtcf_matrix* m, std::uint32_t rows, std::uint32_
     std::size_t total = 0;
     for (std::size_t s : sizes) total += align_up(s);
     char* base = nullptr;
-    if (hipMalloc(&base, total) != hipSuccess) {
+    if (device_malloc(&base, total) != hipSuccess) {
         std::memset(m, 0, sizeof(*m));
         set_last_error("hipMalloc failed for the SWTCF arrays");
         return TCC_ERR_NO_MEMORY;
@@ -1338,7 +1339,7 @@ int tcc_swtcf_alloc_workspace(tcc_swtcf_workspace* ws, std::uint32_t edgeCapacit
     const Carve c = carve(nullptr, edgeCapacity, ws->numColWindows, ws->numSuperWindows, superWindowSize);
     const std::size_t bytes = c.bytes + 256;  // + deviceNumGroups / deviceError
     char* base = nullptr;
-    if (hipMalloc(&base, bytes) != hipSuccess) {
+    if (device_malloc(&base, bytes) != hipSuccess) {
         std::memset(ws, 0, sizeof(*ws));
         set_last_error("hipMalloc failed for the converter workspace");
         return TCC_ERR_NO_MEMORY;

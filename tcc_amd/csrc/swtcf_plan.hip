@@ -282,7 +282,7 @@ struct PlanCache {
         for (auto& b : hashBuf)
             if (b.device == device) return &b;
         HashBuf b{device, nullptr, nullptr};
-        if (hipMalloc(&b.dev, kHashWords * sizeof(std::uint64_t)) != hipSuccess) return nullptr;
+        if (device_malloc(&b.dev, kHashWords * sizeof(std::uint64_t)) != hipSuccess) return nullptr;
         if (hipHostMalloc(&b.host, kHashWords * sizeof(std::uint64_t), hipHostMallocDefault) != hipSuccess) {
             (void)hipFree(b.dev);
             return nullptr;
@@ -335,7 +335,7 @@ int build_plan(const tcc_swtcf_matrix* m, Plan& P, hipStream_t st) {
     const std::uint64_t Tn = std::max<std::uint64_t>(T, 1);
     const std::size_t a = (4 * (Tn + 1) + 255) / 256 * 256;
     const std::size_t tempBytes = (4 * scan_temp_elems(Tn + 1) + 255) / 256 * 256;
-    TCC_HIP_CHECK(hipMalloc(&scratch.p, 2 * a + tempBytes + 256));
+    TCC_HIP_CHECK(device_malloc(&scratch.p, 2 * a + tempBytes + 256));
     auto* counts = static_cast<std::uint32_t*>(scratch.p);
     auto* offset = reinterpret_cast<std::uint32_t*>(static_cast<char*>(scratch.p) + a);
     auto* temp = reinterpret_cast<std::uint32_t*>(static_cast<char*>(scratch.p) + 2 * a);
@@ -352,7 +352,7 @@ int build_plan(const tcc_swtcf_matrix* m, Plan& P, hipStream_t st) {
     TCC_HIP_CHECK(hipStreamSynchronize(st));
     Bufs coo;
     const std::uint64_t En = std::max<std::uint32_t>(nnz, 1);
-    TCC_HIP_CHECK(hipMalloc(&coo.p, 8 * En));
+    TCC_HIP_CHECK(device_malloc(&coo.p, 8 * En));
     auto* dst = static_cast<std::uint32_t*>(coo.p);
     auto* src = dst + En;
     if (T > 0) {
@@ -454,7 +454,7 @@ int swtcf_plan_spmm(const tcc_swtcf_matrix* m, const float* X, float* Y, std::ui
         P->wsF = 0;
         P->wsBytes = P->hybrid ? tcc_hybrid_workspace_bytes(&P->H, F) + 16
                                : (P->packs ? tcc_tf32_packed_bytes(m->cols, F) + 16 : 0);
-        if (P->wsBytes && hipMalloc(&P->ws, P->wsBytes) != hipSuccess) {  // no room for this F: the kernel
+        if (P->wsBytes && device_malloc(&P->ws, P->wsBytes) != hipSuccess) {  // no room for this F: the kernel
             P->ws = nullptr;
             P->wsBytes = 0;
             (void)hipGetLastError();
@@ -463,7 +463,7 @@ int swtcf_plan_spmm(const tcc_swtcf_matrix* m, const float* X, float* Y, std::ui
         P->wsF = F;
     }
     if (quant) {
-        if (!P->xq && hipMalloc(&P->xq, 4ull * m->cols * F) != hipSuccess) {
+        if (!P->xq && device_malloc(&P->xq, 4ull * m->cols * F) != hipSuccess) {
             P->xq = nullptr;
             (void)hipGetLastError();
             return TCC_OK;
@@ -506,6 +506,12 @@ int tcc_swtcf_set_plans(std::uint32_t maxPlans) {
     C.init = true;
     C.maxPlans = maxPlans;
     C.trim();
+    return TCC_OK;
+}
+
+int tcc_release_kept_memory(void) {
+    clear_last_error();
+    pool_release();
     return TCC_OK;
 }
 

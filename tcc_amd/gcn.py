@@ -67,7 +67,7 @@ class LayerGraph:
     def aggregate(self, F: int, x: torch.Tensor | None = None, source=None) -> torch.Tensor:
         """AX [num_rows x F] (a view of the (RW+1)*8-row denseC buffer)."""
         RW = self.bcsr.view.num_rowWindows
-        denseC = torch.empty(((RW + 1) * 8, F), dtype=torch.float32, device="cuda")
+        denseC = swtcf._empty(((RW + 1) * 8, F), torch.float32, "cuda")
         if source is not None:
             bcsc = self.bcsc if self.bcsc is not None else _EMPTY_BCSC
             swtcf.spmm_cnic_forward_mixed(self.bcsr, bcsc, source, denseC, F)

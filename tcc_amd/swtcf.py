@@ -55,6 +55,16 @@ def _ptr(t) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+def _empty(shape, dtype, device) -> torch.Tensor:
+    """torch.empty; where memory is short, what the builders keep is given
+    back first."""
+    try:
+        return torch.empty(shape, dtype=dtype, device=device)
+    except torch.cuda.OutOfMemoryError:
+        check(_lib.lib().tcc_release_kept_memory())
+    return torch.empty(shape, dtype=dtype, device=device)
+
+
 def _f32(t: torch.Tensor, name: str) -> torch.Tensor:
     """A contiguous float32 device tensor (the kernels read raw fp32)."""
     if t.dtype != torch.float32 or not t.is_cuda:
@@ -311,7 +321,7 @@ def bcsr_spmm(A: BlockMatrix, X: torch.Tensor, Y: torch.Tensor | None = None, ac
     X = _f32(X, "X")
     F = X.shape[1]
     if Y is None:
-        Y = torch.empty((A.out_windows * 8, F), dtype=torch.float32, device=X.device)
+        Y = _empty((A.out_windows * 8, F), torch.float32, X.device)
     check(_lib.lib().tcc_bcsr_spmm(ctypes.byref(A.view), X.data_ptr(), Y.data_ptr(), F, int(accumulate),
                                    _stream(stream)))
     return Y
@@ -324,7 +334,7 @@ def tf32_pack(X: torch.Tensor, out: torch.Tensor | None = None, stream=None) -> 
     rows, F = X.shape
     nbytes = _lib.lib().tcc_tf32_packed_bytes(rows, F)
     if out is None:
-        out = torch.empty(nbytes + 16, dtype=torch.uint8, device=X.device)
+        out = _empty(nbytes + 16, torch.uint8, X.device)
     base = out.data_ptr()
     shift = (-base) % 16
     packed = out[shift:shift + nbytes]
@@ -336,7 +346,7 @@ def bcsr_spmm_packed(A: BlockMatrix, packed: torch.Tensor, F: int, Y: torch.Tens
                      accumulate: bool = False, stream=None) -> torch.Tensor:
     """Y[8*W x F] (=|+=) A X with X given by tf32_pack, W = A.out_windows."""
     if Y is None:
-        Y = torch.empty((A.out_windows * 8, F), dtype=torch.float32, device=packed.device)
+        Y = _empty((A.out_windows * 8, F), torch.float32, packed.device)
     check(_lib.lib().tcc_bcsr_spmm_packed(ctypes.byref(A.view), packed.data_ptr(), Y.data_ptr(), F,
                                           int(accumulate), _stream(stream)))
     return Y
@@ -455,10 +465,10 @@ def hybrid_spmm(H: HybridMatrix, X: torch.Tensor, Y: torch.Tensor | None = None,
     X = _f32(X, "X")
     F = X.shape[1]
     if Y is None:
-        Y = torch.empty((H.out_rows, F), dtype=torch.float32, device=X.device)
+        Y = _empty((H.out_rows, F), torch.float32, X.device)
     need = H.workspace_bytes(F)
     if workspace is None:
-        workspace = torch.empty(need + 16, dtype=torch.uint8, device=X.device)
+        workspace = _empty(need + 16, torch.uint8, X.device)
     base = workspace.data_ptr()
     shift = (-base) % 16
     check(_lib.lib().tcc_hybrid_spmm(ctypes.byref(H.view), X.data_ptr(), Y.data_ptr(), F, int(accumulate),
@@ -475,7 +485,7 @@ def hub_tiles_spmm(H: HybridMatrix, X: torch.Tensor, Y: torch.Tensor, workspace:
     F = X.shape[1]
     need = int(_lib.lib().tcc_hub_tiles_workspace_bytes(ctypes.byref(H.view.tiles), F))
     if workspace is None:
-        workspace = torch.empty(need + 16, dtype=torch.uint8, device=X.device)
+        workspace = _empty(need + 16, torch.uint8, X.device)
     base = workspace.data_ptr()
     shift = (-base) % 16
     check(_lib.lib().tcc_hub_tiles_spmm(ctypes.byref(H.view.tiles), X.data_ptr(), Y.data_ptr(), F, base + shift,
@@ -496,7 +506,7 @@ def bcsc_transpose_spmm(A: BlockMatrix, dY: torch.Tensor, dX: torch.Tensor | Non
     dY = _f32(dY, "dY")
     F = dY.shape[1]
     if dX is None:
-        dX = torch.empty((A.view.num_colWindows * 8, F), dtype=torch.float32, device=dY.device)
+        dX = _empty((A.view.num_colWindows * 8, F), torch.float32, dY.device)
     check(_lib.lib().tcc_bcsc_transpose_spmm(ctypes.byref(A.view), dY.data_ptr(), dX.data_ptr(), F,
                                              int(accumulate), _stream(stream)))
     return dX
@@ -523,11 +533,11 @@ def dense_tn(A: torch.Tensor, B: torch.Tensor, C: torch.Tensor | None = None, ac
         raise ValueError(f"A and B need the same number of rows (got {K} and {B.shape[0]})")
     N = B.shape[1]
     if C is None:
-        C = torch.empty((M, N), dtype=torch.float32, device=A.device)
+        C = _empty((M, N), torch.float32, A.device)
     elif C.shape != (M, N) or C.dtype != torch.float32 or C.stride(1) != 1:
         raise ValueError(f"C must be a float32 [{M} x {N}] tensor with contiguous rows")
     nbytes = _lib.lib().tcc_dense_tn_workspace_bytes(K, M, N)
-    ws = torch.empty(max(nbytes, 4), dtype=torch.uint8, device=A.device)
+    ws = _empty(max(nbytes, 4), torch.uint8, A.device)
     check(_lib.lib().tcc_dense_tn(A.data_ptr(), A.stride(0), B.data_ptr(), B.stride(0), C.data_ptr(), C.stride(0),
                                   K, M, N, int(accumulate), ws.data_ptr(), nbytes, _stream(stream)))
     return C
@@ -547,8 +557,8 @@ def gcn_relu_forward(AX: torch.Tensor, W1: torch.Tensor, W2: torch.Tensor,
     Hd, C = W2.shape
     if W1.shape != (F, Hd):
         raise ValueError(f"shape mismatch: AX {tuple(AX.shape)}, W1 {tuple(W1.shape)}, W2 {tuple(W2.shape)}")
-    H = torch.empty((K, Hd), dtype=torch.float32, device=AX.device)
-    XW = torch.empty((K, C), dtype=torch.float32, device=AX.device)
+    H = _empty((K, Hd), torch.float32, AX.device)
+    XW = _empty((K, C), torch.float32, AX.device)
     check(_lib.lib().tcc_gcn_relu_forward(AX.data_ptr(), AX.stride(0), W1.data_ptr(), W2.data_ptr(), H.data_ptr(),
                                           Hd, XW.data_ptr(), C, K, F, Hd, C, _stream(stream)))
     return H, XW
@@ -566,10 +576,10 @@ def gcn_relu_grad(AX: torch.Tensor, H: torch.Tensor, G: torch.Tensor, W2: torch.
     if H.shape != (K, Hd) or G.shape != (K, C):
         raise ValueError(f"shape mismatch: AX {tuple(AX.shape)}, H {tuple(H.shape)}, G {tuple(G.shape)}, "
                          f"W2 {tuple(W2.shape)}")
-    dW1 = torch.empty((F, Hd), dtype=torch.float32, device=AX.device)
-    dW2 = torch.empty((Hd, C), dtype=torch.float32, device=AX.device)
+    dW1 = _empty((F, Hd), torch.float32, AX.device)
+    dW2 = _empty((Hd, C), torch.float32, AX.device)
     nbytes = _lib.lib().tcc_gcn_relu_grad_workspace_bytes(K, F, Hd, C)
-    ws = torch.empty(max(nbytes, 4), dtype=torch.uint8, device=AX.device)
+    ws = _empty(max(nbytes, 4), torch.uint8, AX.device)
     check(_lib.lib().tcc_gcn_relu_grad(AX.data_ptr(), AX.stride(0), H.data_ptr(), H.stride(0), G.data_ptr(),
                                        G.stride(0), W2.data_ptr(), dW1.data_ptr(), dW2.data_ptr(), K, F, Hd, C,
                                        ws.data_ptr(), nbytes, _stream(stream)))
@@ -628,7 +638,7 @@ def spmm_cnic_forward_mixed(bcsr: BlockMatrix, bcsc: BlockMatrix, src: FeatureSo
     if need:
         try:
             with torch.cuda.stream(stream):  # None: the current stream
-                ws = torch.empty(need, dtype=torch.uint8, device=denseC.device)
+                ws = _empty(need, torch.uint8, denseC.device)
         except torch.cuda.OutOfMemoryError:
             need = 0
     check(_lib.lib().tcc_spmm_cnic_forward_mixed_ws(*args, denseC.data_ptr(), F, _ptr(ws), need, _stream(stream)))
