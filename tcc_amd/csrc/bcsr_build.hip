@@ -25,8 +25,9 @@
 //      the lists read off an edge a thread.
 //   3. The lists' lengths give the block offsets (one scan), and one pass
 //      over the edges' positions writes blocks, bitmaps and value offsets.
-// The host waits once (twice where the order check decides the route), to
-// learn the block count; outputs are sized before by what E edges can need.
+// The host waits once (and once more where the order check decides the route),
+// to learn the block count; outputs are sized before by what E edges can need
+// (the largest after one more wait).
 //
 // Bound by launches and by each pass's chain of loads at 1M edges, by the
 // lists' instructions at 100M.  The sort of whole 36-bit keys with an edge
@@ -960,7 +961,14 @@ using namespace tcc;
 namespace {
 
 // The build's output arrays, in one allocation: off[RW + 1], tcOffset,
-// idx, bits for at most maxB blocks, data[E] (with values).
+// idx, bits for at most maxB blocks, data[E] (with values).  A caller holds
+// them for the matrix's life, and where windows share columns they have up to
+// 8 times fewer blocks than their edges could fill: at most kMaxSlack of that
+// is kept.  Arrays for kCountFirst bytes of blocks and more are allocated when
+// the host knows their number (a wait more: 20 us, of 2 ms and more); smaller
+// ones for what the edges could need, and moved to smaller ones at the end
+// where that was much too much.
+constexpr std::uint64_t kBlockBytes = 44, kMaxSlack = 32ull << 20, kCountFirst = 256ull << 20;
 struct BlockArrays {
     char* base = nullptr;
     std::uint32_t *off = nullptr, *tcOffset = nullptr, *idx = nullptr;
@@ -997,6 +1005,9 @@ int build_blocks(Coo c, std::uint32_t RW, const float* val, BlockArrays& out, st
                  hipStream_t st) {
     const bool tryGrouped = !BCSC && c.phases == 1;
     const std::uint64_t E = c.E;
+    // ceil(length / 8) summed over at most min(RW, E) windows with edges
+    const std::uint64_t maxB = std::min<std::uint64_t>(E, (E + 7 * std::min<std::uint64_t>(RW, E)) / 8);
+    const bool exact = kBlockBytes * maxB > kCountFirst;
     const unsigned wBits = ceil_log2(RW);
     const bool places = BCSC && val;
     std::uint64_t *keysA = nullptr, *keysB = nullptr;
@@ -1023,7 +1034,7 @@ int build_blocks(Coo c, std::uint32_t RW, const float* val, BlockArrays& out, st
         flags = reinterpret_cast<std::uint32_t*>(take(64));
         L.length = reinterpret_cast<std::uint32_t*>(take(4ull * RW + 64));
         winStart = reinterpret_cast<std::uint32_t*>(take(4ull * (RW + 1ull)));
-        blocks = reinterpret_cast<std::uint32_t*>(take(RW > kOneScan ? 4ull * RW : 0));
+        blocks = reinterpret_cast<std::uint32_t*>(take(RW > kOneScan || exact ? 4ull * (RW + 1ull) : 0));
         scanTemp = reinterpret_cast<std::uint32_t*>(take(RW > kOneScan ? 4 * scan_temp_elems(RW) : 0));
         L.mid = reinterpret_cast<std::uint32_t*>(take(4 * (E / kShort + 1)));
         L.big = reinterpret_cast<std::uint32_t*>(take(4 * (E / kMid + 1)));
@@ -1098,19 +1109,38 @@ int build_blocks(Coo c, std::uint32_t RW, const float* val, BlockArrays& out, st
         else lists(std::false_type{});
     }
     TCC_LAUNCH_CHECK();
-    // ceil(length / 8) summed over at most min(RW, E) windows with edges
-    const std::uint64_t maxB = std::min<std::uint64_t>(E, (E + 7 * std::min<std::uint64_t>(RW, E)) / 8);
-    TCC_HIP_CHECK(out.allocate(RW, maxB, E, val != nullptr));
-    // the blocks of the lists; mail holds their count and the flags afterwards
-    auto finish = [&]() -> int {
+    auto offsets = [&](std::uint32_t* off) -> int {
         if (RW <= kOneScan) {
-            hipLaunchKernelGGL(window_blocks_kernel, dim3(1), dim3(1024), 0, st, L.length, RW, out.off);
+            hipLaunchKernelGGL(window_blocks_kernel, dim3(1), dim3(1024), 0, st, L.length, RW, off);
         } else {
             hipLaunchKernelGGL(blocks_per_window_kernel, dim3(grid_for(RW, kThreads)), dim3(kThreads), 0, st, L.length,
                                RW, blocks);
-            TCC_HIP_CHECK(exclusive_scan(blocks, out.off, RW, out.off + RW, scanTemp, st));
+            TCC_HIP_CHECK(exclusive_scan(blocks, off, RW, off + RW, scanTemp, st));
         }
         TCC_LAUNCH_CHECK();
+        return TCC_OK;
+    };
+    auto read_mail = [&]() -> int {
+        TCC_HIP_CHECK(scratch.wait());
+        B = scratch.read()[0];
+        what = scratch.read()[1] ? Built::Range : scratch.read()[2] ? Built::Duplicate
+               : scratch.read()[3] ? Built::TooLong : Built::Ok;
+        return TCC_OK;
+    };
+    // the blocks of the lists; the mail holds their count and the flags afterwards
+    auto finish = [&]() -> int {
+        if (exact) {
+            if (const int rc = offsets(blocks)) return rc;
+            hipLaunchKernelGGL(tell_host_kernel, dim3(1), dim3(1), 0, st, L, blocks, scratch.mail());
+            TCC_LAUNCH_CHECK();
+            if (const int rc = read_mail()) return rc;
+            if (what != Built::Ok) return TCC_OK;
+            TCC_HIP_CHECK(out.allocate(RW, B, E, val != nullptr));
+            TCC_HIP_CHECK(hipMemcpyAsync(out.off, blocks, 4ull * (RW + 1ull), hipMemcpyDeviceToDevice, st));
+        } else {
+            if (!out.base) TCC_HIP_CHECK(out.allocate(RW, maxB, E, val != nullptr));
+            if (const int rc = offsets(out.off)) return rc;
+        }
         if constexpr (BCSC) {
             emit(std::true_type{});
         } else {
@@ -1123,11 +1153,7 @@ int build_blocks(Coo c, std::uint32_t RW, const float* val, BlockArrays& out, st
                                out.bits, val, out.data);
             TCC_LAUNCH_CHECK();
         }
-        TCC_HIP_CHECK(scratch.wait());
-        B = scratch.read()[0];
-        what = scratch.read()[1] ? Built::Range : scratch.read()[2] ? Built::Duplicate
-               : scratch.read()[3] ? Built::TooLong : Built::Ok;
-        return TCC_OK;
+        return read_mail();
     };
     // the lists again, of the whole COO sorted
     auto sort_all = [&]() -> int {
@@ -1164,6 +1190,27 @@ int build_blocks(Coo c, std::uint32_t RW, const float* val, BlockArrays& out, st
     if (rc == TCC_OK && what == Built::TooLong) {
         rc = sort_all();
         if (rc == TCC_OK) rc = finish();
+    }
+    if (rc == TCC_OK && what == Built::Ok && !exact && kBlockBytes * (maxB - B) > kMaxSlack) {
+        BlockArrays fit;
+        if (fit.allocate(RW, B, E, val != nullptr) == hipSuccess) {
+            const auto move = [&](void* to, const void* from, std::uint64_t bytes) {
+                return bytes == 0 ? hipSuccess : hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToDevice, st);
+            };
+            if (move(fit.off, out.off, 4ull * (RW + 1ull)) == hipSuccess &&
+                move(fit.tcOffset, out.tcOffset, 4ull * (B + 1ull)) == hipSuccess &&
+                move(fit.idx, out.idx, 32ull * B) == hipSuccess && move(fit.bits, out.bits, 8ull * B) == hipSuccess &&
+                move(fit.data, out.data, val ? 4 * E : 0) == hipSuccess && scratch.wait() == hipSuccess) {
+                (void)pool_free(out.base);
+                out = fit;
+            } else {
+                (void)pool_free(fit.base);
+                set_last_error("HIP error while building the block arrays");
+                rc = TCC_ERR_HIP;
+            }
+        } else {
+            (void)hipGetLastError();  // no room for both: the larger ones stay
+        }
     }
     if (rc == TCC_OK) {  // all work waited for, and none queued after it
         scratch.idle();

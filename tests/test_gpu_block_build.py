@@ -237,3 +237,39 @@ def test_one_row_joined_to_every_column(gpu):
         spread, hub = seconds(build, False, swap), seconds(build, True, swap)
         print(f"spread {spread * 1e3:.2f} ms, with a hub {hub * 1e3:.2f} ms")
         assert hub < 8 * spread
+
+
+@pytest.mark.parametrize("values", [False, True])
+@pytest.mark.parametrize("deg", [250, 800])
+def test_arrays_take_what_their_blocks_need(gpu, deg, values):
+    """A kept matrix holds its blocks, not what its edges could fill: 8 rows a
+    window that share their columns give an eighth of those blocks."""
+    from tcc_amd import _lib, swtcf
+
+    n = 64_000
+    g = torch.Generator(device="cuda").manual_seed(2)
+    start = torch.randint(0, n - 8 * deg, (n // 8,), generator=g, device="cuda").repeat_interleave(8 * deg)
+    k = torch.arange(n // 8, device="cuda").repeat_interleave(8 * deg)
+    r = 8 * k + torch.arange(8, device="cuda").repeat_interleave(deg).repeat(n // 8)
+    c = start + torch.arange(deg, device="cuda").repeat(n)
+    val = torch.arange(r.numel(), device="cuda").float() if values else None
+    for build, a, b in ((swtcf.coo_to_bcsr, r, c), (swtcf.coo_to_bcsc, c, r)):
+        a, b = a.int(), b.int()
+        torch.cuda.synchronize()
+        _lib.check(_lib.lib().tcc_release_kept_memory())
+        free = torch.cuda.mem_get_info()[0]
+        A = build(a, b, val, n, n)
+        _lib.check(_lib.lib().tcc_release_kept_memory())
+        held = free - torch.cuda.mem_get_info()[0]
+        blocks = A.view.num_TCBlocks
+        assert blocks <= r.numel() // 48
+        # 44 bytes a block, the window offsets, and the allocation's granularity
+        assert held <= 44 * blocks + 4 * (n // 8 + 1) + (4 * r.numel() if values else 0) + (8 << 20), (held, blocks)
+        # whole numbers: every order of the sums gives one result
+        X = torch.ones(n, 1, device="cuda")
+        if build is swtcf.coo_to_bcsr and not values:
+            assert torch.equal(swtcf.bcsr_spmm(A, X)[:n, 0], torch.full((n,), float(deg), device="cuda"))
+        if build is swtcf.coo_to_bcsr and values:
+            H = A.to_host()
+            assert np.array_equal(np.sort(H["data"]), val.cpu().numpy())
+        A.release()
