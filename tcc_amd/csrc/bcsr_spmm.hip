@@ -1572,6 +1572,11 @@ int mixed_vec(const tcc_feature_source* src, std::uint32_t F, const float* Y) {
 // 56 : 65 at F = 100 (8 MB).
 constexpr std::uint32_t kMixedPackMinF = 17;
 constexpr std::uint64_t kMixedPackMinTable = 128ull << 20;
+// Output size from which the first layer without a scatter stores its rows: a
+// launch more than the zero fill and the adds (zeros for the windows that units
+// share).  Adds against stores, us: 2000 nodes, F = 100 29.1 : 35.5; 100k nodes,
+// F = 17 (7 MB) 70.9 : 74.2, 64 (26 MB) 75.6 : 77.1, 100 (40 MB) 108 : 101.
+constexpr std::uint64_t kStoreMinBytes = 32ull << 20;
 bool mixed_pack_pays(const tcc_bcsr* A, std::uint32_t F) {
     return 8ull * A->num_TCBlocks >= kPackMinGathers * A->num_cols && F >= kMixedPackMinF &&
            4ull * F * A->num_cols >= kMixedPackMinTable;
@@ -1924,16 +1929,17 @@ int tcc_spmm_cnic_forward_mixed_ws(const tcc_bcsr* bcsr, const tcc_bcsc* bcsc, c
     TCC_REQUIRE(bcsr->phases <= 1, TCC_ERR_UNSUPPORTED, "spmm_cnic forward takes an ordinary (unphased) BCSR");
     const hipStream_t st = as_stream(stream);
     const std::uint64_t F = featureDim;
-    if (bcsc->num_TCBlocks == 0 || bcsc->num_colWindows == 0) {
+    const bool pack = src->row_format == TCC_ROWS_FP32 && bcsr->num_cols != 0 && bcsr->num_TCBlocks != 0 &&
+                      workspace != nullptr && workspaceBytes >= mixed_pack_bytes(bcsr, featureDim);
+    if ((bcsc->num_TCBlocks == 0 || bcsc->num_colWindows == 0) &&
+        (pack || 32 * F * bcsr->num_rowWindows >= kStoreMinBytes)) {
         // No scatter: the gather alone stores every row of the windows it
         // covers (no zero fill, atomics only where units share a window).
         // 2.45M nodes, 61.9M edges, F = 100, all rows on the device: 5.30 ms
         // with the zero fill and every window added; 4.91 from fp32 rows,
         // 2.82 with the rows packed first.
         TCC_HIP_CHECK(fill<float>(denseC + static_cast<std::uint64_t>(bcsr->num_rowWindows) * 8 * F, 8 * F, 0.0f, st));
-        if (src->row_format != TCC_ROWS_FP32 || bcsr->num_cols == 0 || bcsr->num_TCBlocks == 0 ||
-            workspace == nullptr || workspaceBytes < mixed_pack_bytes(bcsr, featureDim))
-            return tcc_bcsr_spmm_mixed(bcsr, src, denseC, featureDim, 0, stream);
+        if (!pack) return tcc_bcsr_spmm_mixed(bcsr, src, denseC, featureDim, 0, stream);
         const std::uint32_t rows = bcsr->num_cols;
         auto* packed = reinterpret_cast<unsigned char*>((reinterpret_cast<std::uintptr_t>(workspace) + 15) & ~std::uintptr_t(15));
         auto* used = reinterpret_cast<std::uint32_t*>(packed + tcc_tf32_packed_bytes(rows, featureDim));

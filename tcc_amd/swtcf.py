@@ -21,6 +21,8 @@ DEFAULT_TC_THRESHOLD = 12
 DEVERR_FEATURE_INDEX = 7  # TCC_DEVERR_FEATURE_INDEX
 TILES_FP32, TILES_BF16X2, TILES_BINARY = 0, 1, 2  # TCC_TILES_*
 FEATURE_DIM = 128
+# Smallest feature table (bytes) for which tcc_spmm_cnic_forward_mixed_workspace_bytes names a workspace
+MIXED_PACK_MIN_TABLE = 128 << 20
 
 
 _hip = None
@@ -633,7 +635,9 @@ def spmm_cnic_forward_mixed(bcsr: BlockMatrix, bcsc: BlockMatrix, src: FeatureSo
     with a workspace of the launch's stream where packing the rows pays and
     memory has room for it."""
     args = (ctypes.byref(bcsr.view), ctypes.byref(bcsc.view), ctypes.byref(src.struct))
-    need = int(_lib.lib().tcc_spmm_cnic_forward_mixed_workspace_bytes(*args, F))
+    need = 0
+    if 4 * F * bcsr.view.num_cols >= MIXED_PACK_MIN_TABLE:  # spares small products the question
+        need = int(_lib.lib().tcc_spmm_cnic_forward_mixed_workspace_bytes(*args, F))
     ws = None
     if need:
         try:

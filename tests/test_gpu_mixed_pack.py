@@ -121,3 +121,24 @@ def test_mixed_workspace_only_where_it_applies(gpu):
         swtcf.spmm_cnic_forward_mixed(g.bcsr, gcn._EMPTY_BCSC, hot.source, out, F, stream=s)
     s.synchronize()
     assert torch.equal(out, direct)
+
+
+@pytest.mark.parametrize("F", [449, 450, 452])
+@pytest.mark.parametrize("rows", [18_000, 20_000])
+def test_mixed_stored_and_added(gpu, rows, F):
+    """Both routes of the unpacked first layer without a scatter, at their line
+    of 32 MiB: whole numbers, so that every order of the sums gives one result."""
+    from tcc_amd import gcn, graphs, swtcf
+
+    n = 20_000
+    r, c = graphs.rmat_graph(n, 200_000, 5, device="cuda")
+    keep = (r < rows) & (r // 8 % 5 != 2)  # windows without an entry
+    r, c = r[keep], c[keep]
+    X = torch.randint(-3, 4, (n, F), generator=torch.Generator().manual_seed(F)).float()
+    table = gcn.FeatureTable(X, c, hot_fraction=1.0)
+    g = gcn.LayerGraph(r, c, rows, n, hot_src=table.hot, backward_bcsc=gcn._EMPTY_BCSC)
+    assert (g.bcsr.view.num_rowWindows * 32 * F >= 32 << 20) == (rows == 20_000)
+    want = torch.zeros(rows, F, dtype=torch.float64, device="cuda").index_add_(0, r, X.cuda().double()[c])
+    out = torch.full(((g.bcsr.view.num_rowWindows + 1) * 8, F), float("nan"), device="cuda")
+    swtcf.spmm_cnic_forward_mixed(g.bcsr, gcn._EMPTY_BCSC, table.source, out, F)
+    assert torch.equal(out[:rows].double(), want) and not out[rows:].any()
