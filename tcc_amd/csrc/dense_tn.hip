@@ -270,7 +270,8 @@ __global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
             w2[e][j] = CT > 0 && static_cast<std::uint32_t>(j) < a.C
                            ? a.W2[static_cast<std::uint64_t>(colB[e]) * a.C + j] : 0.0f;
         }
-    float maxA = 0.0f, maxB[2] = {0.0f, 0.0f};  // of the columns' magnitudes
+    // largest and smallest nonzero magnitudes of the columns, and of G
+    float maxA = 0.0f, maxB[2] = {0.0f, 0.0f}, maxG = 0.0f;
     std::uint32_t lowA = ~0u, lowB[2] = {~0u, ~0u};
 
     f32x4 acc[TW][4];
@@ -302,12 +303,11 @@ __global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
             xg = a.G[static_cast<std::uint64_t>(min(row, k1 - 1)) * a.ldg + min(gj, a.C - 1)];
         }
     };
-    auto put = [&](uint4* to, std::uint32_t part, const float (&x)[8], float& top, std::uint32_t& low) {
+    auto put = [&](uint4* to, std::uint32_t part, const float (&x)[8], std::uint32_t& low) {
         std::uint32_t h[4], m[4], l[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             split3(x[2 * q], x[2 * q + 1], h[q], m[q], l[q]);
-            if constexpr (CT > 0) top = fmaxf(top, fmaxf(fabsf(x[2 * q]), fabsf(x[2 * q + 1])));
             low = min(low, min(smallness(x[2 * q]), smallness(x[2 * q + 1])));
         }
         to[0] = make_uint4(h[0], h[1], h[2], h[3]);
@@ -321,11 +321,15 @@ __global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
 #pragma unroll
         for (std::uint32_t r = 0; r < 8; ++r) f[r] = k + 8 * wn + r < k1 ? sign : 0.0f;
         const float gl = k + 8 * wn + gr < k1 && gj < a.C ? xg : 0.0f;
+        if constexpr (CT > 0) maxG = fmaxf(maxG, fabsf(gl));
         if (BM == 128 || at < BM) {
             float x[8];
 #pragma unroll
-            for (int r = 0; r < 8; ++r) x[r] = f[r] * xa[r];
-            put(to + wn * BM + at, kPartA, x, maxA, lowA);
+            for (int r = 0; r < 8; ++r) {
+                x[r] = f[r] * xa[r];
+                if constexpr (CT > 0) maxA = fmaxf(maxA, fabsf(x[r]));
+            }
+            put(to + wn * BM + at, kPartA, x, lowA);
         }
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
@@ -354,7 +358,7 @@ __global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
 #pragma unroll
                 for (int j = 0; j < GC; ++j) dw2[e][j] += part[j];
             }
-            put(to + 3 * kPartA + wn * BN + 128 * e + at, kPartB, x, maxB[e], lowB[e]);
+            put(to + 3 * kPartA + wn * BN + 128 * e + at, kPartB, x, lowB[e]);
         }
     };
     // B's tile u of this wave: positions 128 (u / 2) + 32 wn + 16 (u % 2) + l%16.
@@ -413,8 +417,16 @@ __global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
     const int tiles = wm == 0 ? TW : TM / 2;
 
     bool redo = k1 - k0 < kSplitMinTerms;
+#pragma unroll
+    for (int t = 0; t < TW; ++t)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) redo |= !(fabsf(acc[t][u][v]) <= 0x1.fffffep127f);
     const bool tinyA = lowA < kSplitExactBits, tinyB[2] = {lowB[0] < kSplitExactBits, lowB[1] < kSplitExactBits};
-    if (__syncthreads_or(tinyA || tinyB[0] || tinyB[1])) {
+    const bool tiny = tinyA || tinyB[0] || tinyB[1];
+    const bool look = __syncthreads_or(redo || tiny) != 0;
+    if (look && __syncthreads_or(tiny)) {
         // the columns' maxima and losses, of the four waves' rows: [4][BM] and
         // [4][BN] of each
         float* const topA = reinterpret_cast<float*>(parts);
@@ -431,6 +443,15 @@ __global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
                     maxB[0] = fmaxf(maxB[0], fabsf(xb[r][0]));
                     maxB[1] = fmaxf(maxB[1], fabsf(xb[r][1]));
                 }
+            }
+        } else {  // small elements of G W2^T are common (confident predictions): bounded by G's
+#pragma unroll
+            for (int d = GC; d < 64; d *= 2) maxG = fmaxf(maxG, __shfl_xor(maxG, d));
+#pragma unroll
+            for (int j = 0; j < GC; ++j) {
+                const float g = __shfl(maxG, j);
+                maxB[0] = fmaf(g, fabsf(w2[0][j]), maxB[0]);
+                maxB[1] = fmaf(g, fabsf(w2[1][j]), maxB[1]);
             }
         }
         if (at < BM) {
@@ -460,13 +481,7 @@ __global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
                 }
             }
     }
-#pragma unroll
-    for (int t = 0; t < TW; ++t)
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) redo |= !(fabsf(acc[t][u][v]) <= 0x1.fffffep127f);
-    if (__syncthreads_or(redo)) {
+    if (look && __syncthreads_or(redo)) {
 #pragma unroll
         for (int t = 0; t < TW; ++t)
 #pragma unroll

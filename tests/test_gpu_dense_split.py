@@ -109,12 +109,13 @@ def test_small_elements_among_ordinary_ones(gpu, e, small):
         _check(swtcf.dense_tn(A.cuda(), B.cuda()), A, B)
 
 
+@pytest.mark.parametrize("C", [1, 2, 3, 8])
 @pytest.mark.parametrize("e", [-109, -115, -140])
-def test_relu_gradient_small_elements(gpu, e):
+def test_relu_gradient_small_elements(gpu, e, C):
     """One row of dOut1, and one of AX, too small to split."""
     from tcc_amd import swtcf
 
-    K, F, Hd, C = 300, 113, 258, 2
+    K, F, Hd = 300, 113, 258
     for small in ("AX", "dOut1"):
         g = torch.Generator().manual_seed(3)
         AX, G, W2 = (torch.randn(s, generator=g) for s in ((K, F), (K, C), (Hd, C)))
@@ -130,7 +131,7 @@ def test_relu_gradient_small_elements(gpu, e):
             AX[:, ::5] = 0.0
             AX[9, ::5] = 2.0**100
         dW1, _ = swtcf.gcn_relu_grad(AX.cuda(), H.cuda(), G.cuda(), W2.cuda())
-        # the kernel's own dOut1, a sum of two rounded products
+        # the kernel's own dOut1, a sum of C rounded products
         d = torch.where(H > 0, G.double() @ W2.double().t(), torch.zeros((), dtype=torch.float64))
         dmag = torch.where(H > 0, G.double().abs() @ W2.double().abs().t(), torch.zeros((), dtype=torch.float64))
         want, mag = AX.double().t() @ d, AX.double().abs().t() @ dmag
