@@ -135,8 +135,9 @@ def test_relu_gradient_small_elements(gpu, e, C):
         d = torch.where(H > 0, G.double() @ W2.double().t(), torch.zeros((), dtype=torch.float64))
         dmag = torch.where(H > 0, G.double().abs() @ W2.double().abs().t(), torch.zeros((), dtype=torch.float64))
         want, mag = AX.double().t() @ d, AX.double().abs().t() @ dmag
-        # below 2^-126 dOut1 is rounded to multiples of 2^-149
-        sub = AX.double().abs().sum(0).unsqueeze(1) * 2.0**-148
+        # below 2^-126 each of the C additions of dOut1 rounds to a multiple of
+        # 2^-149, by half of it at most
+        sub = AX.double().abs().sum(0).unsqueeze(1) * (C * 2.0**-149)
         assert ((dW1.double().cpu() - want).abs() <= 2 * BOUND * mag + sub).all(), small
 
 
