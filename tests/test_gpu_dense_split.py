@@ -2,10 +2,12 @@
 the edges of the blocks and of the 32-row steps, values that do not survive a
 split, and whole numbers, against float64.
 
-An element's error is bounded by its sum of |a b|: the parts dropped are below
-2^-25 of each product, a step's six additions of 32 products each lose at most
-one unit in the last place, 2^-23, of it, and the additions of steps and
-splits (at most 35 steps here) half a unit: below 2^-18 in all."""
+An element's error is bounded by its sum of |a b|: the three part products left
+out come to at most 2^-24 of each product (for a and b in [1, 2) the middle
+parts are at most 2^-8 and the low parts 2^-17), a step's six additions of 32
+products each lose at most one unit in the last place, 2^-23, of it, and the
+additions of steps and splits (at most 35 steps here) half a unit: below 2^-18
+in all."""
 
 import pytest
 import torch
@@ -41,6 +43,31 @@ def test_edges(gpu, K, M, N):
     Ai = torch.randint(-60, 61, (K, M), generator=g, device="cuda").float()
     Bi = torch.randint(-200, 201, (K, N), generator=g, device="cuda").float()
     assert torch.equal(swtcf.dense_tn(Ai, Bi).double(), Ai.double().t() @ Bi.double())
+
+
+@pytest.mark.parametrize("bits", [(24, 1), (1, 24), (12, 12), (17, 7), (8, 16)])
+def test_every_part_counts(gpu, bits):
+    """One product a sum, of whole numbers of 24 significant bits in all, which
+    the middle and low parts hold most of: exact in both operands' parts."""
+    from tcc_amd import swtcf
+
+    def whole(shape, n):  # odd numbers of n bits
+        return (torch.randint(1 << (n - 1), 1 << n, shape, generator=g) | 1).float()
+
+    g = torch.Generator().manual_seed(bits[0])
+    K, M, N = 300, 130, 270
+    A, B = whole((K, M), bits[0]), whole((K, N), bits[1])
+    B[torch.arange(K).unsqueeze(1) != torch.arange(N)] = 0.0  # row k is column k's only one
+    assert torch.equal(swtcf.dense_tn(A.cuda(), B.cuda()).double().cpu(), A.double().t() @ B.double())
+    A, B = whole((K, M), bits[1]), whole((K, N), bits[0])
+    A[torch.arange(K).unsqueeze(1) != torch.arange(M)] = 0.0
+    assert torch.equal(swtcf.dense_tn(A.cuda(), B.cuda()).double().cpu(), A.double().t() @ B.double())
+    AX, W1 = whole((500, 100), bits[0]), whole((100, 200), bits[1])
+    for one in (0, 57, 99):
+        X = torch.zeros_like(AX)
+        X[:, one] = AX[:, one]
+        H, _ = swtcf.gcn_relu_forward(X.cuda(), W1.cuda(), torch.ones(200, 1).cuda())
+        assert torch.equal(H.double().cpu(), X.double() @ W1.double())
 
 
 def _special(kind, A, B):

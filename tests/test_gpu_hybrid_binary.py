@@ -488,3 +488,79 @@ def test_scaled_one_edge_many_times(gpu, groupBlocks):
         Y = swtcf.hybrid_spmm(H, X)[:rows].double()
         want = X.double().sum(0).expand(rows, -1)
         assert float((Y - want).norm()) <= 2.0**-10 * float(want.norm())  # TF32 operands, fp32 sums
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("rows,cols", [(32_768, 40_000), (32_769, 524_288), (600_000, 70_000)])
+def test_scaled_degree_counts(gpu, rows, cols, shift):
+    """Degrees counted in LDS slices of 32,768 indices, of one to sixteen, and
+    past those an atomic an edge, from COOs aligned to 16 and to 4 bytes: the
+    degree order, and the product of whole numbers against float64."""
+    from tcc_amd import _lib, swtcf
+
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    E = 700_003
+    hub = lambda n: (torch.rand(E, generator=g, device="cuda", dtype=torch.float64) ** 3 * n).long()  # noqa: E731
+    r, c = hub(rows), hub(cols)
+    r[:2], c[:2] = rows - 1, torch.tensor([0, cols - 1], device="cuda")
+    key = torch.unique(r * cols + c)
+    r, c = key // cols, key % cols
+    p = torch.randperm(r.numel(), generator=g, device="cuda")
+    r, c = r[p], c[p]
+    d, s = (torch.cat([torch.zeros(shift, dtype=torch.int32, device="cuda"), x.int()])[shift:] for x in (r, c))
+    assert (d.data_ptr() % 16 == 0) == (shift == 0)
+    H = swtcf.coo_to_hybrid_scaled(d, s, rows, cols)
+    order = torch.as_tensor(swtcf._download(H.view.tiles.rowOrder, rows, np.int32).astype(np.int64)).cuda()
+    deg = torch.bincount(r, minlength=rows)
+    assert torch.equal(order, torch.sort(deg, descending=True, stable=True).indices)
+    X = torch.randint(-3, 4, (cols, 20), generator=g, device="cuda").float()
+    want = torch.zeros(rows, 20, dtype=torch.float64, device="cuda").index_add_(0, r, X.double()[c])
+    assert torch.equal(swtcf.hybrid_spmm(H, X)[:rows].double(), want)
+    for bad_row, bad_col in ((rows, 0), (0, cols), (-1, 0)):
+        d2, s2 = d.clone(), s.clone()
+        d2[-1], s2[-1] = bad_row, bad_col
+        with pytest.raises(_lib.TccError, match="out of range"):
+            swtcf.coo_to_hybrid_scaled(d2, s2, rows, cols)
+
+
+def test_hybrid_builds_from_several_threads(gpu):
+    """Kept memory under hybrid builds: four threads on streams of their own
+    build, multiply and release different graphs, all that is kept given back
+    in between."""
+    import threading
+
+    from tcc_amd import _lib, graphs, swtcf
+
+    cases, errors = [], []
+    for k in range(4):
+        n = 3000 + 700 * k
+        r, c = graphs.rmat_graph(n, 60 * n, 20 + k, device="cuda")
+        X = torch.randint(-3, 4, (n, 33), generator=torch.Generator().manual_seed(k)).float().cuda()
+        want = torch.zeros(n, 33, dtype=torch.float64, device="cuda").index_add_(0, r, X.double()[c]).float()
+        cases.append((n, r.int(), c.int(), X, want))
+    torch.cuda.synchronize()
+
+    def work(k):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for i in range(10):
+                    n, r, c, X, want = cases[(k + i) % 4]
+                    if i % 2:
+                        H = swtcf.coo_to_hybrid_scaled(r, c, n, n, phases=1 + i % 3)
+                    else:
+                        H = swtcf.coo_to_hybrid(r, c, None, n, n)
+                    Y = swtcf.hybrid_spmm(H, X)[:n]
+                    if i == 4:
+                        _lib.check(_lib.lib().tcc_release_kept_memory())
+                    if not torch.equal(Y, want):
+                        raise AssertionError((k, i))
+                    H.release()
+        except Exception as e:  # shown by the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors

@@ -142,3 +142,44 @@ def test_mixed_stored_and_added(gpu, rows, F):
     out = torch.full(((g.bcsr.view.num_rowWindows + 1) * 8, F), float("nan"), device="cuda")
     swtcf.spmm_cnic_forward_mixed(g.bcsr, gcn._EMPTY_BCSC, table.source, out, F)
     assert torch.equal(out[:rows].double(), want) and not out[rows:].any()
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("columns", [1_048_575, 1_048_577, 2_450_000, 8_388_608, 8_388_609])
+def test_packed_columns_of_every_slice(gpu, columns, shift):
+    """The columns in use, marked in LDS by one to eight slices of 1,048,576
+    columns and past those in memory, from block arrays aligned to 16 and to 4
+    bytes: whole numbers from a workspace of other bytes, against the rows where
+    they lie and a float64 product."""
+    from tcc_amd import _lib, gcn, swtcf
+
+    nr, F = 700, 17
+    g = torch.Generator(device="cuda").manual_seed(columns)
+    # both sides of every slice's start
+    edge = torch.tensor(list(range(1_048_576, columns, 1_048_576)), dtype=torch.int64, device="cuda")
+    c = torch.cat([torch.randint(0, columns, (20_000,), generator=g, device="cuda"), edge, edge - 1,
+                   torch.tensor([0, columns - 1], device="cuda")])
+    key = torch.unique(torch.randint(0, nr, (c.numel(),), generator=g, device="cuda") * columns + c)
+    r, c = key // columns, key % columns
+    X = torch.randint(-3, 4, (columns, F), generator=g, device="cuda").float()
+    csm = torch.arange(columns, dtype=torch.int32, device="cuda")
+    none = torch.full((columns,), -1, dtype=torch.int32, device="cuda")
+    ptrs = torch.tensor([X.data_ptr()], dtype=torch.int64, device="cuda")
+    src = swtcf.feature_source(none, csm, ptrs, columns, 0, 0)
+    A = swtcf.coo_to_bcsr(r.int(), c.int(), None, nr, columns)
+    idx = torch.as_tensor(A.to_host()["sparseA2B"].view(np.int32)).cuda()
+    moved = torch.empty(idx.numel() + 1, dtype=torch.int32, device="cuda")[shift:]
+    moved[: idx.numel()].copy_(idx)
+    v = _lib.BCSR.from_buffer_copy(A.view)
+    v.sparseA2B = moved.data_ptr()
+    L = _lib.lib()
+    need = L.tcc_tf32_packed_bytes(columns, F) + 16 + 4 * ((columns + 31) // 32)
+    ws = torch.full((need,), 255, dtype=torch.uint8, device="cuda")
+    out = torch.full(((v.num_rowWindows + 1) * 8, F), float("nan"), device="cuda")
+    direct = torch.full_like(out, float("nan"))
+    stream = torch.cuda.current_stream().cuda_stream
+    args = (ctypes.byref(v), ctypes.byref(gcn._EMPTY_BCSC.view), ctypes.byref(src.struct))
+    _lib.check(L.tcc_spmm_cnic_forward_mixed_ws(*args, direct.data_ptr(), F, None, 0, stream))
+    _lib.check(L.tcc_spmm_cnic_forward_mixed_ws(*args, out.data_ptr(), F, ws.data_ptr(), need, stream))
+    want = torch.zeros(nr, F, dtype=torch.float64, device="cuda").index_add_(0, r, X.double()[c])
+    assert torch.equal(out[:nr].double(), want) and torch.equal(direct, out)
