@@ -36,7 +36,9 @@ size_t tcc_dense_tn_workspace_bytes(uint32_t K, uint32_t M, uint32_t N);
  * 4-byte aligned; `workspace` is device memory of at least
  * tcc_dense_tn_workspace_bytes(K, M, N) bytes, not shared with a concurrent
  * call.  Asynchronous on `stream` (a hipStream_t; NULL = the null stream).
- * Replaces torch.mm(X_out.T, d_output), tcgnn_conv_release.py:150. */
+ * Replaces torch.mm(X_out.T, d_output), tcgnn_conv_release.py:150.
+ * With M and N above 16 and K of at least 4, the products are those of the
+ * operands' bf16 parts (as tcc_gcn_relu_forward), else fp32 MFMA's. */
 int tcc_dense_tn(const float* A, uint32_t lda, const float* B, uint32_t ldb, float* C, uint32_t ldc, uint32_t K,
                  uint32_t M, uint32_t N, int accumulate, void* workspace, size_t workspaceBytes, void* stream);
 
@@ -62,10 +64,12 @@ int tcc_dense_tn_noalloc(const float* A, uint32_t lda, const float* B, uint32_t 
  * second layer's transform of a two-layer GCN, which the reference runs as
  * X_gat = torch.mm(X_out, weights) (train/tcgnn_conv_release.py:134),
  * self.relu (:231-238) and the last layer's torch.mm (:134 again) with H
- * written and read back in between.  Products of exact bf16 parts of the fp32
- * operands, summed in fp32 (no less accurate than fp32 MFMA); relu keeps NaN
- * (clamp_min).  F <= 128, Hd <= 256, C <= 4 (TCC_ERR_UNSUPPORTED
- * above).  No workspace. */
+ * written and read back in between.  From F = 4 on AX W1 multiplies the exact
+ * bf16 parts of the fp32 operands, six of the nine part products, summed in
+ * fp32: a single product to 1.6e-7 of it (fp32 MFMA: 6e-8), sums of three and
+ * more normal products closer to 64 bits than with fp32 MFMA.  H W2 in fp32;
+ * relu keeps NaN (clamp_min).  F <= 128, Hd <= 256, C <= 4
+ * (TCC_ERR_UNSUPPORTED above).  No workspace. */
 int tcc_gcn_relu_forward(const float* AX, uint32_t ldax, const float* W1, const float* W2, float* H, uint32_t ldh,
                          float* XW, uint32_t ldxw, uint32_t K, uint32_t F, uint32_t Hd, uint32_t C, void* stream);
 
@@ -84,7 +88,8 @@ size_t tcc_gcn_relu_grad_workspace_bytes(uint32_t K, uint32_t F, uint32_t Hd, ui
  * (train/tcgnn_conv_release.py:147-154 for each layer, with torch's relu
  * backward between): grad_X = grad_sp @ weights.T of the second layer,
  * the relu mask, and grad_weights = X_out.T @ d_output of both layers.
- * Products and sums in fp32; dW1 and dW2 are overwritten.  `workspace` as
+ * G W2^T and dW2 in fp32, dW1's products of bf16 parts (as
+ * tcc_gcn_relu_forward), summed in fp32; dW1 and dW2 are overwritten.  `workspace` as
  * for tcc_dense_tn, at least tcc_gcn_relu_grad_workspace_bytes bytes. */
 int tcc_gcn_relu_grad(const float* AX, uint32_t ldax, const float* H, uint32_t ldh, const float* G, uint32_t ldg,
                       const float* W2, float* dW1, float* dW2, uint32_t K, uint32_t F, uint32_t Hd, uint32_t C,

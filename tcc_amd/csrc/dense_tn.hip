@@ -185,18 +185,20 @@ __device__ __forceinline__ std::uint32_t smallness(float x) { return (__float_as
 constexpr std::uint32_t kSplitExactBits = ((127u - 110u) << 24) - 1u;  // of 2^-110
 
 // Sums of fewer products are left to the fp32 products.  The six part products
-// give a single product to 2^-23 (the three left out and the MFMA's truncation),
-// fp32 MFMA to 2^-24; sums of 1, 2, 3, 4 normal products are off by 3.5, 3.3,
-// 3.3, 3.2e-8 of the result, in fp32 by 2.5, 3.1, 3.6, 4.0e-8, and the longer
-// the sum, the further the part products are ahead (100 products: 5.6e-8
-// against 1.8e-7).
+// give a single product to 1.6e-7 of it (the three left out and the MFMA's
+// truncation), fp32 MFMA to 6e-8; sums of 1, 2, 3, 4 normal products are off by
+// 3.5, 3.3, 3.3, 3.2e-8 of the result, in fp32 by 2.5, 3.1, 3.6, 4.0e-8, and the
+// longer the sum, the further the part products are ahead (100 products: 5.6e-8
+// against 1.8e-7): 32 rows are rounded together.  A long sum with one term that
+// is not zero is a single product all the same.
 constexpr std::uint32_t kSplitMinTerms = 4;
 
 // Wide outputs.  fp32 MFMA runs at 1/16 of the bf16 rate, and the 100 x 256
 // and 602 x 256 products over node rows were bound by it (110 TFLOP/s).  Here
 // each operand is split into three bf16 parts (split3) and a product is the
-// six of the nine part products above 2^-26 of it, summed in fp32, smallest
-// first: every bit of the inputs is used.  The bf16 products' own additions
+// six largest of the nine part products, summed in fp32, smallest first: every
+// bit of the inputs is used, and the three left out (middle by low and low by
+// low) come to at most 2^-24 of a product, 2^-27.5 rms.  The bf16 products' own additions
 // do not round to nearest: summed through all rows, 2.45M of them gave 4.5
 // times the fp32 products' error; so 32 rows are summed by themselves and
 // added to the running sum with an ordinary fma, the sign of A's rows changed
@@ -229,8 +231,8 @@ constexpr std::uint32_t kSplitMinTerms = 4;
 //
 // 233k x 602 x 256: 0.43 ms (0.89 with fp32 products, in 3 turns of one
 // workgroup a compute unit), 1.1 PFLOP/s of bf16 part products, the rate of a
-// large bf16 matrix product here; 2.45M x 100 x 256: 1.03 ms (1.22), with the
-// relu gradient of 2 classes 1.12 ms (1.35).  Error against 64 bits 2.4e-7,
+// large bf16 matrix product here; 2.45M x 100 x 256: 0.87 ms (1.07), with the
+// relu gradient of 2 classes 0.97 ms (1.28).  Error against 64 bits 2.4e-7,
 // 3.3e-7 and 3.3e-7 of the result (8.6e-7, 1.3e-6 and 8.7e-7).
 template <int TM, int CT, bool VB>
 __global__ void __launch_bounds__(512) tn_split_kernel(TnArgs a) {
