@@ -45,7 +45,12 @@ namespace tcc {
 namespace {
 
 constexpr unsigned kThreads = 256;
-constexpr std::uint64_t kGatherPlanMinEdges = 1u << 18;  // any plan
+// Any plan.  R-MAT graphs at F = 128, us a call of the kernel : with a plan (the
+// hash and its wait among it), and the call that builds it: 60k edges 50 : 66;
+// 120k 90 : 67, 390; 264k 180 : 76, 906; 600k 339 : 92, 1,227; 1.5M 790 : 132,
+// 1,988.  A planned call wins from about 80k edges on, but it waits for the
+// stream and pays for its build after ten calls only, so the line lies above.
+constexpr std::uint64_t kGatherPlanMinEdges = 1u << 18;
 constexpr std::uint64_t kPlanMinEdges = 4u << 20;         // the hybrid (with the degree)
 constexpr std::uint32_t kPlanMinRowDegree = 64;
 // Gathers per source row (8 per block column) from which X is packed.
