@@ -132,7 +132,7 @@ def _short(name: str, width: int = 72) -> str:
 def stats_md(args) -> str:
     rows = read_stats(args.csv)
     total = sum(r["total_ms"] for r in rows)
-    lines = [f"# {args.title}", "", "Command (from the repository root on the GPU box, TMPDIR=/tmp):", "", "```",
+    lines = [f"# {args.title}", "", "Command (from the repository root, TMPDIR=/tmp):", "", "```",
              args.command, "```", ""]
     d = re.search(r"rocprofv3 --kernel-trace --stats\b.*? -d (\S+) -o run\b", args.command)
     if d:
@@ -185,7 +185,7 @@ def counters_md(args) -> str:
     per = read_counters(args.csv)
     pat = re.compile(args.kernels)
     names = sorted({c for k, cs in per.items() if pat.search(k) for c in cs})
-    lines = [f"# {args.title}", "", "Command (from the repository root on the GPU box, TMPDIR=/tmp):", "", "```",
+    lines = [f"# {args.title}", "", "Command (from the repository root, TMPDIR=/tmp):", "", "```",
              args.command, "```", "", "Means per dispatch:", ""]
     extra = []
     if "SQ_VALU_MFMA_BUSY_CYCLES" in names and "GRBM_GUI_ACTIVE" in names:
