@@ -1572,7 +1572,11 @@ int mixed_vec(const tcc_feature_source* src, std::uint32_t F, const float* Y) {
 // packed, us: 2.45M rows 2010 : 2018 at F = 17, 2540 : 2124 at 64,
 // 4911 : 2784 at 100, 9337 : 5957 at 256; 200k rows 217 : 246 at F = 64
 // (51 MB), 306 : 317 at 128 (102 MB), 590 : 472 at 200 (160 MB); 20k rows
-// 56 : 65 at F = 100 (8 MB).
+// 56 : 65 at F = 100 (8 MB).  Rows in host memory, if any, cross the link once
+// each instead of once a gather, but before the gather instead of beside it:
+// 400k rows, 8M edges, F = 100, us: a tenth of the rows hot 10,843 : 2,072, a
+// quarter 3,452 : 1,622, half (44,000 cold rows, gathered once each) 611 : 828;
+// 2.45M rows 63,319 : 11,974, 19,146 : 9,272 and 5,163 : 4,403.
 constexpr std::uint32_t kMixedPackMinF = 17;
 constexpr std::uint64_t kMixedPackMinTable = 128ull << 20;
 // Output size from which the first layer without a scatter stores its rows: a
